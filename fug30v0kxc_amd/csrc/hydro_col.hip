@@ -20,7 +20,9 @@
 //   d1bydz(h, 2) and d1bydz(4 scko3 g, 5)            (lines 183-184, 391, 434)
 // with divu = ux + vy + d1bydz(w, 1).  The d/dx d/dx u and d/dy d/dy v parts
 // ride in the x / y passes' second outputs (MUL_D2C), since they differ from
-// d2bydx / d2bydy at the Nyquist mode.
+// d2bydx / d2bydy at the Nyquist mode, and so do dxm, dym, the other Maxwell
+// stresses and the mixed derivatives (the passes' auxiliary lines): each
+// momentum equation reads one array per horizontal direction (uxs .. wys).
 #include <type_traits>
 
 #include "launch.hpp"
@@ -141,8 +143,6 @@ __device__ __forceinline__ void HydroColKernel<TW, MIX, WALL>::body(const HydroC
             tdot = tdot + p.sckg * (w1 + w2) * (w1 + w2);
         }
         // 245-261
-        udot = udot + at(a.ybb, q);
-        vdot = vdot + at(a.xbb, q);
         {
             const double w3 = d.wx, w4 = d.uzu;
             udot = udot - rr * w0 * w4;
@@ -151,7 +151,7 @@ __device__ __forceinline__ void HydroColKernel<TW, MIX, WALL>::body(const HydroC
         }
         // 287-309
         udot = udot + d.zzx;
-        wdot = wdot + at(a.xzx, q) + p.thmplus1 * rr;
+        wdot = wdot + p.thmplus1 * rr;
         {
             const double w1 = d.wy, w2 = d.vzu;
             vdot = vdot - rr * w0 * w2;
@@ -163,20 +163,18 @@ __device__ __forceinline__ void HydroColKernel<TW, MIX, WALL>::body(const HydroC
         wdot = wdot - rr * p.cor * (-u0 * p.cpsi);
         // 331-338
         vdot = vdot + d.zzy;
-        wdot = wdot + at(a.yzy, q);
-        // 360-432 (uxxc and vyyc carry sck*d2 plus the scko3 d/dx d/dx u and
-        // d/dy d/dy v parts of the composite fluxes)
+        // 360-432, 181-184, 230-338: the horizontal viscous and Maxwell stresses
+        // and the composite fluxes' horizontal parts
         udot = udot + p.sck * d.uzz;
         vdot = vdot + p.sck * d.vzz;
-        udot = udot + at(a.uxxc, q);
-        vdot = vdot + p.sck * at(a.vxx, q);
-        wdot = wdot + p.sck * at(a.wxx, q);
-        udot = udot + p.sck * at(a.uyy, q);
-        vdot = vdot + at(a.vyyc, q);
-        wdot = wdot + p.sck * at(a.wyy, q);
-        // composite flux derivatives (181-184)
-        udot = udot + (scko3 * (at(a.vxy, q) + d.dzwx) + at(a.dxm, q));
-        vdot = vdot + (scko3 * (at(a.uxy, q) + d.dzwy) + at(a.dym, q));
+        udot = udot + at(a.uxs, q);
+        vdot = vdot + at(a.vxs, q);
+        wdot = wdot + at(a.wxs, q);
+        udot = udot + at(a.uys, q);
+        vdot = vdot + at(a.vys, q);
+        wdot = wdot + at(a.wys, q);
+        udot = udot + scko3 * d.dzwx;
+        vdot = vdot + scko3 * d.dzwy;
         wdot = wdot + d.c3 + d.c4;
         // 455-470: d(rho)/dz on the walls from dw/dt = 0
         double rzu = d.rzu, rzc = d.rzc;

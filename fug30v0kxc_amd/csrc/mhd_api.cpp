@@ -46,9 +46,8 @@ namespace {
 
 // work buffers of the RHS assembly
 enum Wk {
-    W_RX, W_TX, W_TXX, W_UX, W_UXX, W_VX, W_VXX, W_WX, W_WXX, W_XBB, W_XZX,
-    W_RY, W_TY, W_TYY, W_UY, W_UYY, W_VY, W_VYY, W_WY, W_WYY, W_YBB, W_YZY,
-    W_DXM, W_DYM, W_UXY, W_VXY,
+    W_RX, W_TX, W_TXX, W_UX, W_UXS, W_VX, W_VXS, W_WX, W_WXS,
+    W_RY, W_TY, W_TYY, W_UY, W_UYS, W_VY, W_VYS, W_WY, W_WYS,
     W_COUNT
 };
 
@@ -362,12 +361,10 @@ HydroColArgs colargs(mhd_ctx* c)
     a.kappa = c->kappa; a.dkappa = c->dkappa;
     a.etar = c->eta_on ? c->etar : nullptr;
     void** W = c->wk;
-    a.rx = W[W_RX]; a.tx = W[W_TX]; a.txx = W[W_TXX]; a.ux = W[W_UX]; a.uxxc = W[W_UXX];
-    a.vx = W[W_VX]; a.vxx = W[W_VXX]; a.wx = W[W_WX]; a.wxx = W[W_WXX]; a.xbb = W[W_XBB]; a.xzx = W[W_XZX];
-    a.dxm = W[W_DXM];
-    a.ry = W[W_RY]; a.ty = W[W_TY]; a.tyy = W[W_TYY]; a.uy = W[W_UY]; a.uyy = W[W_UYY];
-    a.vy = W[W_VY]; a.vyyc = W[W_VYY]; a.wy = W[W_WY]; a.wyy = W[W_WYY]; a.ybb = W[W_YBB]; a.yzy = W[W_YZY];
-    a.dym = W[W_DYM]; a.uxy = W[W_UXY]; a.vxy = W[W_VXY];
+    a.rx = W[W_RX]; a.tx = W[W_TX]; a.txx = W[W_TXX]; a.ux = W[W_UX]; a.uxs = W[W_UXS];
+    a.vx = W[W_VX]; a.vxs = W[W_VXS]; a.wx = W[W_WX]; a.wxs = W[W_WXS];
+    a.ry = W[W_RY]; a.ty = W[W_TY]; a.tyy = W[W_TYY]; a.uy = W[W_UY]; a.uys = W[W_UYS];
+    a.vy = W[W_VY]; a.vys = W[W_VYS]; a.wy = W[W_WY]; a.wys = W[W_WYS];
     a.rdot = level_ptr(c, 3, 3);
     a.tdot = level_ptr(c, 4, 3);
     a.udot = level_ptr(c, 0, 3);
@@ -394,9 +391,9 @@ MagArgs margs(mhd_ctx* c)
     void** W = c->wk;
     // the RHS-assembly planes are free while the magnetic routines run
     a.exh = W[W_RX]; a.eyh = W[W_TX]; a.ezh = W[W_TXX];
-    a.d = W[W_UX]; a.cc = W[W_UXX];
-    a.polz = W[W_VXX];
-    a.bxh = W[W_WX]; a.byh = W[W_WXX]; a.bzh = W[W_XBB]; a.jzh = W[W_XZX]; a.dybzh = W[W_RY]; a.dxbzh = W[W_TY];
+    a.d = W[W_UX]; a.cc = W[W_UXS];
+    a.polz = W[W_VXS];
+    a.bxh = W[W_WX]; a.byh = W[W_WXS]; a.bzh = W[W_UY]; a.jzh = W[W_UYS]; a.dybzh = W[W_RY]; a.dxbzh = W[W_TY];
     a.bx = c->bx; a.by = c->by; a.jsq = c->jsq;
     if (c->su) { a.bxm = c->bxbar; a.bym = c->bybar; }
     if (c->eta_on) { a.jx = c->jx; a.jy = c->jy; a.jz = c->jz; }
@@ -465,68 +462,51 @@ int run_hydro_deriv(mhd_ctx* c, const double* cf = nullptr)
     const void* W_ = mx ? (const void*)c->sw : c->w;
     const void* R_ = mx ? (const void*)c->sr : c->r;
     const int sf = mx ? 1 : 0;
-    const double* mbx = mx ? c->bxbar : nullptr;
-    const double* mby = mx ? c->bybar : nullptr;
-    const double* mbz = mx ? c->bzm : nullptr;
-    auto means = [](SpecJob& j, const double* m0, const double* m1, const double* m2) {
-        j.mean[0] = m0; j.mean[1] = m1; j.mean[2] = m2;
+    // second derivatives of u, v, w carry the Maxwell stresses (of the field
+    // components and their means) and mixed derivatives as auxiliary lines
+    auto with_b = [&](SpecLaunch& L) {
+        L.bf[0] = c->bx; L.bf[1] = c->by; L.bf[2] = c->bz;
+        if (mx) { L.bmean[0] = c->bxbar; L.bmean[1] = c->bybar; L.bmean[2] = c->bzm; }
     };
-    // x pass: d/dx, d2/dx2 of t, u, v, w (u's second output also carries the
-    // scko3 d/dx d/dx u of the composite flux, lines 181, 258) and d/dx of r,
-    // a single-output job of the same launch (one launch instead of two: at
-    // 256^2 x 160 FP64 242 against 210 + 47 us); then d/dx of the
-    // Maxwell-stress products F by bx, F bz bx, F/2 (bx^2-by^2-bz^2)
+    auto stress = [](SpecJob& j, double c2, double c11, int op, int ai, int aj, double scale) {
+        j.mc[0] = c2; j.mc[1] = c11;
+        j.aux = op; j.ai = ai; j.aj = aj; j.ascale = scale;
+    };
+    enum { BX = 0, BY = 1, BZ = 2 };
+    // x pass: d/dx of u, v, w, t, r; the second outputs (HydroColArgs) hold
+    // sck d2/dx2 with u's scko3 d/dx d/dx u of the composite flux (lines 181,
+    // 258) and d/dx of F/2 (bx^2-by^2-bz^2), F by bx, F bz bx
     {
         SpecLaunch L = spec_base(c, 0, SM_DERIV2);
-        L.job[0] = sjob(T_, sf, W[W_TX], W[W_TXX], MUL_D1, MUL_D2, wf);
-        L.job[1] = sjob(U_, sf, W[W_UX], W[W_UXX], MUL_D1, MUL_D2C, wf);
-        L.job[1].mc[0] = P.sck; L.job[1].mc[1] = P.scko3;
-        L.job[2] = sjob(V_, sf, W[W_VX], W[W_VXX], MUL_D1, MUL_D2, wf);
-        L.job[3] = sjob(W_, sf, W[W_WX], W[W_WXX], MUL_D1, MUL_D2, wf);
+        with_b(L);
+        L.job[0] = sjob(U_, sf, W[W_UX], W[W_UXS], MUL_D1, MUL_D2C, wf);
+        stress(L.job[0], P.sck, P.scko3, AUX_MAXW, BX, 0, P.fo2);
+        L.job[1] = sjob(V_, sf, W[W_VX], W[W_VXS], MUL_D1, MUL_D2C, wf);
+        stress(L.job[1], P.sck, 0.0, AUX_PROD, BY, BX, f);
+        L.job[2] = sjob(W_, sf, W[W_WX], W[W_WXS], MUL_D1, MUL_D2C, wf);
+        stress(L.job[2], P.sck, 0.0, AUX_PROD, BZ, BX, f);
+        L.job[3] = sjob(T_, sf, W[W_TX], W[W_TXX], MUL_D1, MUL_D2, wf);
         L.job[4] = sjob(R_, sf, W[W_RX], nullptr, MUL_D1, 0, wf);
         L.njobs = 5;
         TRY(spec(c, L, MHD_K_XDERIV2));
-        SpecLaunch M = spec_base(c, 0, SM_DERIV1);
-        M.job[0] = sjob(c->by, wf, W[W_XBB], nullptr, MUL_D1, 0, wf);
-        M.job[0].load_op = LD_PROD; M.job[0].in[1] = c->bx; M.job[0].scale = f;
-        means(M.job[0], mby, mbx, nullptr);
-        M.job[1] = sjob(c->bz, wf, W[W_XZX], nullptr, MUL_D1, 0, wf);
-        M.job[1].load_op = LD_PROD; M.job[1].in[1] = c->bx; M.job[1].scale = f;
-        means(M.job[1], mbz, mbx, nullptr);
-        M.job[2] = sjob(c->bx, wf, W[W_DXM], nullptr, MUL_D1, 0, wf);
-        M.job[2].load_op = LD_MAXW; M.job[2].in[1] = c->by; M.job[2].in[2] = c->bz; M.job[2].scale = P.fo2;
-        means(M.job[2], mbx, mby, mbz);
-        M.njobs = 3;
-        TRY(spec(c, M));
     }
     // y pass: the same along y (v's second output carries scko3 d/dy d/dy v),
-    // with the single-output jobs d/dy of r and the mixed derivatives d/dy(ux),
-    // d/dy(vx) of the composite fluxes (FP64 318 against 219 + 120 us as two
-    // launches); then the Maxwell-stress products
+    // with d/dy of scko3 vx and scko3 ux of the composite fluxes
     {
         SpecLaunch L = spec_base(c, 1, SM_DERIV2);
-        L.job[0] = sjob(T_, sf, W[W_TY], W[W_TYY], MUL_D1, MUL_D2, wf);
-        L.job[1] = sjob(U_, sf, W[W_UY], W[W_UYY], MUL_D1, MUL_D2, wf);
-        L.job[2] = sjob(V_, sf, W[W_VY], W[W_VYY], MUL_D1, MUL_D2C, wf);
-        L.job[2].mc[0] = P.sck; L.job[2].mc[1] = P.scko3;
-        L.job[3] = sjob(W_, sf, W[W_WY], W[W_WYY], MUL_D1, MUL_D2, wf);
+        with_b(L);
+        L.job[0] = sjob(U_, sf, W[W_UY], W[W_UYS], MUL_D1, MUL_D2C, wf);
+        stress(L.job[0], P.sck, 0.0, AUX_PROD, BY, BX, f);
+        L.job[0].xin = W[W_VX]; L.job[0].xcoef = P.scko3;
+        L.job[1] = sjob(V_, sf, W[W_VY], W[W_VYS], MUL_D1, MUL_D2C, wf);
+        stress(L.job[1], P.sck, P.scko3, AUX_MAXW, BY, 0, P.fo2);
+        L.job[1].xin = W[W_UX]; L.job[1].xcoef = P.scko3;
+        L.job[2] = sjob(W_, sf, W[W_WY], W[W_WYS], MUL_D1, MUL_D2C, wf);
+        stress(L.job[2], P.sck, 0.0, AUX_PROD, BZ, BY, f);
+        L.job[3] = sjob(T_, sf, W[W_TY], W[W_TYY], MUL_D1, MUL_D2, wf);
         L.job[4] = sjob(R_, sf, W[W_RY], nullptr, MUL_D1, 0, wf);
-        L.job[5] = sjob(W[W_UX], wf, W[W_UXY], nullptr, MUL_D1, 0, wf);
-        L.job[6] = sjob(W[W_VX], wf, W[W_VXY], nullptr, MUL_D1, 0, wf);
-        L.njobs = 7;
+        L.njobs = 5;
         TRY(spec(c, L, MHD_K_YDERIV2));
-        SpecLaunch M = spec_base(c, 1, SM_DERIV1);
-        M.job[0] = sjob(c->by, wf, W[W_YBB], nullptr, MUL_D1, 0, wf);
-        M.job[0].load_op = LD_PROD; M.job[0].in[1] = c->bx; M.job[0].scale = f;
-        means(M.job[0], mby, mbx, nullptr);
-        M.job[1] = sjob(c->bz, wf, W[W_YZY], nullptr, MUL_D1, 0, wf);
-        M.job[1].load_op = LD_PROD; M.job[1].in[1] = c->by; M.job[1].scale = f;
-        means(M.job[1], mbz, mby, nullptr);
-        M.job[2] = sjob(c->by, wf, W[W_DYM], nullptr, MUL_D1, 0, wf);
-        M.job[2].load_op = LD_MAXW; M.job[2].in[1] = c->bx; M.job[2].in[2] = c->bz; M.job[2].scale = P.fo2;
-        means(M.job[2], mby, mbx, mbz);
-        M.njobs = 3;
-        TRY(spec(c, M));
     }
     HydroColArgs a = colargs(c);
     if (cf) fuse_ab3(c, a, cf, level_ptr(c, 3, 1), level_ptr(c, 3, 2));
@@ -853,7 +833,7 @@ int run_checkdivb(mhd_ctx* c, double out[2])
     L.njobs = 1;
     TRY(spec(c, L));
     SpecLaunch M = spec_base(c, 1, SM_DERIV1);
-    M.job[0] = sjob(c->by, wf, W[W_UYY], nullptr, MUL_D1, 0, wf);
+    M.job[0] = sjob(c->by, wf, W[W_UYS], nullptr, MUL_D1, 0, wf);
     M.njobs = 1;
     TRY(spec(c, M));
     ZLaunch Z = zbase(c);
@@ -861,7 +841,7 @@ int run_checkdivb(mhd_ctx* c, double out[2])
     Z.njobs = 1;
     TRY(zrun(c, Z));
     RedArgs a = rargs(c, RED_DIVB);
-    a.f0 = W[W_UY]; a.f1 = W[W_UYY]; a.f2 = W[W_VY];
+    a.f0 = W[W_UY]; a.f1 = W[W_UYS]; a.f2 = W[W_VY];
     a.f_f32 = wf;
     TRY(kerr(launch_reduce(a, c->s)));
     return fetch_result(c, out, 2);
@@ -1855,7 +1835,7 @@ int mhd_autotune(mhd_ctx_t* c, mhd_tune_t* out)
     // step's (outputs into work arrays); the current choice (the default at
     // first) is timed first
     const int o1[2][4] = {{W_TX, W_UX, W_VX, W_WX}, {W_TY, W_UY, W_VY, W_WY}};
-    const int o2[2][4] = {{W_TXX, W_UXX, W_VXX, W_WXX}, {W_TYY, W_UYY, W_VYY, W_WYY}};
+    const int o2[2][4] = {{W_TXX, W_UXS, W_VXS, W_WXS}, {W_TYY, W_UYS, W_VYS, W_WYS}};
     auto kind_launch = [&](int dir, int kind) {
         SpecLaunch L = spec_base(c, dir, kind);
         for (int j = 0; j < 4; ++j) {
@@ -1866,16 +1846,18 @@ int mhd_autotune(mhd_ctx_t* c, mhd_tune_t* out)
         }
         L.njobs = 4;
         if (kind == SM_DERIV2) {
-            // as in the step: a single-output (first-derivative) job beside the four
+            // as in the step: three jobs with auxiliary lines, one without, and a
+            // single-output (first-derivative) job
+            L.bf[0] = in[1]; L.bf[1] = in[2]; L.bf[2] = in[3];
+            for (int j = 0; j < 3; ++j) {
+                L.job[j].aux = j == 0 ? AUX_MAXW : AUX_PROD;
+                L.job[j].ai = j;
+                L.job[j].aj = 0;
+                L.job[j].ascale = 1.0;
+                if (dir == 1 && j < 2) L.job[j].xin = in[0];
+            }
             L.job[4] = sjob(in[0], sf, W[dir == 0 ? W_RX : W_RY], nullptr, MUL_D1, 0, wf);
             L.njobs = 5;
-        } else if (kind == SM_DERIV1) {
-            // as in the step: the first derivatives of one direction's three
-            // Maxwell-stress loads (products of three fields)
-            L.job[0].in[0] = in[2]; L.job[0].load_op = LD_PROD; L.job[0].in[1] = in[1];
-            L.job[1].in[0] = in[3]; L.job[1].load_op = LD_PROD; L.job[1].in[1] = in[1];
-            L.job[2].in[0] = in[1]; L.job[2].load_op = LD_MAXW; L.job[2].in[1] = in[2]; L.job[2].in[2] = in[3];
-            L.njobs = 3;
         }
         return L;
     };
@@ -2050,9 +2032,9 @@ int mhd_op(mhd_ctx_t* c, int op, const double* in, double* out, double* out2, in
     if (!in || !out) return MHD_E_ARG;
     const int wf = c->wf32;
     const long n3 = c->n3;
-    void* A = c->wk[W_DXM];
-    void* B = c->wk[W_DYM];
-    void* C = c->wk[W_UXY];
+    void* A = c->wk[W_UYS];
+    void* B = c->wk[W_VYS];
+    void* C = c->wk[W_WYS];
     if (op == MHD_OP_D1BYDZ1D || op == MHD_OP_D2BYDZ1D) {
         // nz-vectors: run the 3-D kernel on a 1x1 column broadcast over the plane
         std::vector<double> col(n3);

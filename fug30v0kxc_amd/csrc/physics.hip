@@ -133,7 +133,7 @@ int launch_z(const ZLaunch& L, hipStream_t s)
                 done[j] = true;
             }
         }
-        const bool prod = a.load_op == LD_PROD;
+        const bool prod = a.load_op != 0;
         int e;
         if (a.out_f32) {
             if (L.w_f32) e = a.in_f32 ? launch_z_kind<float, float, float>(G, a.kind, prod, s)

@@ -58,13 +58,16 @@ struct HydroColArgs {
     double bzm;                         // mixed: Bz-bar
     const double *kappa, *dkappa;
     const double* etar;                 // eta(z)/eta_0 for the Ohmic heating, or null (1)
-    // x pass: d/dx of r, t, u, v, w; d2/dx2 of t, v, w; uxxc = sck*uxx +
-    // scko3*d/dx(d/dx u); xbb = d/dx(F by bx); xzx = d/dx(F bz bx);
-    // dxm = d/dx(F/2 (bx^2 - by^2 - bz^2))
-    const void *rx, *tx, *txx, *ux, *uxxc, *vx, *vxx, *wx, *wxx, *xbb, *xzx, *dxm;
-    // y pass: the same along y with vyyc = sck*vyy + scko3*d/dy(d/dy v),
-    // dym = d/dy(F/2 (by^2 - bx^2 - bz^2)), uxy = d/dy(ux), vxy = d/dy(vx)
-    const void *ry, *ty, *tyy, *uy, *uyy, *vy, *vyyc, *wy, *wyy, *ybb, *yzy, *dym, *uxy, *vxy;
+    // x pass: d/dx of r, t, u, v, w, d2/dx2 of t, and the x parts of the
+    // momentum equations' viscous and Maxwell stresses
+    //   uxs = sck*uxx + scko3*d/dx(d/dx u) + d/dx(F/2 (bx^2 - by^2 - bz^2))
+    //   vxs = sck*vxx + d/dx(F by bx), wxs = sck*wxx + d/dx(F bz bx)
+    const void *rx, *tx, *txx, *ux, *uxs, *vx, *vxs, *wx, *wxs;
+    // y pass: the same along y
+    //   uys = sck*uyy + d/dy(scko3 vx + F by bx)
+    //   vys = sck*vyy + scko3*d/dy(d/dy v) + d/dy(scko3 ux + F/2 (by^2 - bx^2 - bz^2))
+    //   wys = sck*wyy + d/dy(F bz by)
+    const void *ry, *ty, *tyy, *uy, *uys, *vy, *vys, *wy, *wys;
     void *rdot, *tdot, *udot, *vdot, *wdot;   // newest history level (working precision)
     int zc;                             // planes per thread
     // fused AB3 update of u v w r t (src/main.F90:413-443); ab3 = 0: RHS only.

@@ -12,29 +12,26 @@ enum SpecMode { SM_DERIV1 = 0, SM_DERIV2 = 1, SM_R2HC = 2, SM_HC2R = 3 };
 // MUL_D2C: mc[0] * d2 + mc[1] * d1(d1(.)); the two differ at the Nyquist
 // mode only, which d2 keeps (akx2) and d1 zeroes.
 enum MulKind { MUL_D1 = 0, MUL_D2 = 1, MUL_MASK = 2, MUL_D2C = 3 };
-// LD_BG: FP64 input minus a per-plane background (the mixed path's
-// fluctuation loads); the others read inputs of the compute type.
-// Products take optional per-plane means m_i of their factors (the mixed
-// path stores B without its means): the load is the product of (in_i + m_i)
-// minus its per-plane constant, which no horizontal derivative sees.
-//   LD_PROD  scale*(in0+m0)*(in1+m1)
+// Inputs have the compute type.  Products take optional per-plane means m_i of
+// their factors (the mixed path stores B without its means): the load is the
+// product of (in_i + m_i) minus its per-plane constant, which no horizontal
+// derivative sees.
 //   LD_CROSS (in0+m0)*(in1+m1) - (in2+m2)*(in3+m3)
-//   LD_MAXW  scale*((in0+m0)^2 - (in1+m1)^2 - (in2+m2)^2)
-enum LoadOp { LD_PLAIN = 0, LD_PROD = 1, LD_CROSS = 2, LD_BG = 3, LD_MAXW = 4,
-              // kernel template value only: each job's own load_op (PLAIN, PROD
-              // or MAXW) chosen at run time, so first-derivative jobs of
-              // different load operations share one launch
-              LD_ANY = 5,
+enum LoadOp { LD_PLAIN = 0, LD_CROSS = 1,
               // kernel template value only: three LD_CROSS jobs that are the
               // components of one cross product a x b, job q loading
               // {a_{q+1}, b_{q+2}, a_{q+2}, b_{q+1}} (indices mod 3); the six
               // factor lines of a line group are loaded once for all three
-              LD_CROSS3 = 6,
-              // kernel template value only: first derivatives of the three
-              // Maxwell-stress loads of one direction, PROD(b1, b0) or PROD(b0, b1),
-              // PROD(b2, b0) and MAXW(b0, b1, b2) (SpecLaunch::bpat), from one
-              // load of the three field components per line group
-              LD_BSTRESS = 7 };
+              LD_CROSS3 = 2 };
+// A second-derivative job may carry a second, auxiliary line a whose first
+// derivative joins its second output, out[1] = mul[1](in) + d1(a):
+//   AUX_PROD  a = ascale*(b_i+m_i)*(b_j+m_j) + xcoef*xin     (i, j = ai, aj)
+//   AUX_MAXW  a = ascale*((b_i+m_i)^2 - (b_j+m_j)^2 - (b_l+m_l)^2) + xcoef*xin
+// with b the launch's three field components (SpecLaunch::bf, bmean).  The
+// multipliers are linear, so the Maxwell stress and the composite viscous flux
+// of a momentum component need no transform back, store and re-read of their
+// own: one inverse transform returns the sum.
+enum AuxOp { AUX_NONE = 0, AUX_PROD = 1, AUX_MAXW = 2 };
 
 constexpr int SPEC_MAX_JOBS = 8;
 // lengths without a register-blocked plan: run-time radix plans up to this length
@@ -54,7 +51,11 @@ struct SpecJob {
     const void* jin;
     const double* jcoef;
     double mc[2];     // MUL_D2C coefficients
-    const double* bg; // optional per-plane value subtracted on load (nz entries)
+    int aux;          // AuxOp (SM_DERIV2 with out[1])
+    int ai, aj;       // its field components
+    double ascale;
+    const void* xin;  // its further term xcoef * xin, or null
+    double xcoef;
     void* out[2];     // SM_DERIV2: out[1] may be null (the job's first derivative only)
     int out_f32;
     int mul[2];       // MulKind for out[0], out[1] (SM_DERIV*)
@@ -68,6 +69,11 @@ struct SpecLaunch {
     int mode;         // SpecMode
     int njobs;
     SpecJob job[SPEC_MAX_JOBS];
+    // SM_DERIV2: field components of the jobs' auxiliary lines and their
+    // per-plane means (null: none); jobs with an auxiliary line come first
+    const void* bf[3];
+    const double* bmean[3];
+    int split;        // SM_DERIV2, set by the launcher: an item is one job of a line group, not all
     double cx;        // 2*pi/xmax (dir x) or 2*pi/ymax (dir y): mode m has wavenumber m*cx
     const void* tw;   // W_N^t table in the compute type
     int icut;         // dealias cut-off (n/2)/3
@@ -76,10 +82,7 @@ struct SpecLaunch {
     int variant;      // radix plan: 0 the default, 1 and 2 the length's alternatives (if any)
     int max_groups;   // optional further cap on the grid; 0 = none
     int group_major;  // set by the launcher: items ordered line group first (see spec_kernel)
-    int any_load;     // set by the launcher: jobs of mixed load operations in one LD_ANY launch
     int cross3;       // set by the launcher: the three jobs form one cross product (LD_CROSS3)
-    int bstress;      // set by the launcher: the three jobs are Maxwell-stress loads (LD_BSTRESS)
-    int bpat;         // ... job 0 is PROD(b1, b0) (0) or PROD(b0, b1) (1)
     // set by the launcher for lengths without a register-blocked plan: the
     // run-time radices and the complex lines per workgroup
     int gen_radix[SPEC_GEN_MAX_PASSES];

@@ -231,16 +231,45 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
                 constexpr int NOUT = (MODE == SM_DERIV2) ? 2 : 1;
                 for (int o = 0; o < NOUT; ++o) {
                     if (o == 1 && out1 == nullptr) break;   // a first-derivative job (uniform)
-                    // multiplied spectrum into `other`, inverse through buf2
+                    cpx<TC>* aux = nullptr;
+                    cpx<TC>* work = buf2;
+                    if (o == 1 && J.aux) {
+                        // the auxiliary line's spectrum
+                        for (int q = threadIdx.x; q < P; q += GNT) {
+                            int b, n;
+                            point(q, b, n);
+                            long ia, ib, st;
+                            int k;
+                            cpx<TC> v = {(TC)0, (TC)0};
+                            if (GenLines<DIR>::base(g, nlb, grp, b, ia, ib, st, k)) {
+                                const AuxLoad<TC> al(L, J, k);
+                                const TC* __restrict__ p0 = (const TC*)L.bf[al.ai];
+                                const TC* __restrict__ p1 = (const TC*)L.bf[al.aj];
+                                const TC* __restrict__ p2 = (const TC*)L.bf[al.al];
+                                const TC* __restrict__ px = (const TC*)J.xin;
+                                const long i = ia + n * st, e = ib + n * st;
+                                const bool mw = J.aux == AUX_MAXW;
+                                v = {al.one(p0[i], p1[i], mw ? p2[i] : (TC)0, px ? px[i] : (TC)0),
+                                     al.one(p0[e], p1[e], mw ? p2[e] : (TC)0, px ? px[e] : (TC)0)};
+                            }
+                            other[b * N + n] = v;
+                        }
+                        __syncthreads();
+                        aux = gen_fft<TC, false>(other, buf2, twl, L, N, nlb);
+                        work = aux == other ? buf2 : other;
+                    }
+                    // multiplied spectrum into `dst`, inverse through `work`
+                    cpx<TC>* dst = aux ? aux : other;
                     for (int q = threadIdx.x; q < P; q += GNT) {
-                        const int b = q / N, kk = q - b * N;
-                        other[q] = apply_mul_rt<TC>(J.mul[o], spec[q], kk, N, L.cx, L.icut, J.mc);
-                        (void)b;
+                        const int kk = q % N;
+                        cpx<TC> m = apply_mul_rt<TC>(J.mul[o], spec[q], kk, N, L.cx, L.icut, J.mc);
+                        if (aux) m = cadd(m, apply_mul_rt<TC>(MUL_D1, aux[q], kk, N, L.cx, L.icut, J.mc));
+                        dst[q] = m;
                     }
                     __syncthreads();
-                    const cpx<TC>* res = gen_fft<TC, true>(other, buf2, twl, L, N, nlb);
+                    const cpx<TC>* res = gen_fft<TC, true>(dst, work, twl, L, N, nlb);
                     store(res, o == 0 ? out0 : out1, (TC)1);
-                    __syncthreads();   // `other` and buf2 are reused by the next output
+                    __syncthreads();   // the buffers are reused by the next output
                 }
             }
         }
@@ -276,11 +305,7 @@ int gen_mode(const SpecLaunch& L, hipStream_t s)
 {
     switch (L.mode * 8 + L.job[0].load_op) {
     case SM_DERIV1 * 8 + LD_PLAIN: return gen_launch<TC, DIR, SM_DERIV1, LD_PLAIN>(L, s);
-    case SM_DERIV1 * 8 + LD_PROD: return gen_launch<TC, DIR, SM_DERIV1, LD_PROD>(L, s);
-    case SM_DERIV1 * 8 + LD_BG: return gen_launch<TC, DIR, SM_DERIV1, LD_BG>(L, s);
-    case SM_DERIV1 * 8 + LD_MAXW: return gen_launch<TC, DIR, SM_DERIV1, LD_MAXW>(L, s);
     case SM_DERIV2 * 8 + LD_PLAIN: return gen_launch<TC, DIR, SM_DERIV2, LD_PLAIN>(L, s);
-    case SM_DERIV2 * 8 + LD_BG: return gen_launch<TC, DIR, SM_DERIV2, LD_BG>(L, s);
     case SM_R2HC * 8 + LD_PLAIN: return gen_launch<TC, DIR, SM_R2HC, LD_PLAIN>(L, s);
     case SM_R2HC * 8 + LD_CROSS: return gen_launch<TC, DIR, SM_R2HC, LD_CROSS>(L, s);
     case SM_HC2R * 8 + LD_PLAIN: return gen_launch<TC, DIR, SM_HC2R, LD_PLAIN>(L, s);

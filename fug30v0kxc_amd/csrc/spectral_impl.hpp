@@ -63,18 +63,13 @@ __device__ __forceinline__ void st_nt(TC* __restrict__ p, long i, TC a)
     __builtin_nontemporal_store(a, p + i);
 }
 
-// Input loaders, fixed at compile time per launch.  Inputs have the compute
-// type TC, except LD_BG, which reads the FP64 state and subtracts a per-plane
-// background in FP64 before rounding to TC.
+// Input loaders, fixed at compile time per launch; inputs have the compute type.
 template <typename TC, int LOP>
 struct Loader {
     const TC* __restrict__ a;
     const TC* __restrict__ b;
     const TC* __restrict__ c;
     const TC* __restrict__ d;
-    const double* __restrict__ s64;
-    TC scale;
-    double bgk;
     TC m0, m1, m2, m3;   // per-plane means of the factors (0 when absent)
     const TC* __restrict__ jj;   // LD_CROSS: current density component, or null
     TC jc;                       // its per-plane coefficient
@@ -84,9 +79,6 @@ struct Loader {
         b = (const TC*)J.in[1];
         c = (const TC*)J.in[2];
         d = (const TC*)J.in[3];
-        s64 = (const double*)J.in[0];
-        scale = (TC)J.scale;
-        bgk = (LOP == LD_BG && J.bg) ? J.bg[k] : 0.0;
         m0 = m1 = m2 = m3 = (TC)0;
         jj = nullptr;
         jc = (TC)0;
@@ -95,8 +87,6 @@ struct Loader {
                 jj = (const TC*)J.jin;
                 jc = (TC)J.jcoef[k];
             }
-        }
-        if constexpr (LOP == LD_PROD || LOP == LD_CROSS || LOP == LD_MAXW) {
             if (J.mean[0]) m0 = (TC)J.mean[0][k];
             if (J.mean[1]) m1 = (TC)J.mean[1][k];
             if (J.mean[2]) m2 = (TC)J.mean[2][k];
@@ -107,40 +97,7 @@ struct Loader {
     __device__ __forceinline__ cpx<TC> pair(long i) const
     {
         if constexpr (LOP == LD_PLAIN) return ld_pair(a, i);
-        else if constexpr (LOP == LD_BG) {
-            const cpx<double> v = ld_pair(s64, i);
-            return {(TC)(v.x - bgk), (TC)(v.y - bgk)};
-        } else if constexpr (LOP == LD_PROD) {
-            const cpx<TC> x = ld_pair(a, i), y = ld_pair(b, i);
-            return {(scale * x.x) * y.x + scale * (x.x * m1 + m0 * y.x),
-                    (scale * x.y) * y.y + scale * (x.y * m1 + m0 * y.y)};
-        } else if constexpr (LOP == LD_MAXW) {
-            const cpx<TC> x = ld_pair(a, i), y = ld_pair(b, i), z = ld_pair(c, i);
-            return {scale * x.x * x.x - scale * y.x * y.x - scale * z.x * z.x +
-                        (TC)2 * scale * (m0 * x.x - m1 * y.x - m2 * z.x),
-                    scale * x.y * x.y - scale * y.y * y.y - scale * z.y * z.y +
-                        (TC)2 * scale * (m0 * x.y - m1 * y.y - m2 * z.y)};
-        } else {
-            return cross_pair(ld_pair(a, i), ld_pair(b, i), ld_pair(c, i), ld_pair(d, i), i);
-        }
-    }
-    // PLAIN, PROD or MAXW from factor values already loaded (x = in0, y = in1,
-    // z = in2; both elements of a pair), the arithmetic of pair()
-    __device__ __forceinline__ cpx<TC> combine(cpx<TC> x, cpx<TC> y, cpx<TC> z) const
-    {
-        if constexpr (LOP == LD_PROD) {
-            return {(scale * x.x) * y.x + scale * (x.x * m1 + m0 * y.x),
-                    (scale * x.y) * y.y + scale * (x.y * m1 + m0 * y.y)};
-        } else if constexpr (LOP == LD_MAXW) {
-            return {scale * x.x * x.x - scale * y.x * y.x - scale * z.x * z.x +
-                        (TC)2 * scale * (m0 * x.x - m1 * y.x - m2 * z.x),
-                    scale * x.y * x.y - scale * y.y * y.y - scale * z.y * z.y +
-                        (TC)2 * scale * (m0 * x.y - m1 * y.y - m2 * z.y)};
-        } else {
-            (void)y;
-            (void)z;
-            return x;
-        }
+        else return cross_pair(ld_pair(a, i), ld_pair(b, i), ld_pair(c, i), ld_pair(d, i), i);
     }
     // LD_CROSS from factor values already loaded (x = in0, y = in1, z = in2,
     // w = in3 at element i), the extra term loaded here
@@ -164,18 +121,46 @@ struct Loader {
     __device__ __forceinline__ TC operator()(long i) const
     {
         if constexpr (LOP == LD_PLAIN) return a[i];
-        else if constexpr (LOP == LD_BG) return (TC)(s64[i] - bgk);
-        else if constexpr (LOP == LD_PROD) {
-            // (s*a)*b is the reference's product; the mean terms drop its constant
-            const TC x = a[i], y = b[i];
-            return (scale * x) * y + scale * (x * m1 + m0 * y);
-        } else if constexpr (LOP == LD_MAXW) {
-            const TC x = a[i], y = b[i], z = c[i];
-            return scale * x * x - scale * y * y - scale * z * z +
-                   (TC)2 * scale * (m0 * x - m1 * y - m2 * z);
-        } else {
-            return cross(a[i], b[i], c[i], d[i], i);
-        }
+        else return cross(a[i], b[i], c[i], d[i], i);
+    }
+};
+
+// A job's auxiliary line (SpecJob::aux) of one plane: the Maxwell-stress load
+// from field components x = b_ai, y = b_aj, z = b_al (l the third; AUX_MAXW
+// only) and the further term's q, with the components' per-plane means.
+// (s*x)*y is the reference's product; the mean terms drop its constant.
+template <typename TC>
+struct AuxLoad {
+    TC s, mi, mj, ml, xc;
+    int op, ai, aj, al;
+    bool xin;
+    __device__ __forceinline__ AuxLoad(const SpecLaunch& L, const SpecJob& J, int k)
+    {
+        op = J.aux;
+        ai = op ? J.ai : 0;
+        aj = op == AUX_PROD ? J.aj : (ai + 1) % 3;
+        al = 3 - ai - aj;
+        s = (TC)J.ascale;
+        xin = op && J.xin;
+        xc = (TC)J.xcoef;
+        mi = ml = mj = (TC)0;
+        if (!op) return;
+        mi = L.bmean[ai] ? (TC)L.bmean[ai][k] : (TC)0;
+        mj = L.bmean[aj] ? (TC)L.bmean[aj][k] : (TC)0;
+        ml = L.bmean[al] ? (TC)L.bmean[al][k] : (TC)0;
+    }
+    // from the three components of an element
+    __device__ __forceinline__ TC pick(TC b0, TC b1, TC b2, TC q) const
+    {
+        return one(ai == 0 ? b0 : ai == 1 ? b1 : b2, aj == 0 ? b0 : aj == 1 ? b1 : b2, al == 0 ? b0 : al == 1 ? b1 : b2,
+                   q);
+    }
+    __device__ __forceinline__ TC one(TC x, TC y, TC z, TC q) const
+    {
+        TC v;
+        if (op == AUX_PROD) v = (s * x) * y + s * (x * mj + mi * y);
+        else v = s * x * x - s * y * y - s * z * z + (TC)2 * s * (mi * x - mj * y - ml * z);
+        return xin ? v + xc * q : v;
     }
 };
 
@@ -250,12 +235,9 @@ struct Lines {
 // are loaded into registers before the current item is transformed, and the
 // transform touches only registers and LDS (twiddles are staged in LDS), so
 // the loads of item i+1 are in flight while item i is computed and stored.
-// With L.group_major (a persistent grid smaller than the items), item i of
-// round r = i / (G njobs) is job (i mod G njobs) / G of line group
-// r G + i mod G: a workgroup then does every job of one line group back to
-// back, so jobs that load the same fields (the cross products of u and B)
-// find the lines in their CU's caches instead of re-reading HBM.
 //
+// SM_DERIV2 runs body_deriv2 instead: an item is every job of one line group
+// (or, with L.split, one job of one group).
 // LOP = LD_CROSS3 (SM_R2HC, three jobs forming one cross product) runs
 // body_cross3 instead: an item is one line group, whose six factor lines are
 // loaded once and combined into the three jobs' inputs.
@@ -271,10 +253,10 @@ struct SpecK {
     static __device__ __forceinline__ void body(const SpecLaunch& L, uint3 bid, uint3 gdim)
     {
         if constexpr (LOP == LD_CROSS3) body_cross3(L, bid, gdim);
-        else if constexpr (LOP == LD_BSTRESS) body_bstress(L, bid, gdim);
+        else if constexpr (MODE == SM_DERIV2) body_deriv2(L, bid, gdim);
         else body_jobs(L, bid, gdim);
     }
-    static __device__ __forceinline__ void body_bstress(const SpecLaunch& L, uint3 bid, uint3 gdim);
+    static __device__ __forceinline__ void body_deriv2(const SpecLaunch& L, uint3 bid, uint3 gdim);
     static __device__ __forceinline__ void body_jobs(const SpecLaunch& L, uint3 bid, uint3 gdim);
     static __device__ __forceinline__ void body_cross3(const SpecLaunch& L, uint3 bid, uint3 gdim);
     // Column groups narrower than a 128-byte line (y, 2 B sizeof(TC) < 128
@@ -412,14 +394,15 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_cross3(co
     }
 }
 
-// The first derivatives of the three Maxwell-stress loads of a direction: an
-// item is one line group; the three field components b0, b1, b2 (job 2's
-// inputs) are loaded once, each job's input formed from them with the job's
-// own means and scale (the arithmetic of the per-job loader), and the three
-// transforms run back to back.
+// First and second derivatives (SM_DERIV2), with the auxiliary lines of
+// SpecJob::aux.  An item is one line group: its field components b0, b1, b2 are
+// loaded once, then its jobs run back to back, each with its line (and extra
+// term) loaded during the job before it, and the next item's components during
+// the jobs without an auxiliary line, which come last.  With L.split an item is
+// one job of one line group (boxes with too few line groups to fill the device).
 template <typename TC, typename PL, int DIR, int B, int MODE, int LOP>
-__device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_bstress(const SpecLaunch& L, uint3 bid,
-                                                                               uint3 gdim)
+__device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_deriv2(const SpecLaunch& L, uint3 bid,
+                                                                              uint3 gdim)
 {
     constexpr int N = PL::N;
     using LN = Lines<PL, DIR, B>;
@@ -434,85 +417,121 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_bstress(c
     cpx<TC>* lds = twl + F::TWN + t * F::SP;
     const long ngrp = LN::groups(g);
     const long G = gdim.x;
+    const int nj = L.njobs;
+    const bool split = L.split != 0;
+    const long nitems = split ? ngrp * nj : ngrp;
     const double cx = L.cx;
     const int icut = L.icut;
-    const TC* __restrict__ f0 = (const TC*)L.job[2].in[0];
-    const TC* __restrict__ f1 = (const TC*)L.job[2].in[1];
-    const TC* __restrict__ f2 = (const TC*)L.job[2].in[2];
-    const bool pat = L.bpat != 0;   // job 0 is PROD(b0, b1) rather than PROD(b1, b0)
     __syncthreads();
 
-    auto fetch = [&](long grp, cpx<TC> (*dst)[R0]) {
+    // first job and line group of an item
+    auto decode = [&](long item, int& q0, long& grp) {
+        q0 = split ? (int)(item / ngrp) : 0;
+        grp = paired_group(item - (long)q0 * ngrp, G, ngrp);
+    };
+    auto load = [&](const TC* __restrict__ p, long grp, cpx<TC>* dst) {
         long ia, ib, st;
         int k;
         const bool ok = LN::base(g, grp, t, ia, ib, st, k);
-        const Loader<TC, LD_PROD> l0(L.job[0], ok ? k : 0), l1(L.job[1], ok ? k : 0);
-        const Loader<TC, LD_MAXW> l2(L.job[2], ok ? k : 0);
 #pragma unroll
         for (int r = 0; r < R0; ++r) {
-            const int n = j + r * NB0;
-            dst[0][r] = dst[1][r] = dst[2][r] = {(TC)0, (TC)0};
+            const long n = (long)(j + r * NB0) * st;
+            dst[r] = {(TC)0, (TC)0};
             if (ok && j < NB0) {
-                cpx<TC> a, b, c;
-                if constexpr (DIR == 1) {
-                    const long i = ia + n * st;
-                    a = ld_pair(f0, i);
-                    b = ld_pair(f1, i);
-                    c = ld_pair(f2, i);
-                } else {
-                    const long i = ia + n * st, e = ib + n * st;
-                    a = {f0[i], f0[e]};
-                    b = {f1[i], f1[e]};
-                    c = {f2[i], f2[e]};
-                }
-                dst[0][r] = pat ? l0.combine(a, b, c) : l0.combine(b, a, c);
-                dst[1][r] = l1.combine(c, a, b);
-                dst[2][r] = l2.combine(a, b, c);
+                if constexpr (DIR == 1) dst[r] = ld_pair(p, ia + n);
+                else dst[r] = {p[ia + n], p[ib + n]};
             }
         }
     };
+    cpx<TC> f[R0], x[R0], b0[R0], b1[R0], b2[R0];
+    auto load_job = [&](int q, long grp) {
+        load((const TC*)L.job[q].in[0], grp, f);
+        if (L.job[q].xin) load((const TC*)L.job[q].xin, grp, x);
+    };
+    auto load_b = [&](long grp) {
+        load((const TC*)L.bf[0], grp, b0);
+        load((const TC*)L.bf[1], grp, b1);
+        load((const TC*)L.bf[2], grp, b2);
+    };
 
-    cpx<TC> nxt[3][R0];
     long item = bid.x;
-    if (item < ngrp) fetch(paired_group(item, G, ngrp), nxt);
-    for (; item < ngrp; item += G) {
-        const long grp = paired_group(item, G, ngrp);
-        cpx<TC> cur[3][R0];
-#pragma unroll
-        for (int q = 0; q < 3; ++q)
-#pragma unroll
-            for (int r = 0; r < R0; ++r) cur[q][r] = nxt[q][r];
+    int q0 = 0;
+    long grp = 0;
+    if (item < nitems) {
+        decode(item, q0, grp);
+        load_job(q0, grp);
+        if (L.job[q0].aux) load_b(grp);
+    }
+    while (item < nitems) {
         long ia, ib, st;
         int k;
         const bool ok = LN::base(g, grp, t, ia, ib, st, k);
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
+        const int q1 = split ? q0 + 1 : nj;
+        int nq0 = 0;
+        long ngroup = 0;
+        const long next = item + G;
+        if (next < nitems) decode(next, nq0, ngroup);
+        bool b_next = next < nitems && L.job[nq0].aux != AUX_NONE;   // components still to be loaded
+        for (int q = q0; q < q1; ++q) {
             const SpecJob& J = L.job[q];
-            // the next group's loads fly during the last job's transform
-            if (q == 2 && item + G < ngrp) fetch(paired_group(item + G, G, ngrp), nxt);
-            cpx<TC> v[F::RMAX];
+            cpx<TC> v[F::RMAX], a[R0];
 #pragma unroll
-            for (int r = 0; r < R0; ++r) v[r] = cur[q][r];
-            F::forward(v, j, lds, twl);
-            if (j < NBL) {
-#pragma unroll
-                for (int r = 0; r < RL; ++r) v[r] = apply_mul<TC, N>(J.mul[0], v[r], j + r * NBL, cx, icut, J.mc);
-            }
-            F::inverse(v, j, lds, twl);
-            if (ok && j < NB0) {
-                TC* __restrict__ out = (TC*)J.out[0];
-                const TC add = (J.addk ? (TC)J.addk[k] : (TC)0) + (TC)J.adds;
+            for (int r = 0; r < R0; ++r) v[r] = f[r];
+            if (J.aux) {
+                const AuxLoad<TC> al(L, J, ok ? k : 0);
 #pragma unroll
                 for (int r = 0; r < R0; ++r) {
-                    const int n = j + r * NB0;
-                    if constexpr (DIR == 1) st_pair_nt(out, ia + n * st, v[r].x + add, v[r].y + add);
-                    else {
-                        st_nt(out, ia + n * st, v[r].x + add);
-                        st_nt(out, ib + n * st, v[r].y + add);
+                    a[r].x = al.pick(b0[r].x, b1[r].x, b2[r].x, x[r].x);
+                    a[r].y = al.pick(b0[r].y, b1[r].y, b2[r].y, x[r].y);
+                }
+            }
+            if (q + 1 < q1) load_job(q + 1, grp);
+            else if (next < nitems) load_job(nq0, ngroup);
+            if (b_next && (q + 1 == q1 || !L.job[q + 1].aux)) {
+                load_b(ngroup);
+                b_next = false;
+            }
+            F::forward(v, j, lds, twl);
+            cpx<TC> z[RL], w[RL];
+#pragma unroll
+            for (int r = 0; r < RL; ++r) z[r] = v[r];
+            if (J.aux) {
+#pragma unroll
+                for (int r = 0; r < R0; ++r) v[r] = a[r];
+                F::forward(v, j, lds, twl);
+#pragma unroll
+                for (int r = 0; r < RL; ++r) w[r] = v[r];
+            }
+            auto second = [&](int r) {
+                const int kk = j + r * NBL;
+                const cpx<TC> d2 = apply_mul<TC, N>(J.mul[1], z[r], kk, cx, icut, J.mc);
+                return J.aux ? cadd(d2, apply_mul<TC, N>(MUL_D1, w[r], kk, cx, icut, J.mc)) : d2;
+            };
+            for (int o = 0; o < 2; ++o) {
+                if (o == 1 && !J.out[1]) break;   // a first-derivative job (uniform)
+#pragma unroll
+                for (int r = 0; r < RL; ++r) {
+                    if (o == 0) v[r] = apply_mul<TC, N>(J.mul[0], z[r], j + r * NBL, cx, icut, J.mc);
+                    else v[r] = second(r);
+                }
+                F::inverse(v, j, lds, twl);
+                if (ok && j < NB0) {
+                    TC* __restrict__ out = (TC*)J.out[o];
+#pragma unroll
+                    for (int r = 0; r < R0; ++r) {
+                        const int n = j + r * NB0;
+                        if constexpr (DIR == 1) st_pair_nt(out, ia + n * st, v[r].x, v[r].y);
+                        else {
+                            st_nt(out, ia + n * st, v[r].x);
+                            st_nt(out, ib + n * st, v[r].y);
+                        }
                     }
                 }
             }
         }
+        item = next;
+        q0 = nq0;
+        grp = ngroup;
     }
 }
 
@@ -533,8 +552,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
     cpx<TC>* lds = twl + F::TWN + t * F::SP;
     const long ngrp = LN::groups(g);
     const long G = gdim.x;
-    const bool gmaj = L.group_major != 0;
-    const long nitems = gmaj ? ((ngrp + G - 1) / G) * G * L.njobs : ngrp * L.njobs;
+    const long nitems = ngrp * L.njobs;
     const double cx = L.cx;
     const int icut = L.icut;
     __syncthreads();
@@ -545,31 +563,22 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
     // c + 8 group 2c + 1: workgroups w and w + 8 run on the same XCD (they are
     // dealt round-robin over 8) at the same time, so a line is fetched once.
     constexpr bool half_line = DIR == 1 && 2 * B * (int)sizeof(TC) < 128;
-    const bool pair = half_line && !gmaj && (G % 16 == 0) && (ngrp % 16 == 0);
-    // (job, line group) of an item; false for the padding of the last round
-    auto decode = [&](long item, int& jb, long& grp) -> bool {
-        if (!gmaj) {
-            if (pair) {
-                const long c = item & 15;
-                item = item - c + (c < 8 ? 2 * c : 2 * (c - 8) + 1);
-            }
-            jb = (int)(item / ngrp);
-            grp = item - (long)jb * ngrp;
-            return true;
+    const bool pair = half_line && (G % 16 == 0) && (ngrp % 16 == 0);
+    // (job, line group) of an item
+    auto decode = [&](long item, int& jb, long& grp) {
+        if (pair) {
+            const long c = item & 15;
+            item = item - c + (c < 8 ? 2 * c : 2 * (c - 8) + 1);
         }
-        const long per = G * L.njobs;
-        const long r = item / per;
-        const long rem = item - r * per;
-        jb = (int)(rem / G);
-        grp = r * G + (rem - (long)jb * G);
-        return grp < ngrp;
+        jb = (int)(item / ngrp);
+        grp = item - (long)jb * ngrp;
     };
 
     // pass-0 inputs of one item (zeros for lines past the end)
     auto fetch = [&](long item, cpx<TC>* dst) {
         int jb;
         long grp;
-        if (!decode(item, jb, grp)) return;
+        decode(item, jb, grp);
         const SpecJob& J = L.job[jb];
         long ia, ib, st;
         int k;
@@ -586,26 +595,15 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
                 }
             }
         } else {
-            auto load_with = [&](auto op) {
-                constexpr int LO = decltype(op)::value;
-                const Loader<TC, LO> ld(J, ok ? k : 0);
+            const Loader<TC, LOP> ld(J, ok ? k : 0);
 #pragma unroll
-                for (int r = 0; r < R0; ++r) {
-                    const int n = j + r * NB0;
-                    dst[r] = {(TC)0, (TC)0};
-                    if (ok && j < NB0) {
-                        if constexpr (DIR == 1) dst[r] = ld.pair(ia + n * st);
-                        else dst[r] = {ld(ia + n * st), ld(ib + n * st)};
-                    }
+            for (int r = 0; r < R0; ++r) {
+                const int n = j + r * NB0;
+                dst[r] = {(TC)0, (TC)0};
+                if (ok && j < NB0) {
+                    if constexpr (DIR == 1) dst[r] = ld.pair(ia + n * st);
+                    else dst[r] = {ld(ia + n * st), ld(ib + n * st)};
                 }
-            };
-            if constexpr (LOP == LD_ANY) {
-                // the job's load operation, uniform over the workgroup
-                if (J.load_op == LD_PROD) load_with(std::integral_constant<int, LD_PROD>());
-                else if (J.load_op == LD_MAXW) load_with(std::integral_constant<int, LD_MAXW>());
-                else load_with(std::integral_constant<int, LD_PLAIN>());
-            } else {
-                load_with(std::integral_constant<int, LOP>());
             }
         }
     };
@@ -621,13 +619,12 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
 
         int jb;
         long grp;
-        if (!decode(item, jb, grp)) continue;   // uniform over the workgroup
+        decode(item, jb, grp);
         const SpecJob& J = L.job[jb];
         long ia, ib, st;
         int k;
         const bool ok = LN::base(g, grp, t, ia, ib, st, k);
         TC* __restrict__ out0 = (TC*)J.out[0];
-        TC* __restrict__ out1 = (TC*)J.out[1];
         // epilogue constant of this line pair (one plane): the mean parts of B
         const TC add = (J.addk && ok ? (TC)J.addk[k] : (TC)0) + (TC)J.adds;
 
@@ -670,31 +667,20 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
             if constexpr (MODE == SM_R2HC) {
                 r2hc_store(v, j, lds, ok, out0, ia, ib, st);
             } else {
-                constexpr int NOUT = (MODE == SM_DERIV2) ? 2 : 1;
-                cpx<TC> z[RL];
-                if constexpr (NOUT == 2) {
+                if (j < NBL) {
 #pragma unroll
-                    for (int r = 0; r < RL; ++r) z[r] = v[r];
+                    for (int r = 0; r < RL; ++r)
+                        v[r] = apply_mul<TC, N>(J.mul[0], v[r], j + r * NBL, cx, icut, J.mc);
                 }
+                F::inverse(v, j, lds, twl);
+                if (ok && j < NB0) {
 #pragma unroll
-                for (int o = 0; o < NOUT; ++o) {
-                    if (o == 1 && out1 == nullptr) break;   // a first-derivative job (uniform)
-                    if (j < NBL) {
-#pragma unroll
-                        for (int r = 0; r < RL; ++r)
-                            v[r] = apply_mul<TC, N>(J.mul[o], o == 0 ? v[r] : z[r], j + r * NBL, cx, icut, J.mc);
-                    }
-                    F::inverse(v, j, lds, twl);
-                    if (ok && j < NB0) {
-                        TC* __restrict__ out = (o == 0) ? out0 : out1;
-#pragma unroll
-                        for (int r = 0; r < R0; ++r) {
-                            const int n = j + r * NB0;
-                            if constexpr (DIR == 1) st_pair_nt(out, ia + n * st, v[r].x + add, v[r].y + add);
-                            else {
-                                st_nt(out, ia + n * st, v[r].x + add);
-                                st_nt(out, ib + n * st, v[r].y + add);
-                            }
+                    for (int r = 0; r < R0; ++r) {
+                        const int n = j + r * NB0;
+                        if constexpr (DIR == 1) st_pair_nt(out0, ia + n * st, v[r].x + add, v[r].y + add);
+                        else {
+                            st_nt(out0, ia + n * st, v[r].x + add);
+                            st_nt(out0, ib + n * st, v[r].y + add);
                         }
                     }
                 }
@@ -742,8 +728,7 @@ static int launch_one(const SpecLaunch& L, hipStream_t s)
     constexpr size_t lds = spec_lds_bytes<TC, PL, B>();
     static_assert(lds <= (size_t)SPEC_LDS_Y, "transform workgroup exceeds 160 KB of LDS");
     auto kern = single_kernel<K>;
-    // LD_CROSS3, LD_BSTRESS: one item per line group for all three jobs
-    const long items = Lines<PL, DIR, B>::groups(L.g) * (LOP == LD_CROSS3 || LOP == LD_BSTRESS ? 1 : L.njobs);
+    const long ngrp = Lines<PL, DIR, B>::groups(L.g);
     // more than 64 KB of dynamic LDS is opted into once per kernel
     static int lds_ok = lds <= 65536 ? 1 : 0;
     if (!lds_ok) {
@@ -759,15 +744,24 @@ static int launch_one(const SpecLaunch& L, hipStream_t s)
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, NT, lds) != hipSuccess || n < 1) n = 1;
         per_cu = n;
     }
-    long grid = items;
     const long resident = (long)per_cu * L.ncu * (L.grid_mult > 1 ? L.grid_mult : 1);
+    SpecLaunch La = L;
+    // items: the (job, line group) pairs, or line groups whose jobs share loads;
+    // second derivatives share them where the line groups alone fill the device
+    if (MODE == SM_DERIV2) {
+        La.split = L.njobs == 1 || ngrp < resident;
+        // two different field components, all three present
+        for (int q = 0; q < L.njobs; ++q) {
+            const SpecJob& J = L.job[q];
+            if (!J.aux) continue;
+            if (!L.bf[0] || !L.bf[1] || !L.bf[2] || !J.out[1] || J.ai < 0 || J.ai > 2) return -23;
+            if (J.aux == AUX_PROD && (J.aj < 0 || J.aj > 2 || J.aj == J.ai)) return -23;
+        }
+    }
+    const bool shared = LOP == LD_CROSS3 || (MODE == SM_DERIV2 && !La.split);
+    long grid = ngrp * (shared ? 1 : L.njobs);
     if (L.ncu > 0 && grid > resident) grid = resident;
     if (L.max_groups > 0 && grid > L.max_groups) grid = L.max_groups;
-    // line group first only for the FP64 EMF pass, whose three jobs load the same
-    // six fields (at 256^2 x 160: 235 -> 191 us); with independent inputs, and in
-    // FP32, the job-major order measured 5-10 % faster
-    SpecLaunch La = L;
-    La.group_major = grid < items && L.njobs > 1 && LOP == LD_CROSS && sizeof(TC) == 8;
     return mhd_launch<K>(dim3((unsigned)grid), dim3(NT), lds, s, La);
 }
 
@@ -775,40 +769,17 @@ static int launch_one(const SpecLaunch& L, hipStream_t s)
 template <typename TC, typename PL, int DIR, int B>
 static int launch_mode(const SpecLaunch& L, hipStream_t s)
 {
-    if (L.any_load) return launch_one<TC, PL, DIR, B, SM_DERIV1, LD_ANY>(L, s);
-    if (L.bstress) return launch_one<TC, PL, DIR, B, SM_DERIV1, LD_BSTRESS>(L, s);
     if constexpr (DIR == 0) {
         if (L.cross3) return launch_one<TC, PL, DIR, B, SM_R2HC, LD_CROSS3>(L, s);
     }
     const int lop = L.job[0].load_op;
     switch (L.mode * 8 + lop) {
     case SM_DERIV1 * 8 + LD_PLAIN: return launch_one<TC, PL, DIR, B, SM_DERIV1, LD_PLAIN>(L, s);
-    case SM_DERIV1 * 8 + LD_PROD: return launch_one<TC, PL, DIR, B, SM_DERIV1, LD_PROD>(L, s);
-    case SM_DERIV1 * 8 + LD_BG: return launch_one<TC, PL, DIR, B, SM_DERIV1, LD_BG>(L, s);
-    case SM_DERIV1 * 8 + LD_MAXW: return launch_one<TC, PL, DIR, B, SM_DERIV1, LD_MAXW>(L, s);
     case SM_DERIV2 * 8 + LD_PLAIN: return launch_one<TC, PL, DIR, B, SM_DERIV2, LD_PLAIN>(L, s);
-    case SM_DERIV2 * 8 + LD_BG: return launch_one<TC, PL, DIR, B, SM_DERIV2, LD_BG>(L, s);
     case SM_R2HC * 8 + LD_PLAIN: return launch_one<TC, PL, DIR, B, SM_R2HC, LD_PLAIN>(L, s);
-    case SM_R2HC * 8 + LD_CROSS: return launch_one<TC, PL, DIR, B, SM_R2HC, LD_CROSS>(L, s);
     case SM_HC2R * 8 + LD_PLAIN: return launch_one<TC, PL, DIR, B, SM_HC2R, LD_PLAIN>(L, s);
     }
     return -23;
-}
-
-// the single-output derivative passes along y (one input, one output per
-// line) with half the column pairs per workgroup (512 threads instead of 1024
-// at 256 points: two workgroups per CU fit where one did)
-template <typename TC, typename PL, int B>
-static int launch_y_deriv1(const SpecLaunch& L, hipStream_t s)
-{
-    if (L.any_load) return launch_one<TC, PL, 1, B, SM_DERIV1, LD_ANY>(L, s);
-    if (L.bstress) return launch_one<TC, PL, 1, B, SM_DERIV1, LD_BSTRESS>(L, s);
-    switch (L.job[0].load_op) {
-    case LD_PLAIN: return launch_one<TC, PL, 1, B, SM_DERIV1, LD_PLAIN>(L, s);
-    case LD_PROD: return launch_one<TC, PL, 1, B, SM_DERIV1, LD_PROD>(L, s);
-    case LD_MAXW: return launch_one<TC, PL, 1, B, SM_DERIV1, LD_MAXW>(L, s);
-    }
-    return launch_mode<TC, PL, 1, B>(L, s);
 }
 
 template <typename TC, typename PL>
@@ -817,18 +788,14 @@ static int launch_plan(const SpecLaunch& L, hipStream_t s)
     if (L.dir == 0) return launch_mode<TC, PL, 0, spec_b<TC, PL, 0>()>(L, s);
     constexpr int B0 = spec_b<TC, PL, 1>();
     // FP32 only, where a full group would be a 1024-thread workgroup (one per
-    // CU): at 256 points 8 pairs beat 16 for these passes (76, 72, 45 us
+    // CU): at 256 points 8 pairs beat 16 for the first derivatives (76, 72, 45 us
     // against 81, 83, 48); in FP64 4 pairs lose to 8.  The other FP32 modes keep
-    // 16 pairs (8 pairs: d1+d2 155 against 137 us, hc2r 125 against 109, r2hc
-    // 63 against 58)
+    // 16 pairs (8 pairs: hc2r 125 against 109, r2hc 63 against 58)
     constexpr int BH = (sizeof(TC) == 4 && B0 >= 8 && B0 * plan_tpt<PL>() >= 1024) ? B0 / 2 : B0;
-    if (BH != B0 && L.mode == SM_DERIV1 && L.g.nx % (2 * BH) == 0) return launch_y_deriv1<TC, PL, BH>(L, s);
-    // FP64 Maxwell-stress triple (about 150 VGPRs): half groups, 3 workgroups
-    // per CU instead of 1 (at 256^2 x 160: 153 against 171 us; the groups
-    // sharing a line are paired onto one XCD, so each line is fetched once)
-    if constexpr (sizeof(TC) == 8 && B0 >= 8) {
-        if (L.bstress && L.g.nx % B0 == 0) return launch_one<TC, PL, 1, B0 / 2, SM_DERIV1, LD_BSTRESS>(L, s);
-    }
+    if (BH != B0 && L.mode == SM_DERIV1 && L.g.nx % (2 * BH) == 0) return launch_one<TC, PL, 1, BH, SM_DERIV1, LD_PLAIN>(L, s);
+    // second derivatives
+    constexpr int B2 = B0 >= 8 && B0 * plan_tpt<PL>() >= (sizeof(TC) == 4 ? 1024 : 512) ? B0 / 2 : B0;
+    if (B2 != B0 && L.mode == SM_DERIV2 && L.g.nx % (2 * B2) == 0) return launch_one<TC, PL, 1, B2, SM_DERIV2, LD_PLAIN>(L, s);
     if (L.g.nx % (2 * B0) == 0) return launch_mode<TC, PL, 1, B0>(L, s);
     return launch_mode<TC, PL, 1, 1>(L, s);
 }
@@ -842,6 +809,7 @@ static int launch_n(const SpecLaunch& L, hipStream_t s)
     if constexpr (!std::is_void<typename AltPlan2<N>::type>::value) {
         if (L.variant == 2) return launch_plan<TC, typename AltPlan2<N>::type>(L, s);
     }
+    if (L.mode == SM_DERIV2) return launch_plan<TC, typename D2Plan<N>::type>(L, s);
     return launch_plan<TC, FftPlan<N>>(L, s);
 }
 
