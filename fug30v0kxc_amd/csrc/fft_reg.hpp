@@ -334,6 +334,14 @@ struct RegFFT {
         }
     }
 
+    // j as a value the compiler cannot hoist from: the addresses and multipliers
+    // computed from it stay inside the loop iteration instead of being kept in
+    // registers across it
+    static __device__ __forceinline__ int own(int j)
+    {
+        asm volatile("" : "+v"(j));
+        return j;
+    }
     // forward: v holds x[j + r*NB0] (j < NB0) -> X[j + r*NBL] (j < NBL)
     static __device__ __forceinline__ void forward(cpx<T>* v, int j, cpx<T>* lds, const cpx<T>* __restrict__ tw)
     {

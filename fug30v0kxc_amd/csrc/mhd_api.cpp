@@ -556,6 +556,24 @@ int run_closure_tend(mhd_ctx* c)
     return kerr(closure_tend(c->n3, c->cdx, c->cdy, c->cdz, wf, c->r, dots, c->h32, c->s));
 }
 
+MagSpecArgs mag_spec_args(mhd_ctx* c, const MagArgs& m)
+{
+    MagSpecArgs a;
+    memset(&a, 0, sizeof(a));
+    a.g = c->g;
+    a.tw = c->twx;
+    a.cx = 8.0 * std::atan(1.0) / c->p.xmax;
+    a.cy = 8.0 * std::atan(1.0) / c->p.ymax;
+    a.icutx = c->icutx;
+    a.icuty = c->icuty;
+    a.ncu = c->ncu;
+    a.ex = m.exh; a.ey = m.eyh; a.ez = m.ezh;
+    a.cc = m.cc; a.d = m.d;
+    a.pol = c->pol; a.tor = c->tor; a.polz = m.polz;
+    a.out[0] = m.bxh; a.out[1] = m.byh; a.out[2] = m.jzh; a.out[3] = m.bzh; a.out[4] = m.dxbzh;
+    return a;
+}
+
 // ---------------------------------------------------------------------------
 // mag_deriv, src/magnetic.f90:285-487
 // ---------------------------------------------------------------------------
@@ -566,8 +584,10 @@ int run_mag_deriv(mhd_ctx* c, const double* cf = nullptr)
     const int wf = c->wf32;
     MagArgs m = margs(c);
     {
-        SpecLaunch L = spec_base(c, 0, SM_R2HC);
-        // E = u x B (308-316), fused into the x pass of forwardfft
+        // E = u x B (308-316), fused into the first pass of forwardfft: y where
+        // the x pass can follow with the spectral derivatives (emf_x), else x
+        const bool fused = spectral_len_fixed(c->nx);
+        SpecLaunch L = spec_base(c, fused ? 1 : 0, SM_R2HC);
         // mixed precision: FP32 velocity shadows, B without its means (added by the loads)
         const bool mx = c->su != nullptr;
         const void* U_ = mx ? (const void*)c->su : c->u;
@@ -599,15 +619,20 @@ int run_mag_deriv(mhd_ctx* c, const double* cf = nullptr)
         }
         L.njobs = 3;
         TRY(spec(c, L));
-        SpecLaunch M = spec_base(c, 1, SM_R2HC);
-        M.job[0] = sjob(m.exh, wf, m.exh, nullptr, 0, 0, wf);
-        M.job[1] = sjob(m.eyh, wf, m.eyh, nullptr, 0, 0, wf);
-        M.job[2] = sjob(m.ezh, wf, m.ezh, nullptr, 0, 0, wf);
-        M.njobs = 3;
-        TRY(spec(c, M));
+        if (fused) {
+            MagSpecArgs x = mag_spec_args(c, m);
+            TRY(kerr(launch_emf_x(x, wf, c->s)));
+        } else {
+            SpecLaunch M = spec_base(c, 1, SM_R2HC);
+            M.job[0] = sjob(m.exh, wf, m.exh, nullptr, 0, 0, wf);
+            M.job[1] = sjob(m.eyh, wf, m.eyh, nullptr, 0, 0, wf);
+            M.job[2] = sjob(m.ezh, wf, m.ezh, nullptr, 0, 0, wf);
+            M.njobs = 3;
+            TRY(spec(c, M));
+            TRY(kerr(launch_mag_spec1(m, c->s)));
+        }
     }
     TRY(kerr(launch_mean_emf(m, c->s)));
-    TRY(kerr(launch_mag_spec1(m, c->s)));
     // D_z of d (line 419) is taken inside mag_rhs from a window of d
     if (cf) {
         m.ab3 = 1;
@@ -659,7 +684,8 @@ int inverse_b_and_j(mhd_ctx* c, MagArgs& m, bool with_b)
     return kerr(launch_jsq(m, c->s));
 }
 
-int run_bandj(mhd_ctx* c)
+// clean: pol and tor are zero in the 2/3 band (magdealias has just run)
+int run_bandj(mhd_ctx* c, bool clean)
 {
     const int wf = c->wf32;
     MagArgs m = margs(c);
@@ -667,8 +693,29 @@ int run_bandj(mhd_ctx* c)
     Z.job[0] = zjob(c->pol, 0, m.polz, wf, ZK_D1, 5);  // 519
     Z.njobs = 1;
     TRY(zrun(c, Z));
-    TRY(kerr(launch_bandj_spec(m, c->s)));
-    return inverse_b_and_j(c, m, true);
+    if (!spectral_len_fixed(c->nx)) {
+        TRY(kerr(launch_bandj_spec(m, c->s)));
+        return inverse_b_and_j(c, m, true);
+    }
+    MagSpecArgs x = mag_spec_args(c, m);
+    x.skip = clean;
+    TRY(kerr(launch_bandj_x(x, wf, c->s)));
+    // 575-593: y transforms and the mean parts of B (the mixed path keeps B
+    // without its means: no additions); dBz/dy rides with Bz
+    const bool mx = c->su != nullptr;
+    SpecLaunch M = spec_base(c, 1, SM_HC2R);
+    M.skip = clean;
+    M.job[0] = sjob(m.bzh, wf, c->bz, m.dybzh, 0, MUL_D1, wf);
+    M.job[0].adds = mx ? 0.0 : c->sc.bzbar;
+    M.job[1] = sjob(m.bxh, wf, c->bx, nullptr, 0, 0, wf);
+    M.job[1].addk = mx ? nullptr : c->bxbar;
+    M.job[2] = sjob(m.byh, wf, c->by, nullptr, 0, 0, wf);
+    M.job[2].addk = mx ? nullptr : c->bybar;
+    M.job[3] = sjob(m.dxbzh, wf, m.dxbzh, nullptr, 0, 0, wf);
+    M.job[4] = sjob(m.jzh, wf, m.jzh, nullptr, 0, 0, wf);
+    M.njobs = 5;
+    TRY(spec(c, M));
+    return kerr(launch_jsq(m, c->s));
 }
 
 int run_mag_boundary(mhd_ctx* c, int hydro, int mag)
@@ -1417,7 +1464,7 @@ int mhd_mag_deriv(mhd_ctx_t* c)
 int mhd_bandj(mhd_ctx_t* c)
 {
     TRY(check_ctx(c));
-    TRY(run_bandj(c));
+    TRY(run_bandj(c, false));
     return mhd_sync(c);
 }
 
@@ -1477,7 +1524,7 @@ int mhd_step(mhd_ctx_t* c, int nsteps, double dt_fixed, int ndu06, mhd_diag_t* l
         S.dt2 = dt + S.dt1;
         S.dt1 = dt;
         if (S.nit % 10 == 0) TRY(run_dealias5(c));
-        if (mag) TRY(run_bandj(c));
+        if (mag) TRY(run_bandj(c, true));
         TRY(run_mag_boundary(c, 1, mag ? 1 : 0));
         if (ndu06 > 0 && S.nit % ndu06 == 0) {
             double ga[4], nu, db[2];

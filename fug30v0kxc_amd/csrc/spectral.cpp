@@ -7,11 +7,17 @@
 namespace mhd {
 
 int launch_spectral_g0(int n, const SpecLaunch& L, int f32, hipStream_t s);
+int launch_spectral_g0_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
 int launch_spectral_g1(int n, const SpecLaunch& L, int f32, hipStream_t s);
+int launch_spectral_g1_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
 int launch_spectral_g2(int n, const SpecLaunch& L, int f32, hipStream_t s);
+int launch_spectral_g2_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
 int launch_spectral_g3(int n, const SpecLaunch& L, int f32, hipStream_t s);
+int launch_spectral_g3_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
 int launch_spectral_g4(int n, const SpecLaunch& L, int f32, hipStream_t s);
+int launch_spectral_g4_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
 int launch_spectral_g5(int n, const SpecLaunch& L, int f32, hipStream_t s);
+int launch_spectral_g5_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
 
 #define MHD_ALL_SIZES(X) X(8) X(12) X(16) X(20) X(24) X(30) X(32) X(40) X(48) X(60) X(64) X(80) X(96) X(120) X(128) X(160) X(192) X(240) X(256) X(320) X(384) X(480) X(512) X(640) X(768) X(1024)
 
@@ -56,6 +62,20 @@ static int launch_group(const SpecLaunch& L, int compute_f32, hipStream_t s)
     return launch_spectral_g5(n, L, compute_f32, s);
 }
 
+static int launch_mag_x(int which, const MagSpecArgs& a, int f32, hipStream_t s)
+{
+    const int n = a.g.nx;
+    if (!spectral_len_fixed(n)) return -20;
+    if (n <= 60) return launch_spectral_g0_mag(n, which, a, f32, s);
+    if (n <= 128) return launch_spectral_g1_mag(n, which, a, f32, s);
+    if (n <= 256) return launch_spectral_g2_mag(n, which, a, f32, s);
+    if (n <= 480) return launch_spectral_g3_mag(n, which, a, f32, s);
+    if (n <= 640) return launch_spectral_g4_mag(n, which, a, f32, s);
+    return launch_spectral_g5_mag(n, which, a, f32, s);
+}
+int launch_emf_x(const MagSpecArgs& a, int f32, hipStream_t s) { return launch_mag_x(0, a, f32, s); }
+int launch_bandj_x(const MagSpecArgs& a, int f32, hipStream_t s) { return launch_mag_x(1, a, f32, s); }
+
 // Three LD_CROSS jobs whose factors are the components of two vectors a, b
 // with job q = a_{q+1} b_{q+2} - a_{q+2} b_{q+1}: the EMF u x B.
 static bool is_cross_product(const SpecLaunch& L)
@@ -77,12 +97,12 @@ static bool is_cross_product(const SpecLaunch& L)
 
 // The load operation is a compile-time parameter of the kernels, so jobs are
 // launched in groups of equal load operation -- except, on the
-// register-blocked lengths, the three components of a cross product along x,
+// register-blocked lengths, the three components of a cross product along y,
 // which share their six factor loads (LD_CROSS3).
 int launch_spectral(const SpecLaunch& L, int compute_f32, hipStream_t s)
 {
     if (L.njobs <= 0) return 0;
-    if (L.mode == SM_R2HC && L.dir == 0 && spectral_len_fixed(L.g.nx) && is_cross_product(L)) {
+    if (L.mode == SM_R2HC && L.dir == 1 && spectral_len_fixed(L.g.ny) && is_cross_product(L)) {
         SpecLaunch G = L;
         G.cross3 = 1;
         return launch_group(G, compute_f32, s);

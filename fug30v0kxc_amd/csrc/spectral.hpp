@@ -56,7 +56,10 @@ struct SpecJob {
     double ascale;
     const void* xin;  // its further term xcoef * xin, or null
     double xcoef;
-    void* out[2];     // SM_DERIV2: out[1] may be null (the job's first derivative only)
+    // SM_DERIV2: out[1] may be null (the job's first derivative only).
+    // SM_HC2R: out[1], when set, takes mul[1] of the same line (d/dx or d/dy of
+    // the output, from the spectrum in registers)
+    void* out[2];
     int out_f32;
     int mul[2];       // MulKind for out[0], out[1] (SM_DERIV*)
     const double* addk; // optional per-plane value added on store (nz entries)
@@ -82,6 +85,7 @@ struct SpecLaunch {
     int variant;      // radix plan: 0 the default, 1 and 2 the length's alternatives (if any)
     int max_groups;   // optional further cap on the grid; 0 = none
     int group_major;  // set by the launcher: items ordered line group first (see spec_kernel)
+    int skip;         // SM_HC2R: the rows within icut of N/2 are zero and not read (magdealias's band)
     int cross3;       // set by the launcher: the three jobs form one cross product (LD_CROSS3)
     // set by the launcher for lengths without a register-blocked plan: the
     // run-time radices and the complex lines per workgroup
@@ -89,6 +93,25 @@ struct SpecLaunch {
     int gen_npass;
     int gen_nlb;
 };
+
+// x transforms of the magnetic part over row pairs (j, ny - j), with
+// mag_deriv's and bandj's spectral algebra (spectral_mag.hpp)
+struct MagSpecArgs {
+    Geom g;
+    const void* tw;          // W_nx^t table in the working precision
+    double cx, cy;           // 2 pi / xmax, 2 pi / ymax
+    int icutx, icuty;
+    int skip;                // bandj_x: pol and tor are zero in the 2/3 band
+    int ncu;
+    void *ex, *ey, *ez;      // emf_x: E along physical x, halfcomplex y; ez in place
+    void *cc, *d;
+    const double *pol, *tor; // bandj_x
+    const void* polz;
+    void* out[5];            // Bx, By, Jz, Bz, dBz/dx
+};
+// register-blocked lengths nx only (spectral_len_fixed), else -20
+int launch_emf_x(const MagSpecArgs& a, int f32, hipStream_t s);
+int launch_bandj_x(const MagSpecArgs& a, int f32, hipStream_t s);
 
 // Returns 0 or a negative code (-20: unsupported length).
 int launch_spectral(const SpecLaunch& L, int compute_f32, hipStream_t s);

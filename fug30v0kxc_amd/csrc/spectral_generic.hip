@@ -167,7 +167,8 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
             if (GenLines<DIR>::base(g, nlb, grp, b, ia, ib, st, k)) {
                 if constexpr (MODE == SM_HC2R) {
                     const TC* __restrict__ src = (const TC*)J.in[0];
-                    v = {src[ia + n * st], src[ib + n * st]};
+                    if (!(L.skip && n >= N / 2 - L.icut && n <= N / 2 + L.icut))
+                        v = {src[ia + n * st], src[ib + n * st]};
                 } else {
                     const Loader<TC, LOP> ld(J, k);
                     v = {ld(ia + n * st), ld(ib + n * st)};
@@ -179,14 +180,14 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
 
         TC* __restrict__ out0 = (TC*)J.out[0];
         TC* __restrict__ out1 = (TC*)J.out[1];
-        auto store = [&](const cpx<TC>* res, TC* __restrict__ out, TC scale) {
+        auto store = [&](const cpx<TC>* res, TC* __restrict__ out, TC scale, bool plus = true) {
             for (int q = threadIdx.x; q < P; q += GNT) {
                 int b, n;
                 point(q, b, n);
                 long ia, ib, st;
                 int k;
                 if (!GenLines<DIR>::base(g, nlb, grp, b, ia, ib, st, k)) continue;
-                const TC add = (J.addk ? (TC)J.addk[k] : (TC)0) + (TC)J.adds;
+                const TC add = plus ? (J.addk ? (TC)J.addk[k] : (TC)0) + (TC)J.adds : (TC)0;
                 const cpx<TC> v = res[b * N + n];
                 out[ia + n * st] = v.x * scale + add;
                 out[ib + n * st] = v.y * scale + add;
@@ -206,6 +207,15 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
                 buf1[b * N + kk] = {A.x - Bv.y, A.y + Bv.x};
             }
             __syncthreads();
+            if (out1) {
+                // the derivative output first, from a copy of the spectrum
+                for (int q = threadIdx.x; q < P; q += GNT)
+                    buf0[q] = apply_mul_rt<TC>(J.mul[1], buf1[q], q % N, N, L.cx, L.icut, J.mc);
+                __syncthreads();
+                const cpx<TC>* der = gen_fft<TC, true>(buf0, buf2, twl, L, N, nlb);
+                store(der, out1, (TC)1, false);
+                __syncthreads();
+            }
             const cpx<TC>* res = gen_fft<TC, true>(buf1, buf2, twl, L, N, nlb);
             store(res, out0, (TC)(1.0 / N));
         } else {

@@ -400,6 +400,14 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_cross3(co
 // term) loaded during the job before it, and the next item's components during
 // the jobs without an auxiliary line, which come last.  With L.split an item is
 // one job of one line group (boxes with too few line groups to fill the device).
+//
+// What bounds it: HBM through the few waves its registers allow (FP64 210: two
+// per SIMD), LDS busy 35-46 % and the VALU 23-31 % of the time.  The auxiliary
+// lines replace a launch of their own per direction (three first derivatives
+// from one load of b) and, in y, two single-output jobs: at 256^2 x 160 FP64 x
+// 241 + 104 -> 318 us, y 324 + 151 -> 449, FP32 132 + 72 -> 165 and 209 + 91 ->
+// 246; hydro_col reads 18 arrays for 26 (855 -> 723 us).  Reloading b per job
+// (three waves per SIMD) measured slower: x 336, y 460, FP32 213 and 292.
 template <typename TC, typename PL, int DIR, int B, int MODE, int LOP>
 __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_deriv2(const SpecLaunch& L, uint3 bid,
                                                                               uint3 gdim)
@@ -589,7 +597,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
             for (int r = 0; r < R0; ++r) {
                 const int n = j + r * NB0;
                 dst[r] = {(TC)0, (TC)0};
-                if (ok && j < NB0) {
+                if (ok && j < NB0 && !(L.skip && n >= N / 2 - icut && n <= N / 2 + icut)) {
                     if constexpr (DIR == 1) dst[r] = ld_pair(src, ia + n * st);
                     else dst[r] = {src[ia + n * st], src[ib + n * st]};
                 }
@@ -649,18 +657,29 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
                 }
             }
             F::sync();
-            F::inverse(v, j, lds, twl);
-            if (ok && j < NB0) {
+            cpx<TC> z[RL];
 #pragma unroll
-                for (int r = 0; r < R0; ++r) {
-                    const int n = j + r * NB0;
-                    const TC xa = v[r].x * (TC)(1.0 / N) + add, xb = v[r].y * (TC)(1.0 / N) + add;
-                    if constexpr (DIR == 1) st_pair(out0, ia + n * st, xa, xb);
-                    else {
-                        out0[ia + n * st] = xa;
-                        out0[ib + n * st] = xb;
+            for (int r = 0; r < RL; ++r) z[r] = v[r];
+            for (int o = 0;; ++o) {
+                F::inverse(v, j, lds, twl);
+                if (ok && j < NB0) {
+                    TC* __restrict__ out = (TC*)J.out[o];
+                    const TC sc = o == 0 ? (TC)(1.0 / N) : (TC)1, ad = o == 0 ? add : (TC)0;
+#pragma unroll
+                    for (int r = 0; r < R0; ++r) {
+                        const int n = j + r * NB0;
+                        const TC xa = v[r].x * sc + ad, xb = v[r].y * sc + ad;
+                        if constexpr (DIR == 1) st_pair(out, ia + n * st, xa, xb);
+                        else {
+                            out[ia + n * st] = xa;
+                            out[ib + n * st] = xb;
+                        }
                     }
                 }
+                if (o == 1 || !J.out[1]) break;
+#pragma unroll
+                for (int r = 0; r < RL; ++r)
+                    v[r] = apply_mul<TC, N>(J.mul[1], z[r], j + r * NBL, cx, icut, J.mc);
             }
         } else {
             F::forward(v, j, lds, twl);
@@ -769,7 +788,7 @@ static int launch_one(const SpecLaunch& L, hipStream_t s)
 template <typename TC, typename PL, int DIR, int B>
 static int launch_mode(const SpecLaunch& L, hipStream_t s)
 {
-    if constexpr (DIR == 0) {
+    if constexpr (DIR == 1) {
         if (L.cross3) return launch_one<TC, PL, DIR, B, SM_R2HC, LD_CROSS3>(L, s);
     }
     const int lop = L.job[0].load_op;
@@ -793,9 +812,14 @@ static int launch_plan(const SpecLaunch& L, hipStream_t s)
     // 16 pairs (8 pairs: hc2r 125 against 109, r2hc 63 against 58)
     constexpr int BH = (sizeof(TC) == 4 && B0 >= 8 && B0 * plan_tpt<PL>() >= 1024) ? B0 / 2 : B0;
     if (BH != B0 && L.mode == SM_DERIV1 && L.g.nx % (2 * BH) == 0) return launch_one<TC, PL, 1, BH, SM_DERIV1, LD_PLAIN>(L, s);
-    // second derivatives
+    // second derivatives: half groups where a full one has 512 threads (FP64) or
+    // 1024 (FP32), so that two or more workgroups share a CU (256 points: y 449
+    // against 458 us FP64, 246 against 241 FP32; 512 points FP32: 8 pairs spill)
     constexpr int B2 = B0 >= 8 && B0 * plan_tpt<PL>() >= (sizeof(TC) == 4 ? 1024 : 512) ? B0 / 2 : B0;
     if (B2 != B0 && L.mode == SM_DERIV2 && L.g.nx % (2 * B2) == 0) return launch_one<TC, PL, 1, B2, SM_DERIV2, LD_PLAIN>(L, s);
+    // the EMF's cross products: 3 lines and their 6 factors per thread
+    constexpr int BC = sizeof(TC) == 8 && B0 >= 8 ? B0 / 2 : B0;
+    if (L.cross3 && L.g.nx % (2 * BC) == 0) return launch_one<TC, PL, 1, BC, SM_R2HC, LD_CROSS3>(L, s);
     if (L.g.nx % (2 * B0) == 0) return launch_mode<TC, PL, 1, B0>(L, s);
     return launch_mode<TC, PL, 1, 1>(L, s);
 }
@@ -825,7 +849,18 @@ static int launch_n(const SpecLaunch& L, hipStream_t s)
         }                                                                      \
         return -20;                                                            \
     }                                                                          \
+    int name##_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s) \
+    {                                                                          \
+        switch (n) {                                                           \
+            SIZES(MHD_MAG_CASE)                                                \
+        }                                                                      \
+        (void)which; (void)a; (void)f32; (void)s;                              \
+        return -20;                                                            \
+    }                                                                          \
     }
+#define MHD_MAG_CASE(n_)                                                       \
+    case n_:                                                                   \
+        return f32 ? launch_mag_n<float, n_>(which, a, s) : launch_mag_n<double, n_>(which, a, s);
 #define MHD_SPEC_CASE(n_)                                                      \
     case n_:                                                                   \
         return f32 ? launch_n<float, n_>(L, s) : launch_n<double, n_>(L, s);
