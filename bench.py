@@ -472,7 +472,7 @@ def measured_traffic(precision, kernel):
 #           outputs of T, u, v, w and the first derivative of rho, working
 #           precision: 17 arrays
 #  yderiv2: the same along y, reading d/dx u and d/dx v too: 19 arrays
-#  hydro:   hydro_col with the fused AB3 update (interior and wall-row launches):
+#  hydro:   hydro_col with the fused AB3 update (interior and wall planes, one launch):
 #           reads the state (5), B and J^2 (4), the 18 x/y derivative arrays and
 #           history levels 1, 2 of 5 fields; writes 5 RHS and the 5 new state
 #           fields.  FP64: 47 x 8 = 376 B.  Mixed: FP32 state shadows, B, J^2,
@@ -482,9 +482,9 @@ KERNEL_BYTES_PER_CELL = {"xderiv2": {8: 136, 4: 68}, "yderiv2": {8: 152, 4: 76},
 KERNEL_DESC = {"xderiv2": "SpecK<T, plan, 0, 2, 1, 0> (xderiv2: d/dx and d2/dx2 of T, u, v, w with the x "
                           "derivatives of the Maxwell stresses; d/dx of rho)",
                "yderiv2": "SpecK<T, plan, 1, B, 1, 0> (yderiv2: the same along y, with d/dy of d/dx u, d/dx v)",
-               "hydro": "HydroColKernel<T, mixed, false> + <T, mixed, true> (hydro_col, interior and wall "
-                        "rows): hydro_deriv's right-hand side after the x/y passes with the fused AB3 "
-                        "update of u, v, w, rho, T"}
+               "hydro": "HydroColKernel<T, mixed, HP_ALL> (hydro_col, interior and wall planes): "
+                        "hydro_deriv's right-hand side after the x/y passes with the fused AB3 update of "
+                        "u, v, w, rho, T"}
 
 
 # algorithmic bytes per cell-step of the whole step: 139 working-precision array

@@ -58,19 +58,25 @@ __device__ __forceinline__ double dupi(const T* f, int c, double h, bool up)
     return h * (f[c + 3] - 6.0 * f[c + 2] + 18.0 * f[c + 1] - 10.0 * f[c] - 3.0 * f[c - 1]);
 }
 
-// WALL = false: interior planes [4, nz-4), zc per thread, register windows;
-// WALL = true: one boundary row per thread (planes 0..3 and nz-4..nz-1).
-template <typename TW, bool MIX, bool WALL>
+// Grid rows y < nch: interior planes [4, nz-4), zc per thread, register
+// windows; the rows after them: one boundary plane per thread (0..3 and
+// nz-4..nz-1).  The boundary planes ride in the interior's launch and fill its
+// last wave; as a launch of their own they took 14.8 us at 64^2 x 48 and 68 at
+// 256^2 x 160 FP64.  Recorded launches (PART) keep the two apart: there the
+// boundary planes of many boxes fill a launch, and the kernel over a table that
+// holds both takes 256 registers and one wave per SIMD (six mixed boxes of 64^2
+// to 128^2 columns: 223 against 178 ms).
+enum HydroPart { HP_ALL, HP_INTERIOR, HP_WALLS };
+template <typename TW, bool MIX, HydroPart PART>
 struct HydroColKernel {
     using Args = HydroColArgs;
     static constexpr int NT = HNT;
     static __device__ __forceinline__ void body(const HydroColArgs& a, uint3 bid, uint3 gdim);
 };
 
-template <typename TW, bool MIX, bool WALL>
-__device__ __forceinline__ void HydroColKernel<TW, MIX, WALL>::body(const HydroColArgs& a, uint3 bid, uint3 gdim)
+template <typename TW, bool MIX, HydroPart PART>
+__device__ __forceinline__ void HydroColKernel<TW, MIX, PART>::body(const HydroColArgs& a, uint3 bid, uint3 gdim)
 {
-    (void)bid;
     (void)gdim;
     using TS = typename std::conditional<MIX, float, double>::type;
     const int nxy = a.g.nxy, nz = a.g.nz;
@@ -281,9 +287,10 @@ __device__ __forceinline__ void HydroColKernel<TW, MIX, WALL>::body(const HydroC
         finish(k, d);
     };
 
-    if constexpr (WALL) {
+    const int nch = PART != HP_ALL || nz <= 8 ? 0 : (nz - 8 + a.zc - 1) / a.zc;
+    if (PART == HP_WALLS || (PART == HP_ALL && (int)bid.y >= nch)) {
         const int nb = nz < 8 ? nz : 8;
-        const int pr = (int)bid.y;
+        const int pr = (int)bid.y - nch;
         slow(pr < 4 ? pr : nz - (nb - pr));
         return;
     }
@@ -376,16 +383,20 @@ int launch_hydro_col(const HydroColArgs& a, int mixed, hipStream_t s)
 {
     if (a.zc <= 0) return -10;
     const unsigned bx = (unsigned)((a.g.nxy + HNT - 1) / HNT);
-    const int nin = a.g.nz - 8;                   // interior planes
-    if (nin > 0) {
-        const dim3 grid(bx, (unsigned)((nin + a.zc - 1) / a.zc));
-        const int e = mixed ? mhd_launch<HydroColKernel<float, true, false>>(grid, dim3(HNT), 0, s, a)
-                            : mhd_launch<HydroColKernel<double, false, false>>(grid, dim3(HNT), 0, s, a);
-        if (e) return e;
-    }
-    const dim3 gw(bx, (unsigned)(a.g.nz < 8 ? a.g.nz : 8));
-    return mixed ? mhd_launch<HydroColKernel<float, true, true>>(gw, dim3(HNT), 0, s, a)
-                 : mhd_launch<HydroColKernel<double, false, true>>(gw, dim3(HNT), 0, s, a);
+    const int nin = a.g.nz > 8 ? a.g.nz - 8 : 0;   // interior planes
+    const unsigned chunks = (unsigned)((nin + a.zc - 1) / a.zc), walls = (unsigned)(a.g.nz < 8 ? a.g.nz : 8);
+    auto go = [&](auto all, auto interior, auto wall) -> int {
+        if (!launch_recorder()) return mhd_launch<decltype(all)>(dim3(bx, chunks + walls), dim3(HNT), 0, s, a);
+        if (chunks) {
+            const int e = mhd_launch<decltype(interior)>(dim3(bx, chunks), dim3(HNT), 0, s, a);
+            if (e) return e;
+        }
+        return mhd_launch<decltype(wall)>(dim3(bx, walls), dim3(HNT), 0, s, a);
+    };
+    return mixed ? go(HydroColKernel<float, true, HP_ALL>{}, HydroColKernel<float, true, HP_INTERIOR>{},
+                      HydroColKernel<float, true, HP_WALLS>{})
+                 : go(HydroColKernel<double, false, HP_ALL>{}, HydroColKernel<double, false, HP_INTERIOR>{},
+                      HydroColKernel<double, false, HP_WALLS>{});
 }
 
 }  // namespace mhd

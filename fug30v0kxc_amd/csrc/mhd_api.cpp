@@ -237,6 +237,17 @@ double ran0(int* idum)
 
 int kerr(int e) { return e ? MHD_E_DEVICE : 0; }
 
+// Planes per thread of a column walk over `planes` planes with `groups`
+// workgroups of columns: `most`, or fewer where even 8 planes would leave the
+// device with less than two workgroups per compute unit.  Recorded launches run
+// together with those of other boxes, so there the walk is not cut short.
+int walk_planes(const mhd_ctx* c, long groups, int planes, int most)
+{
+    const long fit = groups * planes / (2L * c->ncu);
+    if (fit >= 8 || launch_recorder()) return most;
+    return fit < 1 ? 1 : fit < most ? (int)fit : most;
+}
+
 // f64: FP64 transform in the mixed path (launched with spec64)
 SpecLaunch spec_base(mhd_ctx* c, int dir, int mode, bool f64 = false)
 {
@@ -370,7 +381,7 @@ HydroColArgs colargs(mhd_ctx* c)
     a.udot = level_ptr(c, 0, 3);
     a.vdot = level_ptr(c, 1, 3);
     a.wdot = level_ptr(c, 2, 3);
-    a.zc = c->hzc;
+    a.zc = walk_planes(c, (c->nxy + 255) / 256, c->nz > 8 ? c->nz - 8 : 1, c->hzc);
     return a;
 }
 
@@ -398,7 +409,7 @@ MagArgs margs(mhd_ctx* c)
     if (c->su) { a.bxm = c->bxbar; a.bym = c->bybar; }
     if (c->eta_on) { a.jx = c->jx; a.jy = c->jy; a.jz = c->jz; }
     a.wf32 = c->wf32;
-    a.zc = c->mzc;
+    a.zc = walk_planes(c, (c->nxy + 511) / 512, c->nz, c->mzc);
     return a;
 }
 
@@ -632,11 +643,18 @@ int run_mag_deriv(mhd_ctx* c, const double* cf = nullptr)
             TRY(kerr(launch_mag_spec1(m, c->s)));
         }
     }
-    TRY(kerr(launch_mean_emf(m, c->s)));
-    // D_z of d (line 419) is taken inside mag_rhs from a window of d
     if (cf) {
         m.ab3 = 1;
         m.c0 = cf[0]; m.c1 = cf[1]; m.c2 = cf[2];
+        for (int f = 0; f < 2; ++f) {
+            m.mh1[f] = mlevel_ptr(c, f, 1);
+            m.mh2[f] = mlevel_ptr(c, f, 2);
+        }
+    }
+    const auto means = [&] { return kerr(launch_mean_emf(m, c->s)); };
+    TRY(cf ? timed(c, MHD_K_AB3, means) : means());   // with cf, the last of the AB3 update
+    // D_z of d (line 419) is taken inside mag_rhs from a window of d
+    if (cf) {
         m.ph1 = level_ptr(c, 5, 1); m.ph2 = level_ptr(c, 5, 2);
         m.th1 = level_ptr(c, 6, 1); m.th2 = level_ptr(c, 6, 2);
         m.polnew = c->pol2;
@@ -927,9 +945,10 @@ void ab3_coeffs(mhd_scalars_t& s, double dt, double cf[3])
     }
 }
 
-// f0 = 5: the hydro fields were updated by the fused hydro kernel; pol, tor
-// and the means here.  f0 = 7: pol and tor too (fused into mag_rhs); the means
-// here.  Then the history ring turns and the state ping-pong swaps.
+// f0 = 0: all fields and the means.  f0 = 5: the hydro fields were updated by
+// the fused hydro kernel.  f0 = 7: pol, tor and the means too (fused into
+// mag_rhs and mean_emf).  Then the history ring turns and the state ping-pong
+// swaps.
 int run_ab3(mhd_ctx* c, const double cf[3], int f0 = 0)
 {
     AB3Args a;
@@ -956,7 +975,8 @@ int run_ab3(mhd_ctx* c, const double cf[3], int f0 = 0)
     a.nfields = a.mag ? 7 : 5;
     a.icutx = c->icutx;
     a.icuty = c->icuty;
-    if (a.f0 < a.nfields || a.mag) TRY(timed(c, MHD_K_AB3, [&] { return kerr(launch_ab3(a, c->s)); }));
+    // f0 = 7: the means were updated by mean_emf
+    if (a.f0 < a.nfields) TRY(timed(c, MHD_K_AB3, [&] { return kerr(launch_ab3(a, c->s)); }));
     if (f0 >= 5) {
         std::swap(c->u, c->u2); std::swap(c->v, c->v2); std::swap(c->w, c->w2);
         std::swap(c->t, c->t2); std::swap(c->r, c->r2);
@@ -1519,7 +1539,7 @@ int mhd_step(mhd_ctx_t* c, int nsteps, double dt_fixed, int ndu06, mhd_diag_t* l
         } else {
             TRY(run_hydro_deriv(c, cf));       // hydro RHS + AB3 of u v w r t into the ping-pong
             if (mag) TRY(run_mag_deriv(c, cf)); // reads the old u v w; + AB3 of pol, tor, magdealias
-            TRY(run_ab3(c, cf, mag ? 7 : 5));  // the means (src/main.F90:508); swaps
+            TRY(run_ab3(c, cf, mag ? 7 : 5));  // swaps
         }
         S.dt2 = dt + S.dt1;
         S.dt1 = dt;

@@ -20,19 +20,21 @@ static inline unsigned nblk(long n, int nt = NT) { return (unsigned)((n + nt - 1
 // the boundary rows hold planes k0-3 .. k0+KC+2 in a register window and
 // apply the interior stencils at compile-time offsets; the chunks touching
 // the first or last three planes apply the row-specific stencils.
-constexpr int ZKC = 16;
+// KC: planes per thread, 16, or 4 where 16 would leave the device with less
+// than one workgroup per compute unit (64^2 x 48: 9.0 us with 48 workgroups).
+// Recorded launches keep 16, so that boxes differing in nz stay one class.
 
 // TC: compute/output type; TIN: input element type; KIND: ZKind; PROD: the
 // input is scale*in*in1.  w (upwind selector) has the element type TW.
-template <typename TC, typename TIN, typename TW, int KIND, bool PROD>
+template <typename TC, typename TIN, typename TW, int KIND, bool PROD, int ZKC>
 struct ZKernel {
     using Args = ZLaunch;
     static constexpr int NT = 256;
     static __device__ __forceinline__ void body(const ZLaunch& L, uint3 bid, uint3 gdim);
 };
 
-template <typename TC, typename TIN, typename TW, int KIND, bool PROD>
-__device__ __forceinline__ void ZKernel<TC, TIN, TW, KIND, PROD>::body(const ZLaunch& L, uint3 bid, uint3 gdim)
+template <typename TC, typename TIN, typename TW, int KIND, bool PROD, int ZKC>
+__device__ __forceinline__ void ZKernel<TC, TIN, TW, KIND, PROD, ZKC>::body(const ZLaunch& L, uint3 bid, uint3 gdim)
 {
     (void)bid;
     (void)gdim;
@@ -95,8 +97,13 @@ __device__ __forceinline__ void ZKernel<TC, TIN, TW, KIND, PROD>::body(const ZLa
 template <typename TC, typename TIN, typename TW, int KIND, bool PROD>
 static int launch_z_group(ZLaunch& G, hipStream_t s)
 {
-    dim3 grid(nblk(G.g.nxy), (unsigned)((G.g.nz + ZKC - 1) / ZKC), G.njobs);
-    return mhd_launch<ZKernel<TC, TIN, TW, KIND, PROD>>(grid, dim3(NT), 0, s, G);
+    const unsigned bx = nblk(G.g.nxy);
+    const long wide = (long)bx * ((G.g.nz + 15) / 16) * G.njobs;
+    if (wide >= 256 || launch_recorder())
+        return mhd_launch<ZKernel<TC, TIN, TW, KIND, PROD, 16>>(dim3(bx, (unsigned)((G.g.nz + 15) / 16), G.njobs),
+                                                                dim3(NT), 0, s, G);
+    return mhd_launch<ZKernel<TC, TIN, TW, KIND, PROD, 4>>(dim3(bx, (unsigned)((G.g.nz + 3) / 4), G.njobs), dim3(NT),
+                                                           0, s, G);
 }
 
 template <typename TC, typename TIN, typename TW>
@@ -246,7 +253,8 @@ __device__ __forceinline__ void MagSpec1Kernel<TW>::body(const MagArgs& a, uint3
         }
 }
 
-// mean-field equations, src/magnetic.f90:328-352 (one workgroup)
+// mean-field equations, src/magnetic.f90:328-352, and the means' AB3 update (one
+// workgroup, bound by its latency: as a launch of its own the update took 4.5 us)
 template <typename TW>
 struct MeanEmfKernel {
     using Args = MagArgs;
@@ -279,8 +287,14 @@ __device__ __forceinline__ void MeanEmfKernel<TW>::body(const MagArgs& a, uint3 
         const double dby = dz1<double>(k, nz, 5, h, [&](int kk) { return w1d[kk]; });
         const double d2x = dz2<double>(k, nz, 3, s, [&](int kk) { return bxb[kk]; });
         const double d2y = dz2<double>(k, nz, 3, s, [&](int kk) { return byb[kk]; });
-        a.bxbardot[k] = a.p.zck * d2x - dbx;
-        a.bybardot[k] = a.p.zck * d2y + dby;
+        const double fx = a.p.zck * d2x - dbx, fy = a.p.zck * d2y + dby;
+        a.bxbardot[k] = fx;
+        a.bybardot[k] = fy;
+        if (a.ab3) {
+            // the means' AB3 update, x + c0 f3 + c1 f2 + c2 f1
+            a.bxbar[k] = bxb[k] + a.c0 * fx + a.c1 * a.mh2[0][k] + a.c2 * a.mh1[0][k];
+            a.bybar[k] = byb[k] + a.c0 * fy + a.c1 * a.mh2[1][k] + a.c2 * a.mh1[1][k];
+        }
     }
 }
 

@@ -109,6 +109,7 @@ struct MagArgs {
     int ab3;
     double c0, c1, c2;
     const void *ph1, *ph2, *th1, *th2;   // history levels 1 and 2 of pol, tor
+    const double *mh1[2], *mh2[2];       // ... and of the means
     double *polnew, *tornew;
 };
 int launch_mag_spec1(const MagArgs& a, hipStream_t s);   // D, C from E-hat

@@ -203,9 +203,11 @@ long mhd_dump_header(const mhd_dump_t* meta, int iprec, unsigned char* buf, long
  * second derivatives, real to halfcomplex and back) the radix plan (the
  * default or one of the length's alternatives) together with the
  * persistent-grid multiple (1 or 2 x resident), on a launch of that kind
- * shaped like the step's; the planes per thread of the column-walking
- * hydro kernel, in the variant the step runs (with the fused AB3 update
- * unless a closure is attached; the magnetic column kernels keep 8 planes).
+ * shaped like the step's; the planes per thread, at most, of the
+ * column-walking hydro kernel, in the variant the step runs (with the fused
+ * AB3 update unless a closure is attached; the magnetic column kernels keep
+ * 8 planes).  Boxes too small to fill the GPU with walks of 8 planes take
+ * shorter ones whatever zc says.
  * Needs a state; overwrites only work arrays, the buffers the next step's
  * new state goes to and the newest RHS level (all rewritten by every step
  * before they are read), so it may run between steps. */
