@@ -4,15 +4,21 @@
 //
 // A workgroup holds `nlb` complex lines (two real lines each, as in
 // spectral_impl.hpp) in LDS and runs a self-sorting (Stockham) FFT whose
-// radices are the length's factors, found at run time: 4s, then 2, 3, 5, 7
-// and any remaining prime.  Each pass computes every output point directly,
-//   dst[o] = sum_r src[j + r N/R] W_N^(r (N / (Ns R)) (kk + m Ns)),
-// with o = (j / Ns) Ns R + kk + m Ns, kk = j mod Ns, m < R, from one twiddle
-// table W_N^t (LDS), ping-ponging between two LDS buffers.  This costs N R
-// multiply-adds per line and pass (R a prime factor), against the
-// register-blocked kernels' fixed radix-2/3/4/5/8 butterflies, which serve
-// the usual lengths; loads (every LoadOp), spectral multipliers, the
-// halfcomplex packing and the stores are those of spec_kernel.
+// radices are the length's factors, found at run time: 4s (and one 8 where the
+// power of two is odd), then 3, 5, 7 and any larger prime.  In a pass with radix
+// R up to 13 a thread owns one butterfly: it reads its R points, multiplies them
+// by the twiddles of one LDS table W_N^t and writes the R outputs
+//   dst[(j / Ns) Ns R + (j mod Ns) + m Ns], m < R,
+// ping-ponging between two LDS buffers.  Larger primes compute every output
+// point directly, N R multiply-adds per line and pass.  Loads (every LoadOp),
+// spectral multipliers, the halfcomplex packing and the stores are those of
+// spec_kernel.
+//
+// What bounds it: the latency of the passes (a barrier each) at the three
+// workgroups per CU that three LDS buffers leave.  The transforms of a step on
+// lengths 100 (4 5 5) and 144 (4 4 3 3), 61 planes FP64: 507 us with one output
+// point per thread (R reads and twiddles each, a 64-bit division per point for
+// its line), 445 with a butterfly per thread.
 #include "spectral_impl.hpp"
 
 namespace mhd {
@@ -20,6 +26,7 @@ namespace mhd {
 namespace {
 
 constexpr int GNT = 256;
+constexpr int GEN_MAX_LINES = 64;
 
 template <typename TC>
 __device__ __forceinline__ cpx<TC> apply_mul_rt(int kind, cpx<TC> z, int k, int N, double cx, int icut,
@@ -43,7 +50,79 @@ __device__ __forceinline__ cpx<TC> apply_mul_rt(int kind, cpx<TC> z, int k, int 
     }
 }
 
-// one pass over the workgroup's nlb lines, src -> dst
+// q / d for 0 <= q < 2^16, inv = 1.0f / d
+__device__ __forceinline__ int fdiv(int q, float inv) { return (int)(((float)q + 0.5f) * inv); }
+
+// R-point DFT in registers; odd primes from 7 on take their roots of unity
+// W_R^t = tw[t N / R] from the table (uniform reads)
+template <typename TC, int R, bool INV>
+__device__ __forceinline__ void gen_dft(cpx<TC>* v, const cpx<TC>* __restrict__ tw, int NR)
+{
+    if constexpr (R <= 5 || R == 8) {
+        (void)tw;
+        (void)NR;
+        dft_r<TC, R, INV>(v);
+    } else {
+        constexpr int H = (R - 1) / 2;
+        cpx<TC> s[H], d[H], o[R];
+#pragma unroll
+        for (int r = 0; r < H; ++r) {
+            s[r] = cadd(v[r + 1], v[R - 1 - r]);
+            d[r] = csub(v[r + 1], v[R - 1 - r]);
+        }
+        o[0] = v[0];
+#pragma unroll
+        for (int r = 0; r < H; ++r) o[0] = cadd(o[0], s[r]);
+#pragma unroll
+        for (int m = 1; m <= H; ++m) {
+            cpx<TC> a = v[0], b = {(TC)0, (TC)0};
+#pragma unroll
+            for (int r = 1; r <= H; ++r) {
+                const cpx<TC> w = tw[(r * m % R) * NR];   // cos, -sin
+                a.x += w.x * s[r - 1].x;
+                a.y += w.x * s[r - 1].y;
+                b.x -= w.y * d[r - 1].x;
+                b.y -= w.y * d[r - 1].y;
+            }
+            // a -+ i b
+            const cpx<TC> ib = cmul_i<TC, INV ? 1 : -1>(b);
+            o[m] = cadd(a, ib);
+            o[R - m] = csub(a, ib);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = o[r];
+    }
+}
+
+// one pass over the workgroup's nlb lines, src -> dst, one butterfly per thread
+template <typename TC, int R, bool INV>
+__device__ __forceinline__ void gen_pass_r(const cpx<TC>* __restrict__ src, cpx<TC>* __restrict__ dst,
+                                           const cpx<TC>* __restrict__ tw, int N, int nlb, int Ns)
+{
+    const int NB = N / R, ts = NB / Ns;   // twiddle of butterfly kk, point r: W_N^(r kk ts)
+    const float iNB = 1.0f / (float)NB, iNs = 1.0f / (float)Ns;
+    for (int q = threadIdx.x; q < nlb * NB; q += GNT) {
+        const int b = fdiv(q, iNB), j = q - b * NB;
+        const int blk = fdiv(j, iNs), kk = j - blk * Ns;
+        const cpx<TC>* s = src + b * N + j;
+        cpx<TC> v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = s[r * NB];
+        const int e = kk * ts;
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+            const cpx<TC> w = tw[r * e];   // r kk ts < N
+            v[r] = INV ? cmulc(v[r], w) : cmul(v[r], w);
+        }
+        gen_dft<TC, R, INV>(v, tw, NB);
+        cpx<TC>* d = dst + b * N + blk * Ns * R + kk;
+#pragma unroll
+        for (int r = 0; r < R; ++r) d[r * Ns] = v[r];
+    }
+    __syncthreads();
+}
+
+// any radix, one output point per thread
 template <typename TC, bool INV>
 __device__ __forceinline__ void gen_pass(const cpx<TC>* __restrict__ src, cpx<TC>* __restrict__ dst,
                                          const cpx<TC>* __restrict__ tw, int N, int nlb, int Ns, int R)
@@ -80,7 +159,17 @@ __device__ __forceinline__ cpx<TC>* gen_fft(cpx<TC>* a, cpx<TC>* b, const cpx<TC
     int Ns = 1;
     for (int p = 0; p < L.gen_npass; ++p) {
         const int R = L.gen_radix[p];
-        gen_pass<TC, INV>(a, b, tw, N, nlb, Ns, R);
+        switch (R) {
+        case 2: gen_pass_r<TC, 2, INV>(a, b, tw, N, nlb, Ns); break;
+        case 3: gen_pass_r<TC, 3, INV>(a, b, tw, N, nlb, Ns); break;
+        case 4: gen_pass_r<TC, 4, INV>(a, b, tw, N, nlb, Ns); break;
+        case 5: gen_pass_r<TC, 5, INV>(a, b, tw, N, nlb, Ns); break;
+        case 7: gen_pass_r<TC, 7, INV>(a, b, tw, N, nlb, Ns); break;
+        case 8: gen_pass_r<TC, 8, INV>(a, b, tw, N, nlb, Ns); break;
+        case 11: gen_pass_r<TC, 11, INV>(a, b, tw, N, nlb, Ns); break;
+        case 13: gen_pass_r<TC, 13, INV>(a, b, tw, N, nlb, Ns); break;
+        default: gen_pass<TC, INV>(a, b, tw, N, nlb, Ns, R);
+        }
         cpx<TC>* t = a;
         a = b;
         b = t;
@@ -135,15 +224,21 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
     const int N = DIR == 0 ? g.nx : g.ny;
     const int nlb = L.gen_nlb;
     extern __shared__ __align__(16) unsigned char smem[];
-    cpx<TC>* twl = reinterpret_cast<cpx<TC>*>(smem);
+    // the lines of the item: elements 0 of lines a and b (a < 0: past the end), plane
+    long* line_a = reinterpret_cast<long*>(smem);
+    long* line_b = line_a + GEN_MAX_LINES;
+    int* line_k = reinterpret_cast<int*>(line_b + GEN_MAX_LINES);
+    cpx<TC>* twl = reinterpret_cast<cpx<TC>*>(line_k + GEN_MAX_LINES);
     cpx<TC>* buf0 = twl + N;
     cpx<TC>* buf1 = buf0 + nlb * N;
-    cpx<TC>* buf2 = buf1 + nlb * N;   // the kept spectrum of two-output passes
+    cpx<TC>* buf2 = buf1 + nlb * N;   // two-output jobs only (gen_lds_bytes)
     const cpx<TC>* __restrict__ twg = reinterpret_cast<const cpx<TC>*>(L.tw);
     for (int i = threadIdx.x; i < N; i += GNT) twl[i] = twg[i];
     const long ngrp = GenLines<DIR>::groups(g, nlb);
     const long nitems = ngrp * L.njobs;
     const int P = nlb * N;
+    const float iN = 1.0f / (float)N, iL = 1.0f / (float)nlb;
+    const long st = DIR == 0 ? 1 : g.nx;
     __syncthreads();
 
     for (long item = bid.x; item < nitems; item += gdim.x) {
@@ -154,17 +249,26 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
         // columns: the line fastest, so a row of adjacent column pairs is one
         // contiguous load)
         auto point = [&](int q, int& b, int& n) {
-            if constexpr (DIR == 0) { b = q / N; n = q - b * N; }
-            else { n = q / nlb; b = q - n * nlb; }
+            if constexpr (DIR == 0) { b = fdiv(q, iN); n = q - b * N; }
+            else { n = fdiv(q, iL); b = q - n * nlb; }
         };
+        if ((int)threadIdx.x < nlb) {
+            long ia, ib, s1;
+            int k;
+            const bool ok = GenLines<DIR>::base(g, nlb, grp, threadIdx.x, ia, ib, s1, k);
+            line_a[threadIdx.x] = ok ? ia : -1;
+            line_b[threadIdx.x] = ib;
+            line_k[threadIdx.x] = k;
+        }
+        __syncthreads();
         // load
         for (int q = threadIdx.x; q < P; q += GNT) {
             int b, n;
             point(q, b, n);
-            long ia, ib, st;
-            int k;
+            const long ia = line_a[b], ib = line_b[b];
+            const int k = line_k[b];
             cpx<TC> v = {(TC)0, (TC)0};
-            if (GenLines<DIR>::base(g, nlb, grp, b, ia, ib, st, k)) {
+            if (ia >= 0) {
                 if constexpr (MODE == SM_HC2R) {
                     const TC* __restrict__ src = (const TC*)J.in[0];
                     if (!(L.skip && n >= N / 2 - L.icut && n <= N / 2 + L.icut))
@@ -184,9 +288,9 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
             for (int q = threadIdx.x; q < P; q += GNT) {
                 int b, n;
                 point(q, b, n);
-                long ia, ib, st;
-                int k;
-                if (!GenLines<DIR>::base(g, nlb, grp, b, ia, ib, st, k)) continue;
+                const long ia = line_a[b], ib = line_b[b];
+                if (ia < 0) continue;
+                const int k = line_k[b];
                 const TC add = plus ? (J.addk ? (TC)J.addk[k] : (TC)0) + (TC)J.adds : (TC)0;
                 const cpx<TC> v = res[b * N + n];
                 out[ia + n * st] = v.x * scale + add;
@@ -197,7 +301,7 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
         if constexpr (MODE == SM_HC2R) {
             // two halfcomplex lines -> the spectrum of z = a + i b
             for (int q = threadIdx.x; q < P; q += GNT) {
-                const int b = q / N, kk = q - b * N;
+                const int b = fdiv(q, iN), kk = q - b * N;
                 const cpx<TC> u = buf0[b * N + kk];
                 const cpx<TC> m = buf0[b * N + (N - kk) % N];
                 cpx<TC> A, Bv;
@@ -210,13 +314,13 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
             if (out1) {
                 // the derivative output first, from a copy of the spectrum
                 for (int q = threadIdx.x; q < P; q += GNT)
-                    buf0[q] = apply_mul_rt<TC>(J.mul[1], buf1[q], q % N, N, L.cx, L.icut, J.mc);
+                    buf0[q] = apply_mul_rt<TC>(J.mul[1], buf1[q], q - fdiv(q, iN) * N, N, L.cx, L.icut, J.mc);
                 __syncthreads();
                 const cpx<TC>* der = gen_fft<TC, true>(buf0, buf2, twl, L, N, nlb);
                 store(der, out1, (TC)1, false);
                 __syncthreads();
             }
-            const cpx<TC>* res = gen_fft<TC, true>(buf1, buf2, twl, L, N, nlb);
+            const cpx<TC>* res = gen_fft<TC, true>(buf1, buf0, twl, L, N, nlb);
             store(res, out0, (TC)(1.0 / N));
         } else {
             cpx<TC>* spec = gen_fft<TC, false>(buf0, buf1, twl, L, N, nlb);
@@ -225,9 +329,8 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
                 for (int q = threadIdx.x; q < P; q += GNT) {
                     int b, n;
                     point(q, b, n);
-                    long ia, ib, st;
-                    int k;
-                    if (!GenLines<DIR>::base(g, nlb, grp, b, ia, ib, st, k)) continue;
+                    const long ia = line_a[b], ib = line_b[b];
+                    if (ia < 0) continue;
                     const int kk = (2 * n <= N) ? n : N - n;
                     const cpx<TC> zk = spec[b * N + kk];
                     const cpx<TC> zn = spec[b * N + (N - kk) % N];
@@ -242,16 +345,17 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
                 for (int o = 0; o < NOUT; ++o) {
                     if (o == 1 && out1 == nullptr) break;   // a first-derivative job (uniform)
                     cpx<TC>* aux = nullptr;
-                    cpx<TC>* work = buf2;
+                    // a job with one output needs no third buffer
+                    cpx<TC>* work = out1 ? buf2 : spec;
                     if (o == 1 && J.aux) {
                         // the auxiliary line's spectrum
                         for (int q = threadIdx.x; q < P; q += GNT) {
                             int b, n;
                             point(q, b, n);
-                            long ia, ib, st;
-                            int k;
+                            const long ia = line_a[b], ib = line_b[b];
+                            const int k = line_k[b];
                             cpx<TC> v = {(TC)0, (TC)0};
-                            if (GenLines<DIR>::base(g, nlb, grp, b, ia, ib, st, k)) {
+                            if (ia >= 0) {
                                 const AuxLoad<TC> al(L, J, k);
                                 const TC* __restrict__ p0 = (const TC*)L.bf[al.ai];
                                 const TC* __restrict__ p1 = (const TC*)L.bf[al.aj];
@@ -271,7 +375,7 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
                     // multiplied spectrum into `dst`, inverse through `work`
                     cpx<TC>* dst = aux ? aux : other;
                     for (int q = threadIdx.x; q < P; q += GNT) {
-                        const int kk = q % N;
+                        const int kk = q - fdiv(q, iN) * N;
                         cpx<TC> m = apply_mul_rt<TC>(J.mul[o], spec[q], kk, N, L.cx, L.icut, J.mc);
                         if (aux) m = cadd(m, apply_mul_rt<TC>(MUL_D1, aux[q], kk, N, L.cx, L.icut, J.mc));
                         dst[q] = m;
@@ -287,12 +391,23 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
     }
 }
 
-size_t gen_lds_bytes(int N, int nlb, size_t csz) { return (size_t)(N + 3 * nlb * N) * csz; }
+// the table of lines, twiddles, the two buffers of the passes and, where a
+// spectrum outlives them (two outputs), a third
+size_t gen_lds_bytes(int N, int nlb, size_t csz, bool keep)
+{
+    return GEN_MAX_LINES * (2 * sizeof(long) + sizeof(int)) + (size_t)(N + (keep ? 3 : 2) * nlb * N) * csz;
+}
+bool gen_keeps(const SpecLaunch& L)
+{
+    for (int q = 0; q < L.njobs; ++q)
+        if (L.job[q].out[1]) return true;
+    return false;
+}
 
 template <typename TC, int DIR, int MODE, int LOP>
 int gen_launch(const SpecLaunch& L, hipStream_t s)
 {
-    const size_t lds = gen_lds_bytes(L.dir == 0 ? L.g.nx : L.g.ny, L.gen_nlb, sizeof(cpx<TC>));
+    const size_t lds = gen_lds_bytes(L.dir == 0 ? L.g.nx : L.g.ny, L.gen_nlb, sizeof(cpx<TC>), gen_keeps(L));
     using K = GenK<TC, DIR, MODE, LOP>;
     auto kern = single_kernel<K>;
     // more than 64 KB of dynamic LDS is opted into once per kernel
@@ -329,6 +444,10 @@ bool generic_plan(int n, int radix[SPEC_GEN_MAX_PASSES], int* npass)
 {
     if (n < 2 || n % 2 || n > SPEC_GEN_MAX_N) return false;
     int p = 0, m = n;
+    // one 8 where the power of two is odd and at least 8, then 4s
+    int e2 = 0;
+    while (m % (2 << e2) == 0) ++e2;
+    if (e2 >= 3 && e2 % 2) { radix[p++] = 8; m /= 8; }
     while (m % 4 == 0 && p < SPEC_GEN_MAX_PASSES) { radix[p++] = 4; m /= 4; }
     for (int f = 2; m > 1 && p < SPEC_GEN_MAX_PASSES; ++f)
         while (m % f == 0 && p < SPEC_GEN_MAX_PASSES) { radix[p++] = f; m /= f; }
@@ -344,10 +463,11 @@ int launch_spectral_generic(const SpecLaunch& L0, int f32, hipStream_t s)
     // lines per workgroup: about 1024 points, at most 64 KB of LDS where one
     // line fits in that
     const size_t csz = f32 ? sizeof(cpx<float>) : sizeof(cpx<double>);
+    const bool keep = gen_keeps(L);
     int nlb = 1024 / N;
     if (nlb < 1) nlb = 1;
-    if (nlb > 64) nlb = 64;
-    while (nlb > 1 && gen_lds_bytes(N, nlb, csz) > 65536) --nlb;
+    if (nlb > GEN_MAX_LINES) nlb = GEN_MAX_LINES;
+    while (nlb > 1 && gen_lds_bytes(N, nlb, csz, keep) > 65536) --nlb;
     L.gen_nlb = nlb;
     if (f32) return L.dir == 0 ? gen_mode<float, 0>(L, s) : gen_mode<float, 1>(L, s);
     return L.dir == 0 ? gen_mode<double, 0>(L, s) : gen_mode<double, 1>(L, s);
