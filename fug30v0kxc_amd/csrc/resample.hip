@@ -2,14 +2,14 @@
 // interpolate/fft.F90:832-927) and the block box filter of coarse-grained
 // data, on gfx950.
 //
-// expand doubles nx and ny by zero-padding the spectrum of every plane.  It
-// is composed from the horizontal transform kernels: x r2hc (length nx), a
-// padding kernel into rows of 2nx, x hc2r (length 2nx), y r2hc (length ny,
-// stride 2nx), a padding kernel into columns of 2ny, y hc2r (length 2ny).
-// The padding follows the reference: r_0, the (r_m, i_m) of m = 1..n/2-1
-// and the coarse Nyquist r_{n/2} as an ordinary cosine coefficient of mode
-// n/2; each inverse divides by the coarse length (the padding kernels apply
-// a factor 2 against the transform's 1/(2n)).
+// expand doubles nx and ny by zero-padding the spectrum of every plane, x then
+// y, each direction in one pass (spectral_expand.hpp).  A length without a
+// register-blocked plan takes three: the real to halfcomplex transform, a
+// padding kernel into lines of twice the length, and the inverse transform of
+// that length.  The padding follows the reference: r_0, the (r_m, i_m) of
+// m = 1..n/2-1 and the coarse Nyquist r_{n/2} as an ordinary cosine coefficient
+// of mode n/2; each inverse divides by the coarse length (the padding kernels
+// apply a factor 2 against the transform's 1/(2n)).
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -78,16 +78,20 @@ __global__ void __launch_bounds__(RNT) box_kernel(const double* __restrict__ in,
 
 unsigned nb(long n) { return (unsigned)((n + RNT - 1) / RNT); }
 
-// W_n^t = exp(-2 pi i t / n) for t < n, as (cos, sin) pairs, computed on the
-// device so that no host staging is needed
-__global__ void __launch_bounds__(RNT) twiddle_kernel(double* __restrict__ tw, int n)
+// W_n^t = exp(-2 pi i t / n), t < n, as (cos, sin) pairs for up to four lengths
+// (blockIdx.y), computed on the device so that no host staging is needed
+struct TwiddleArgs {
+    double* tw[4];
+    int n[4];
+};
+__global__ void __launch_bounds__(RNT) twiddle_kernel(TwiddleArgs a)
 {
-    const int t = blockIdx.x * RNT + threadIdx.x;
+    const int t = blockIdx.x * RNT + threadIdx.x, n = a.n[blockIdx.y];
     if (t >= n) return;
     double s, c;
     sincospi(-2.0 * (double)t / (double)n, &s, &c);
-    tw[2 * t] = c;
-    tw[2 * t + 1] = s;
+    a.tw[blockIdx.y][2 * t] = c;
+    a.tw[blockIdx.y][2 * t + 1] = s;
 }
 
 int ncus()
@@ -140,9 +144,9 @@ int expand_check(int nx, int ny, int nz, const void* in, const void* out)
 }
 
 // expand of device arrays: in (nx, ny, nz) -> out (2nx, 2ny, nz), with
-// `work` holding expand_work_doubles() doubles; `in` is only read.  The x
-// forward pass writes the first quarter of `out`, which the y padding later
-// overwrites.
+// `work` holding expand_work_doubles() doubles; `in` is only read.  (A length
+// without a one-pass kernel: the x forward pass writes the first quarter of
+// `out`, which the y padding later overwrites.)
 int expand_device(int nx, int ny, int nz, const double* in, double* out, double* work, hipStream_t s)
 {
     const long n3 = (long)nx * ny * nz;
@@ -151,18 +155,36 @@ int expand_device(int nx, int ny, int nz, const double* in, double* out, double*
     double* twx2 = twx + 2 * nx;
     double* twy = twx2 + 4 * nx;
     double* twy2 = twy + 2 * ny;
-    const int lens[4] = {nx, 2 * nx, ny, 2 * ny};
-    double* tws[4] = {twx, twx2, twy, twy2};
-    for (int q = 0; q < 4; ++q)
-        hipLaunchKernelGGL(twiddle_kernel, dim3(nb(lens[q])), dim3(RNT), 0, s, tws[q], lens[q]);
+    const bool fx = spectral_len_fixed(nx), fy = spectral_len_fixed(ny);
+    const TwiddleArgs tw = {{twx, twy, twx2, twy2}, {nx, ny, 2 * nx, 2 * ny}};
+    const int longest = 2 * (nx > ny ? nx : ny);
+    hipLaunchKernelGGL(twiddle_kernel, dim3(nb(fx && fy ? longest / 2 : longest), fx && fy ? 2 : 4), dim3(RNT), 0, s,
+                       tw);
     if (hipGetLastError() != hipSuccess) return MHD_E_DEVICE;
-    int e = hc_pass(in, out, nx, ny, nz, 0, SM_R2HC, twx, s);                 // x forward, length nx
-    if (e) return e;
-    hipLaunchKernelGGL(pad_x_kernel, dim3(nb(2 * n3)), dim3(RNT), 0, s, out, b, nx, (long)ny * nz);
-    if ((e = hc_pass(b, b, 2 * nx, ny, nz, 0, SM_HC2R, twx2, s))) return e;   // x inverse, 2nx
-    if ((e = hc_pass(b, b, 2 * nx, ny, nz, 1, SM_R2HC, twy, s))) return e;    // y forward, ny
-    hipLaunchKernelGGL(pad_y_kernel, dim3(nb(4 * n3)), dim3(RNT), 0, s, b, out, 2 * nx, ny, nz);
-    if ((e = hc_pass(out, out, 2 * nx, 2 * ny, nz, 1, SM_HC2R, twy2, s))) return e;   // y inverse, 2ny
+    ExpandArgs a;
+    memset(&a, 0, sizeof(a));
+    a.ncu = ncus();
+    a.g.nz = nz;
+    a.g.ny = ny;
+    int e;
+    if (fx) {
+        a.g.nx = nx; a.g.nxy = nx * ny; a.g.n3 = n3;
+        a.dir = 0; a.tw = twx; a.in = in; a.out = b;
+        if (launch_expand(a, s)) return MHD_E_DEVICE;
+    } else {
+        if ((e = hc_pass(in, out, nx, ny, nz, 0, SM_R2HC, twx, s))) return e;     // x forward, length nx
+        hipLaunchKernelGGL(pad_x_kernel, dim3(nb(2 * n3)), dim3(RNT), 0, s, out, b, nx, (long)ny * nz);
+        if ((e = hc_pass(b, b, 2 * nx, ny, nz, 0, SM_HC2R, twx2, s))) return e;   // x inverse, 2nx
+    }
+    if (fy) {
+        a.g.nx = 2 * nx; a.g.nxy = 2 * nx * ny; a.g.n3 = 2 * n3;
+        a.dir = 1; a.tw = twy; a.in = b; a.out = out;
+        if (launch_expand(a, s)) return MHD_E_DEVICE;
+    } else {
+        if ((e = hc_pass(b, b, 2 * nx, ny, nz, 1, SM_R2HC, twy, s))) return e;    // y forward, ny
+        hipLaunchKernelGGL(pad_y_kernel, dim3(nb(4 * n3)), dim3(RNT), 0, s, b, out, 2 * nx, ny, nz);
+        if ((e = hc_pass(out, out, 2 * nx, 2 * ny, nz, 1, SM_HC2R, twy2, s))) return e;   // y inverse, 2ny
+    }
     return hipGetLastError() == hipSuccess ? 0 : MHD_E_DEVICE;
 }
 

@@ -8,16 +8,22 @@ namespace mhd {
 
 int launch_spectral_g0(int n, const SpecLaunch& L, int f32, hipStream_t s);
 int launch_spectral_g0_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
+int launch_spectral_g0_expand(int n, const ExpandArgs& a, hipStream_t s);
 int launch_spectral_g1(int n, const SpecLaunch& L, int f32, hipStream_t s);
 int launch_spectral_g1_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
+int launch_spectral_g1_expand(int n, const ExpandArgs& a, hipStream_t s);
 int launch_spectral_g2(int n, const SpecLaunch& L, int f32, hipStream_t s);
 int launch_spectral_g2_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
+int launch_spectral_g2_expand(int n, const ExpandArgs& a, hipStream_t s);
 int launch_spectral_g3(int n, const SpecLaunch& L, int f32, hipStream_t s);
 int launch_spectral_g3_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
+int launch_spectral_g3_expand(int n, const ExpandArgs& a, hipStream_t s);
 int launch_spectral_g4(int n, const SpecLaunch& L, int f32, hipStream_t s);
 int launch_spectral_g4_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
+int launch_spectral_g4_expand(int n, const ExpandArgs& a, hipStream_t s);
 int launch_spectral_g5(int n, const SpecLaunch& L, int f32, hipStream_t s);
 int launch_spectral_g5_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
+int launch_spectral_g5_expand(int n, const ExpandArgs& a, hipStream_t s);
 
 #define MHD_ALL_SIZES(X) X(8) X(12) X(16) X(20) X(24) X(30) X(32) X(40) X(48) X(60) X(64) X(80) X(96) X(120) X(128) X(160) X(192) X(240) X(256) X(320) X(384) X(480) X(512) X(640) X(768) X(1024)
 
@@ -75,6 +81,18 @@ static int launch_mag_x(int which, const MagSpecArgs& a, int f32, hipStream_t s)
 }
 int launch_emf_x(const MagSpecArgs& a, int f32, hipStream_t s) { return launch_mag_x(0, a, f32, s); }
 int launch_bandj_x(const MagSpecArgs& a, int f32, hipStream_t s) { return launch_mag_x(1, a, f32, s); }
+
+int launch_expand(const ExpandArgs& a, hipStream_t s)
+{
+    const int n = a.dir == 0 ? a.g.nx : a.g.ny;
+    if (!spectral_len_fixed(n)) return -20;
+    if (n <= 60) return launch_spectral_g0_expand(n, a, s);
+    if (n <= 128) return launch_spectral_g1_expand(n, a, s);
+    if (n <= 256) return launch_spectral_g2_expand(n, a, s);
+    if (n <= 480) return launch_spectral_g3_expand(n, a, s);
+    if (n <= 640) return launch_spectral_g4_expand(n, a, s);
+    return launch_spectral_g5_expand(n, a, s);
+}
 
 // Three LD_CROSS jobs whose factors are the components of two vectors a, b
 // with job q = a_{q+1} b_{q+2} - a_{q+2} b_{q+1}: the EMF u x B.

@@ -113,6 +113,17 @@ struct MagSpecArgs {
 int launch_emf_x(const MagSpecArgs& a, int f32, hipStream_t s);
 int launch_bandj_x(const MagSpecArgs& a, int f32, hipStream_t s);
 
+// one direction of expand on an FP64 box g: out has 2 g.nx columns (dir 0) or
+// 2 g.ny rows (dir 1); spectral_len_fixed lengths only (spectral_expand.hpp)
+struct ExpandArgs {
+    Geom g;
+    int dir, ncu;
+    const void* tw;          // W_n^t table of the doubled direction's length n
+    const double* in;
+    double* out;
+};
+int launch_expand(const ExpandArgs& a, hipStream_t s);
+
 // Returns 0 or a negative code (-20: unsupported length).
 int launch_spectral(const SpecLaunch& L, int compute_f32, hipStream_t s);
 

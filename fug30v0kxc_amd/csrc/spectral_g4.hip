@@ -1,5 +1,6 @@
 // spectral_g4.hip -- transform kernels instantiated for one group of
 // lengths (split so the kernels compile in parallel).
+#include "spectral_expand.hpp"
 #include "spectral_mag.hpp"
 
 #define SIZES_G4(X) X(512) X(640)

@@ -857,7 +857,18 @@ static int launch_n(const SpecLaunch& L, hipStream_t s)
         (void)which; (void)a; (void)f32; (void)s;                              \
         return -20;                                                            \
     }                                                                          \
+    int name##_expand(int n, const ExpandArgs& a, hipStream_t s)               \
+    {                                                                          \
+        switch (n) {                                                           \
+            SIZES(MHD_EXPAND_CASE)                                             \
+        }                                                                      \
+        (void)a; (void)s;                                                      \
+        return -20;                                                            \
+    }                                                                          \
     }
+#define MHD_EXPAND_CASE(n_)                                                    \
+    case n_:                                                                   \
+        return launch_expand_n<n_>(a, s);
 #define MHD_MAG_CASE(n_)                                                       \
     case n_:                                                                   \
         return f32 ? launch_mag_n<float, n_>(which, a, s) : launch_mag_n<double, n_>(which, a, s);
