@@ -13,6 +13,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -21,6 +22,7 @@
 #include <vector>
 
 #include "closure.hpp"
+#include "host_copy.hpp"
 #include "launch.hpp"
 #include "physics.hpp"
 #include "spectral.hpp"
@@ -104,6 +106,8 @@ struct mhd_ctx {
     int hzc;           // planes per thread of the column-walking hydro kernel
     int mzc;           // ... of the magnetic column kernels (mag_rhs, jsq)
     double* hbuf;      // pinned host staging (one field)
+    hipEvent_t xev[XFER_CHUNKS];   // its transfers' chunks
+    int xev_created;
 
     mhd_scalars_t sc;
     int have_state;
@@ -1216,6 +1220,12 @@ int mhd_create(const mhd_params_t* p, int nx, int ny, int nz, int precision, mhd
         mhd_destroy(c);
         return MHD_E_DEVICE;
     }
+    for (int i = 0; i < XFER_CHUNKS; ++i)
+        if (hipEventCreateWithFlags(&c->xev[i], hipEventDisableTiming) != hipSuccess) {
+            mhd_destroy(c);
+            return MHD_E_DEVICE;
+        } else
+            c->xev_created = i + 1;
     for (int i = 0; i < 2 * MAXEV; ++i)
         if (hipEventCreate(&c->ev[i]) != hipSuccess) {
             mhd_destroy(c);
@@ -1231,6 +1241,7 @@ void mhd_destroy(mhd_ctx_t* c)
     if (!c) return;
     if (c->s) (void)hipStreamSynchronize(c->s);
     for (int i = 0; i < c->ev_created; ++i) (void)hipEventDestroy(c->ev[i]);
+    for (int i = 0; i < c->xev_created; ++i) (void)hipEventDestroy(c->xev[i]);
     if (c->hbuf) (void)hipHostFree(c->hbuf);
     if (c->pool) (void)hipFree(c->pool);
     if (c->cl_mem) (void)hipFree(c->cl_mem);
@@ -1241,11 +1252,10 @@ void mhd_destroy(mhd_ctx_t* c)
 static int upload(mhd_ctx* c, void* dst, int dst_f32, const double* src, long n)
 {
     if (!src) return 0;
-    memcpy(c->hbuf, src, n * sizeof(double));
     if (!dst_f32) {
-        MHD_HIP_CHECK(hipMemcpyAsync(dst, c->hbuf, n * sizeof(double), hipMemcpyHostToDevice, c->s));
+        MHD_HIP_CHECK(send_doubles((double*)dst, src, n, c->hbuf, c->s));
     } else {
-        MHD_HIP_CHECK(hipMemcpyAsync(c->stage, c->hbuf, n * sizeof(double), hipMemcpyHostToDevice, c->s));
+        MHD_HIP_CHECK(send_doubles(c->stage, src, n, c->hbuf, c->s));
         TRY(kerr(launch_copy_cvt(c->stage, 0, dst, 1, n, c->s)));
     }
     MHD_HIP_CHECK(hipStreamSynchronize(c->s));
@@ -1260,23 +1270,7 @@ static int download(mhd_ctx* c, double* dst, const void* src, int src_f32, long 
         TRY(kerr(launch_copy_cvt(src, 1, c->stage, 0, n, c->s)));
         from = c->stage;
     }
-    MHD_HIP_CHECK(hipMemcpyAsync(c->hbuf, from, n * sizeof(double), hipMemcpyDeviceToHost, c->s));
-    MHD_HIP_CHECK(hipStreamSynchronize(c->s));
-    memcpy(dst, c->hbuf, n * sizeof(double));
-    return 0;
-}
-
-// mixed precision: the per-plane mean of B component comp (0 bx, 1 by, 2 bz)
-static int b_means(mhd_ctx* c, int comp, std::vector<double>& m)
-{
-    m.assign(c->nz, 0.0);
-    if (comp == 2) {
-        for (int k = 0; k < c->nz; ++k) m[k] = c->sc.bzbar;
-        return 0;
-    }
-    MHD_HIP_CHECK(hipMemcpyAsync(m.data(), comp == 0 ? c->bxbar : c->bybar, c->nz * sizeof(double),
-                                 hipMemcpyDeviceToHost, c->s));
-    MHD_HIP_CHECK(hipStreamSynchronize(c->s));
+    MHD_HIP_CHECK(fetch_doubles(dst, (const double*)from, n, c->hbuf, c->xev, c->s));
     return 0;
 }
 
@@ -1285,13 +1279,10 @@ static int download_b(mhd_ctx* c, double* dst, int comp)
 {
     if (!dst) return 0;
     const void* src = comp == 0 ? c->bx : (comp == 1 ? c->by : c->bz);
-    TRY(download(c, dst, src, c->wf32, c->n3));
-    if (!c->su) return 0;
-    std::vector<double> m;
-    TRY(b_means(c, comp, m));
-    for (int k = 0; k < c->nz; ++k)
-        for (long q = 0; q < c->nxy; ++q) dst[(long)k * c->nxy + q] += m[k];
-    return 0;
+    if (!c->su) return download(c, dst, src, c->wf32, c->n3);
+    TRY(kerr(launch_add_mean((const float*)src, c->stage, comp == 0 ? c->bxbar : comp == 1 ? c->bybar : nullptr,
+                             comp == 2 ? c->sc.bzbar : 0.0, c->g, c->s)));
+    return download(c, dst, c->stage, 0, c->n3);
 }
 
 int mhd_static(mhd_ctx_t* c)
@@ -1345,22 +1336,29 @@ int mhd_set_state(mhd_ctx_t* c, const double* r, const double* t, const double* 
         const long m = c->nxy;
         std::vector<double> mxv(nz, 0.0), myv(nz, 0.0), fl(n);
         double mz = 0.0;
-        for (int k = 0; k < nz; ++k) {
-            for (long q = 0; q < m; ++q) {
-                mxv[k] += bx[(long)k * m + q];
-                myv[k] += by[(long)k * m + q];
+        // planes (and elements) are independent, so the threads' results are those of one
+        host_parallel(nz, std::max(1L, XFER_SERIAL / m), [&](long k0, long k1) {
+            for (long k = k0; k < k1; ++k) {
+                for (long q = 0; q < m; ++q) {
+                    mxv[k] += bx[k * m + q];
+                    myv[k] += by[k * m + q];
+                }
+                mxv[k] /= (double)m;
+                myv[k] /= (double)m;
             }
-            mxv[k] /= (double)m;
-            myv[k] /= (double)m;
-        }
+        });
         for (long q = 0; q < m; ++q) mz += bz[q];
         mz /= (double)m;
-        for (long q = 0; q < n; ++q) fl[q] = bx[q] - mxv[q / m];
-        TRY(upload(c, c->bx, 1, fl.data(), n));
-        for (long q = 0; q < n; ++q) fl[q] = by[q] - myv[q / m];
-        TRY(upload(c, c->by, 1, fl.data(), n));
-        for (long q = 0; q < n; ++q) fl[q] = bz[q] - mz;
-        TRY(upload(c, c->bz, 1, fl.data(), n));
+        auto send = [&](void* dst, const double* b, auto mean) -> int {
+            host_parallel(nz, std::max(1L, XFER_SERIAL / m), [&](long k0, long k1) {
+                for (long k = k0; k < k1; ++k)
+                    for (long q = k * m; q < (k + 1) * m; ++q) fl[q] = b[q] - mean(k);
+            });
+            return upload(c, dst, 1, fl.data(), n);
+        };
+        TRY(send(c->bx, bx, [&](long k) { return mxv[k]; }));
+        TRY(send(c->by, by, [&](long k) { return myv[k]; }));
+        TRY(send(c->bz, bz, [&](long) { return mz; }));
         MHD_HIP_CHECK(hipMemcpy(c->bxbar, mxv.data(), nz * sizeof(double), hipMemcpyHostToDevice));
         MHD_HIP_CHECK(hipMemcpy(c->bybar, myv.data(), nz * sizeof(double), hipMemcpyHostToDevice));
         c->sc.bzbar = mz;
