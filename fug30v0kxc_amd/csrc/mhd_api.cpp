@@ -111,6 +111,7 @@ struct mhd_ctx {
 
     mhd_scalars_t sc;
     int have_state;
+    int band_clean;    // pol and tor are zero in the 2/3 band
 
     int timed_kernel;
     int nev;
@@ -650,6 +651,8 @@ int run_mag_deriv(mhd_ctx* c, const double* cf = nullptr)
     if (cf) {
         m.ab3 = 1;
         m.c0 = cf[0]; m.c1 = cf[1]; m.c2 = cf[2];
+        // a recorded step may replay after set_field has put values in the band
+        m.clean = c->band_clean && !launch_recorder();
         for (int f = 0; f < 2; ++f) {
             m.mh1[f] = mlevel_ptr(c, f, 1);
             m.mh2[f] = mlevel_ptr(c, f, 2);
@@ -714,8 +717,10 @@ int run_bandj(mhd_ctx* c, bool clean)
     ZLaunch Z = zbase(c);
     Z.job[0] = zjob(c->pol, 0, m.polz, wf, ZK_D1, 5);  // 519
     Z.njobs = 1;
+    const bool fused = spectral_len_fixed(c->nx);
+    if (fused && clean) { Z.band = 1; Z.icutx = c->icutx; Z.icuty = c->icuty; }
     TRY(zrun(c, Z));
-    if (!spectral_len_fixed(c->nx)) {
+    if (!fused) {
         TRY(kerr(launch_bandj_spec(m, c->s)));
         return inverse_b_and_j(c, m, true);
     }
@@ -834,6 +839,7 @@ int run_mag_init(mhd_ctx* c)
         TRY(fill_bzm(c));
         MHD_HIP_CHECK(hipStreamSynchronize(c->s));
     }
+    c->band_clean = 1;   // pol and tor come from truncated spectra
     TRY(inverse_b_and_j(c, m, false));
     return run_mag_boundary(c, 0, 1);
 }
@@ -1442,6 +1448,7 @@ int mhd_set_field(mhd_ctx_t* c, int id, int level, const double* src)
     TRY(field_ref(c, id, level, &p, &f32, &n));
     // mixed: B is kept as fluctuations about its means; set it with mhd_set_state
     if (c->su && (id == MHD_F_BX || id == MHD_F_BY || id == MHD_F_BZ)) return MHD_E_ARG;
+    if (id == MHD_F_POL || id == MHD_F_TOR) c->band_clean = 0;
     TRY(upload(c, p, f32, src, n));
     if (id == MHD_F_U || id == MHD_F_V || id == MHD_F_W || id == MHD_F_T || id == MHD_F_R)
         TRY(refresh_shadows(c));
@@ -1539,6 +1546,7 @@ int mhd_step(mhd_ctx_t* c, int nsteps, double dt_fixed, int ndu06, mhd_diag_t* l
             if (mag) TRY(run_mag_deriv(c, cf)); // reads the old u v w; + AB3 of pol, tor, magdealias
             TRY(run_ab3(c, cf, mag ? 7 : 5));  // swaps
         }
+        c->band_clean = 1;   // magdealias is part of either update
         S.dt2 = dt + S.dt1;
         S.dt1 = dt;
         if (S.nit % 10 == 0) TRY(run_dealias5(c));

@@ -24,6 +24,12 @@ static inline unsigned nblk(long n, int nt = NT) { return (unsigned)((n + nt - 1
 // than one workgroup per compute unit (64^2 x 48: 9.0 us with 48 workgroups).
 // Recorded launches keep 16, so that boxes differing in nz stay one class.
 
+// 2/3 truncation band, src/magnetic.f90:666-717
+__device__ __forceinline__ bool in_band(int p, int q, int nx, int ny, int icx, int icy)
+{
+    return (p >= nx / 2 - icx && p <= nx / 2 + icx) || (q >= ny / 2 - icy && q <= ny / 2 + icy);
+}
+
 // TC: compute/output type; TIN: input element type; KIND: ZKind; PROD: the
 // input is scale*in*in1.  w (upwind selector) has the element type TW.
 template <typename TC, typename TIN, typename TW, int KIND, bool PROD, int ZKC>
@@ -42,6 +48,10 @@ __device__ __forceinline__ void ZKernel<TC, TIN, TW, KIND, PROD, ZKC>::body(cons
     const int nxy = L.g.nxy, nz = L.g.nz;
     const long col = (long)bid.x * NT + threadIdx.x;
     if (col >= nxy) return;
+    if (L.band) {
+        const int jq = (int)col / L.g.nx, ip = (int)col - jq * L.g.nx;
+        if (in_band(ip, jq, L.g.nx, L.g.ny, L.icutx, L.icuty)) return;
+    }
     const TIN* __restrict__ in = (const TIN*)J.in;
     const TIN* __restrict__ in1 = (const TIN*)J.in1;
     const TC scale = (TC)J.scale;
@@ -187,11 +197,6 @@ __device__ __forceinline__ double sdy(const TA* a, long base, int p, int q, int 
     const double v = (double)a[base + (long)(ny - q) * nx + p] * aky1[q];
     return (q < ny / 2) ? -v : v;
 }
-// 2/3 truncation band, src/magnetic.f90:666-717
-__device__ __forceinline__ bool in_band(int p, int q, int nx, int ny, int icx, int icy)
-{
-    return (p >= nx / 2 - icx && p <= nx / 2 + icx) || (q >= ny / 2 - icy && q <= ny / 2 + icy);
-}
 
 // src/magnetic.f90:362-407: cc = dEx/dy - dEy/dx, d = dEx/dx + dEy/dy by index
 // swaps, one thread per mirror quad as in bandj_spec_kernel
@@ -334,13 +339,26 @@ __device__ __forceinline__ void MagRhsKernel<TW>::body(const MagArgs& a, uint3 b
         dc[c] = (ip0 + c == 0 && jq == 0);
         band[c] = in_band(ip0 + c, jq, nx, a.g.ny, a.icutx, a.icuty);
     }
+    // magdealias clears pol and tor on the band (56 % of the plane) every step,
+    // so there neither they nor their histories, whose sum is cleared again,
+    // need be read; the right-hand sides and the zeros are still written
+    const bool zero = a.ab3 && a.clean && band[0] && band[1];
     const double* pol = a.pol;
     const double* tor = a.tor;
     const TW* __restrict__ dd = (const TW*)a.d;
     const double zck = a.p.zck, s = a.p.sc1;
     const TW hz = (TW)a.p.ho12;
     auto ld2 = [](const void* p, long q) { return *(const TW2*)((const TW*)p + q); };
-    auto ldd = [](const double* p, long q) { return *(const D2*)(p + q); };
+    auto ldd = [zero](const double* p, long q) {
+        D2 v = {0.0, 0.0};
+        if (!zero) v = *(const D2*)(p + q);
+        return v;
+    };
+    auto ldh = [zero](const void* p, long q) {
+        TW2 v = {(TW)0, (TW)0};
+        if (!zero) v = *(const TW2*)((const TW*)p + q);
+        return v;
+    };
     // interior planes [2, nz-2) use the centred stencils from the windows
     const int ki0 = k0 > 2 ? k0 : 2, ki1 = k1 < nz - 2 ? k1 : nz - 2;
     double pw[2][5], tw[2][5];
@@ -409,7 +427,7 @@ __device__ __forceinline__ void MagRhsKernel<TW>::body(const MagArgs& a, uint3 b
         *(TW2*)((TW*)a.tordot + q) = tdv;
         if (a.ab3) {
             // x + c0 f3 + c1 f2 + c2 f1, then the 2/3 band of pol and tor cleared
-            const TW2 ph2 = ld2(a.ph2, q), ph1 = ld2(a.ph1, q), th2 = ld2(a.th2, q), th1 = ld2(a.th1, q);
+            const TW2 ph2 = ldh(a.ph2, q), ph1 = ldh(a.ph1, q), th2 = ldh(a.th2, q), th1 = ldh(a.th1, q);
             const double ph2v[2] = {(double)ph2.x, (double)ph2.y}, ph1v[2] = {(double)ph1.x, (double)ph1.y};
             const double th2v[2] = {(double)th2.x, (double)th2.y}, th1v[2] = {(double)th1.x, (double)th1.y};
             D2 pn, tn;

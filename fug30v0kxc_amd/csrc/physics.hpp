@@ -32,6 +32,7 @@ struct ZLaunch {
     double ho12, sc1;
     const void* w;     // upwind selector (the solver's w)
     int w_f32;
+    int band, icutx, icuty;   // band: the columns of the 2/3 band are neither read nor written
     int njobs;
     ZJob job[Z_MAX_JOBS];
 };
@@ -107,6 +108,7 @@ struct MagArgs {
     // magdealias; the new values go to polnew, tornew (other threads' z-windows
     // still read the old ones); ab3 = 0: right-hand sides only
     int ab3;
+    int clean;                           // pol and tor are zero in the 2/3 band
     double c0, c1, c2;
     const void *ph1, *ph2, *th1, *th2;   // history levels 1 and 2 of pol, tor
     const double *mh1[2], *mh2[2];       // ... and of the means
