@@ -871,12 +871,13 @@ RedArgs rargs(mhd_ctx* c, int op)
     if (c->su) { a.bxm = c->bxbar; a.bym = c->bybar; a.bzm = c->sc.bzbar; }
     a.partial = c->red_partial;
     a.result = c->red_result;
+    a.host = c->hbuf;
     return a;
 }
 
 int fetch_result(mhd_ctx* c, double* out, int n)
 {
-    MHD_HIP_CHECK(hipMemcpyAsync(c->hbuf, c->red_result, n * sizeof(double), hipMemcpyDeviceToHost, c->s));
+    // the finishing kernel wrote them into the pinned buffer
     MHD_HIP_CHECK(hipStreamSynchronize(c->s));
     memcpy(out, c->hbuf, n * sizeof(double));
     return 0;

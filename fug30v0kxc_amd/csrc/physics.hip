@@ -1058,7 +1058,6 @@ __global__ void __launch_bounds__(NT) reduce_plane_kernel(RedArgs a)
 __global__ void __launch_bounds__(NT) reduce_finish_kernel(RedArgs a)
 {
     const int nz = a.g.nz;
-    double* R = a.result;
     // per plane: its chunks combined in order (sums for the averages and
     // Nusselt, min / max for the others), one (plane, value) per thread, into
     // P[k * 8 + i]: in LDS when the planes fit, else past the chunk partials
@@ -1080,67 +1079,74 @@ __global__ void __launch_bounds__(NT) reduce_finish_kernel(RedArgs a)
         P[k * 8 + i] = x;
     }
     __syncthreads();
-    if (threadIdx.x != 0) return;
-    if (a.op == RED_GLOBALAVG) {
-        // src/utils.F90:83-127
-        double urbar = 0, vrbar = 0, rbar = 0, me = 0, ke = 0;
-        for (int k = 0; k < nz; ++k) {
-            const double* v = P + k * 8;
-            if (k == 0 || k == nz - 1) {
-                urbar += 0.5 * v[1];
-                vrbar += 0.5 * v[2];
-                rbar += 0.5 * v[0];
-                me += 0.25 * v[4];
-                ke += 0.5 * v[3];
-            } else {
-                urbar += v[1];
-                vrbar += v[2];
-                rbar += v[0];
-                me += 0.5 * v[4];
-                ke += v[3];
+    // The planes combined: minima and maxima by all threads (any order gives the
+    // same), the sums in plane order, one value per thread and eight planes
+    // loaded ahead.  With one thread for everything the LDS latency of its 2 nz
+    // dependent reads made this kernel 17 us at nz = 160.
+    __shared__ double sR[8];
+    if (sum) {
+        if ((int)threadIdx.x < nv && a.op == RED_GLOBALAVG) {
+            // src/utils.F90:83-127 (r, u, v, ke, B^2 sums; half weight on the walls)
+            const int i = threadIdx.x;
+            const double wall = i == 4 ? 0.25 : 0.5, inner = i == 4 ? 0.5 : 1.0;
+            double x = 0;
+            for (int k0 = 0; k0 < nz; k0 += 8) {
+                double y[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) y[q] = P[(k0 + q < nz ? k0 + q : 0) * 8 + i];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const int k = k0 + q;
+                    if (k < nz) x += (k == 0 || k == nz - 1 ? wall : inner) * y[q];
+                }
             }
+            sR[i] = x;
         }
-        R[0] = urbar / rbar;
-        R[1] = vrbar / rbar;
-        R[2] = ke * a.p.xzn;
-        R[3] = me * a.p.xzn;
+    } else if ((int)threadIdx.x < 64 * nv) {
+        // one wave per value
+        const int i = threadIdx.x / 64, lane = threadIdx.x % 64;
+        double x = P[i];
+        for (int k = lane; k < nz; k += 64) x = i == 0 ? fmin(x, P[k * 8 + i]) : fmax(x, P[k * 8 + i]);
+        for (int m = 32; m > 0; m >>= 1) {
+            const double y = __shfl_xor(x, m);
+            x = i == 0 ? fmin(x, y) : fmax(x, y);
+        }
+        if (lane == 0) sR[i] = x;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    double out[4] = {0.0, 0.0, 0.0, 0.0};
+    if (a.op == RED_GLOBALAVG) {
+        out[0] = sR[1] / sR[0];
+        out[1] = sR[2] / sR[0];
+        out[2] = sR[3] * a.p.xzn;
+        out[3] = sR[4] * a.p.xzn;
     } else if (a.op == RED_MINMAX) {
-        double mn = P[0], mx = P[1];
-        for (int k = 1; k < nz; ++k) {
-            mn = fmin(mn, P[k * 8]);
-            mx = fmax(mx, P[k * 8 + 1]);
-        }
-        R[0] = mn;
-        R[1] = mx;
+        out[0] = sR[0];
+        out[1] = sR[1];
     } else if (a.op == RED_DIVB) {
         // src/utils.F90:270-288: divbmax starts at -1e30, divbmin at 1.0
-        double mx = -1.0e30, mn = 1.0;
-        for (int k = 0; k < nz; ++k) {
-            mx = fmax(mx, P[k * 8 + 1]);
-            mn = fmin(mn, P[k * 8]);
-        }
-        R[0] = mx;
-        R[1] = mn;
+        out[0] = fmax(-1.0e30, sR[1]);
+        out[1] = fmin(1.0, sR[0]);
     } else if (a.op == RED_CALCDT) {
         // src/utils.F90:205-242
-        double denmn = P[0], vx = P[1], vz = P[2];
-        for (int k = 1; k < nz; ++k) {
-            denmn = fmin(denmn, P[k * 8]);
-            vx = fmax(vx, P[k * 8 + 1]);
-            vz = fmax(vz, P[k * 8 + 2]);
-        }
+        const double denmn = sR[0], vx = sR[1], vz = sR[2];
         const double dtcflx = 0.16 * a.p.dd / vx;
         const double dtcflz = 0.3 * a.p.dz / vz;
         const double dtviscx = a.p.dtvisc0x * denmn, dtviscz = a.p.dtvisc0z * denmn;
         const double dtdiffx = a.p.dtdiff0x * denmn, dtdiffz = a.p.dtdiff0z * denmn;
         const double mn = fmin(fmin(fmin(dtcflx, dtcflz), fmin(dtviscx, dtviscz)), fmin(dtdiffx, dtdiffz));
-        R[0] = a.p.sf * mn;
-        R[1] = denmn;
-        R[2] = vx;
-        R[3] = vz;
+        out[0] = a.p.sf * mn;
+        out[1] = denmn;
+        out[2] = vx;
+        out[3] = vz;
     } else if (a.op == RED_NUSSELT) {
         const double tzbar = P[0] * a.p.xn;
-        R[0] = (tzbar - a.p.nusstmp) / (a.p.theta - a.p.nusstmp);
+        out[0] = (tzbar - a.p.nusstmp) / (a.p.theta - a.p.nusstmp);
+    }
+    for (int i = 0; i < 4; ++i) {
+        a.result[i] = out[i];
+        a.host[i] = out[i];
     }
 }
 

@@ -173,6 +173,7 @@ struct RedArgs {
     double bzm;                 // mixed: mean of bz
     double* partial;            // nz * (RED_CHUNKS + 1) * 8
     double* result;             // 8 doubles
+    double* host;               // the same in pinned host memory (no copy is queued for them)
 };
 // workgroups per plane of a reduction: nz * RED_CHUNKS workgroups fill the
 // device (nz alone, 160 at 256x256x160, leaves CUs idle); the finishing
