@@ -55,6 +55,7 @@ constexpr int LDC = 32 + 8;     // [unit][cell] activations of one wave's 32 cel
 
 constexpr int FWD_NT = 256;     // 4 waves x 32 cells
 constexpr int CELLS_PER_WAVE = 32;
+constexpr int TRAIN_NT = 256;   // 4 waves share a tile of 32 cells, 16 hidden units each
 
 __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c)
 {
@@ -528,7 +529,9 @@ __global__ void __launch_bounds__(FWD_NT, 2) mlp_fwd_kernel(FwdArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// training: forward and backward of 32 cells per wave, one wave per workgroup
+// training: forward and backward of 32 cells by four waves, 16 hidden units each.
+// Bound by the latency of its chain of layers: with one wave per 32 cells, 128
+// waves on 256 compute units, a batch of 4096 took 31.5 us, with four 22.9.
 // ---------------------------------------------------------------------------
 struct TrainArgs {
     const bf16x8* grid;
@@ -553,7 +556,7 @@ __device__ __forceinline__ long sample_id(const TrainArgs& a, long r)
     return (long)(h % (unsigned long long)a.nsamples);
 }
 
-__global__ void __launch_bounds__(64) mlp_train_kernel(TrainArgs a)
+__global__ void __launch_bounds__(TRAIN_NT) mlp_train_kernel(TrainArgs a)
 {
     __shared__ __bf16 XT[NINP * LDC];          // [feature][cell]
     __shared__ __bf16 S0[NH * LDC];            // H1 [cell][LDH], later dZ1T [unit][LDC]
@@ -562,7 +565,8 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(TrainArgs a)
     __shared__ __bf16 S3[NH * LDC];            // H2T, later dZ2T [unit][cell]
     __shared__ __bf16 DY[CELLS_PER_WAVE * LDC];   // dL/dy [cell][32] (outputs 12..31 zero)
     __shared__ __bf16 DYT[NOUTP * LDC];           // [output][cell]
-    const int l = threadIdx.x, lr = l & 15, lg = l >> 4;
+    const int l = threadIdx.x & 63, lr = l & 15, lg = l >> 4;
+    const int wv = threadIdx.x >> 6, col = wv * 16 + lr;   // this wave's block of 16 units
     const long w = blockIdx.x;
     const long r0 = w * CELLS_PER_WAVE;
     float* P = a.partial + w * (long)NPARAM;
@@ -570,11 +574,9 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(TrainArgs a)
     const float sc = 2.0f / (12.0f * (float)a.batch);
 
     // ---- forward, layer 1 (features also stored transposed for dW1)
-    f32x4 z1[2][4], z2[2][4];
+    f32x4 z1[2], z2[2];
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) z1[rb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int rb = 0; rb < 2; ++rb) z1[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
         const Nbhd nbh(sample_id(a, r0 + rb * 16 + lr), a.n3, a.nx, a.ny, a.nz);
@@ -582,95 +584,87 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(TrainArgs a)
         for (int s = 0; s < 7; ++s) {
             const int nbr = s * 4 + lg;
             const bf16x8 av = nbr < 27 ? a.grid[nbh.at(nbr)] : zero8;
+            if ((s & 3) == wv)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) XT[(s * 32 + lg * 8 + j) * LDC + rb * 16 + lr] = av[j];
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb)
-                z1[rb][nb] = mfma(av, frag(a.w1t + (nb * 16 + lr) * NINP + s * 32 + lg * 8), z1[rb][nb]);
+                for (int j = 0; j < 8; ++j) XT[(s * 32 + lg * 8 + j) * LDC + rb * 16 + lr] = av[j];
+            z1[rb] = mfma(av, frag(a.w1t + col * NINP + s * 32 + lg * 8), z1[rb]);
         }
     }
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int rb = 0; rb < 2; ++rb) {
+        const float b = a.b1[col];
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            const int col = nb * 16 + lr;
-            const float b = a.b1[col];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = rb * 16 + lg * 4 + i;
-                z1[rb][nb][i] += b;
-                const __bf16 h = (__bf16)gelu(z1[rb][nb][i]);
-                S0[row * LDH + col] = h;
-                S1[col * LDC + row] = h;
-            }
+        for (int i = 0; i < 4; ++i) {
+            const int row = rb * 16 + lg * 4 + i;
+            z1[rb][i] += b;
+            const __bf16 h = (__bf16)gelu(z1[rb][i]);
+            S0[row * LDH + col] = h;
+            S1[col * LDC + row] = h;
         }
+    }
     __syncthreads();
     // ---- layer 2
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) z2[rb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int rb = 0; rb < 2; ++rb) z2[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const bf16x8 av = frag(&S0[(rb * 16 + lr) * LDH + s * 32 + lg * 8]);
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb)
-                z2[rb][nb] = mfma(av, frag(a.w2t + (nb * 16 + lr) * NH + s * 32 + lg * 8), z2[rb][nb]);
+            z2[rb] = mfma(av, frag(a.w2t + col * NH + s * 32 + lg * 8), z2[rb]);
         }
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            const int col = nb * 16 + lr;
-            const float b = a.b2[col];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = rb * 16 + lg * 4 + i;
-                z2[rb][nb][i] += b;
-                const __bf16 h = (__bf16)gelu(z2[rb][nb][i]);
-                S2[row * LDH + col] = h;
-                S3[col * LDC + row] = h;
-            }
-        }
-    __syncthreads();
-    // ---- layer 3 and dL/dy
-    f32x4 y[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-            y[rb] = mfma(frag(&S2[(rb * 16 + lr) * LDH + s * 32 + lg * 8]), frag(a.w3t + lr * NH + s * 32 + lg * 8),
-                         y[rb]);
-    const int o = lr;
-    float se = 0.f, db = 0.f;
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int rb = 0; rb < 2; ++rb) {
+        const float b = a.b2[col];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int row = rb * 16 + lg * 4 + i;
-            float dy = 0.f;
-            if (o < CL_NOUT && r0 + row < a.batch) {
-                const long sid = sample_id(a, r0 + row);
-                const long snap = sid / a.n3;
-                const float e = y[rb][i] + a.b3[o] - a.tn[(snap * CL_NOUT + o) * a.n3 + (sid - snap * a.n3)];
-                se += e * e;
-                dy = sc * e;
-            }
-            db += dy;
-            const __bf16 d = (__bf16)dy;
-            DY[row * LDC + o] = d;
-            DY[row * LDC + 16 + o] = (__bf16)0.f;
-            DYT[o * LDC + row] = d;
+            z2[rb][i] += b;
+            const __bf16 h = (__bf16)gelu(z2[rb][i]);
+            S2[row * LDH + col] = h;
+            S3[col * LDC + row] = h;
         }
-    db += __shfl_xor(db, 16);
-    db += __shfl_xor(db, 32);
-    if (lg == 0 && o < CL_NOUT) P[OFF_B3 + o] = db;
+    }
+    __syncthreads();
+    // ---- layer 3 and dL/dy (16 outputs: one wave)
+    const int o = lr;
+    float se = 0.f;
+    if (wv == 0) {
+        f32x4 y[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+                y[rb] = mfma(frag(&S2[(rb * 16 + lr) * LDH + s * 32 + lg * 8]), frag(a.w3t + lr * NH + s * 32 + lg * 8),
+                             y[rb]);
+        float db = 0.f;
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = rb * 16 + lg * 4 + i;
+                float dy = 0.f;
+                if (o < CL_NOUT && r0 + row < a.batch) {
+                    const long sid = sample_id(a, r0 + row);
+                    const long snap = sid / a.n3;
+                    const float e = y[rb][i] + a.b3[o] - a.tn[(snap * CL_NOUT + o) * a.n3 + (sid - snap * a.n3)];
+                    se += e * e;
+                    dy = sc * e;
+                }
+                db += dy;
+                const __bf16 d = (__bf16)dy;
+                DY[row * LDC + o] = d;
+                DY[row * LDC + 16 + o] = (__bf16)0.f;
+                DYT[o * LDC + row] = d;
+            }
+        db += __shfl_xor(db, 16);
+        db += __shfl_xor(db, 32);
+        if (lg == 0 && o < CL_NOUT) P[OFF_B3 + o] = db;
+    }
     __syncthreads();
     // ---- dW3 = H2^T dY
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
+    {
+        const int mb = wv;
         f32x4 g = mfma(frag(&S3[(mb * 16 + lr) * LDC + lg * 8]), frag(&DYT[lr * LDC + lg * 8]),
                        f32x4{0.f, 0.f, 0.f, 0.f});
         if (o < CL_NOUT)
@@ -682,23 +676,18 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(TrainArgs a)
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
         const bf16x8 av = frag(&DY[(rb * 16 + lr) * LDC + lg * 8]);
+        const f32x4 d = mfma(av, frag(a.w3n + col * 32 + lg * 8), f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            const f32x4 d = mfma(av, frag(a.w3n + (nb * 16 + lr) * 32 + lg * 8), f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int i = 0; i < 4; ++i) z2[rb][nb][i] = d[i] * dgelu(z2[rb][nb][i]);   // now dZ2
-        }
+        for (int i = 0; i < 4; ++i) z2[rb][i] = d[i] * dgelu(z2[rb][i]);   // now dZ2
     }
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-        const int col = nb * 16 + lr;
+    {
         float s = 0.f;
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int row = rb * 16 + lg * 4 + i;
-                const float v = z2[rb][nb][i];
+                const float v = z2[rb][i];
                 s += v;
                 const __bf16 h = (__bf16)v;
                 S2[row * LDH + col] = h;
@@ -713,36 +702,28 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(TrainArgs a)
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
         const bf16x8 av = frag(&S1[(mb * 16 + lr) * LDC + lg * 8]);
+        const f32x4 g = mfma(av, frag(&S3[col * LDC + lg * 8]), f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            const f32x4 g = mfma(av, frag(&S3[(nb * 16 + lr) * LDC + lg * 8]), f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int i = 0; i < 4; ++i) P[OFF_W2 + (mb * 16 + lg * 4 + i) * NH + nb * 16 + lr] = g[i];
-        }
+        for (int i = 0; i < 4; ++i) P[OFF_W2 + (mb * 16 + lg * 4 + i) * NH + col] = g[i];
     }
     // ---- dZ1 = (dZ2 W2^T) gelu'(z1)
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int rb = 0; rb < 2; ++rb) {
+        f32x4 d = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            f32x4 d = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < 2; ++s)
+            d = mfma(frag(&S2[(rb * 16 + lr) * LDH + s * 32 + lg * 8]), frag(a.w2n + col * NH + s * 32 + lg * 8), d);
 #pragma unroll
-            for (int s = 0; s < 2; ++s)
-                d = mfma(frag(&S2[(rb * 16 + lr) * LDH + s * 32 + lg * 8]),
-                         frag(a.w2n + (nb * 16 + lr) * NH + s * 32 + lg * 8), d);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) z1[rb][nb][i] = d[i] * dgelu(z1[rb][nb][i]);   // now dZ1
-        }
+        for (int i = 0; i < 4; ++i) z1[rb][i] = d[i] * dgelu(z1[rb][i]);   // now dZ1
+    }
     __syncthreads();   // S0 (H1) is free: reused for dZ1T
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-        const int col = nb * 16 + lr;
+    {
         float s = 0.f;
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float v = z1[rb][nb][i];
+                const float v = z1[rb][i];
                 s += v;
                 S0[col * LDC + rb * 16 + lg * 4 + i] = (__bf16)v;
             }
@@ -752,43 +733,18 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(TrainArgs a)
     }
     __syncthreads();
     // ---- dW1 = X^T dZ1 (feature rows 216..223 are padding)
-    bf16x8 bz[4];
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) bz[nb] = frag(&S0[(nb * 16 + lr) * LDC + lg * 8]);
+    const bf16x8 bz = frag(&S0[col * LDC + lg * 8]);
     for (int mb = 0; mb < NINP / 16; ++mb) {
-        const bf16x8 av = frag(&XT[(mb * 16 + lr) * LDC + lg * 8]);
+        const f32x4 g = mfma(frag(&XT[(mb * 16 + lr) * LDC + lg * 8]), bz, f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            const f32x4 g = mfma(av, bz[nb], f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int f = mb * 16 + lg * 4 + i;
-                if (f < NIN) P[OFF_W1 + f * NH + nb * 16 + lr] = g[i];
-            }
+        for (int i = 0; i < 4; ++i) {
+            const int f = mb * 16 + lg * 4 + i;
+            if (f < NIN) P[OFF_W1 + f * NH + col] = g[i];
         }
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) se += __shfl_xor(se, off);
-    if (l == 0) a.lossp[w] = se;
-}
-
-// fixed-order sum of the per-wave gradients (and of the loss partials)
-__global__ void __launch_bounds__(256) grad_reduce_kernel(const float* partial, const float* lossp, long nw,
-                                                          float* grad, double* loss)
-{
-    const long p = (long)blockIdx.x * 256 + threadIdx.x;
-    // the sums run in wave order; unrolled, so a thread keeps 16 loads in flight
-    if (p < NPARAM) {
-        double s = 0.0;
-#pragma unroll 16
-        for (long w = 0; w < nw; ++w) s += (double)partial[w * NPARAM + p];
-        grad[p] = (float)s;
-    } else if (p == NPARAM) {
-        double s = 0.0;
-#pragma unroll 16
-        for (long w = 0; w < nw; ++w) s += (double)lossp[w];
-        *loss = s;
-    }
+    if (threadIdx.x == 0) a.lossp[w] = se;
 }
 
 struct Packed {
@@ -827,19 +783,44 @@ __global__ void __launch_bounds__(256) pack_kernel(const float* prm, Packed k)
 }
 
 // Adam (beta1 0.9, beta2 0.999, eps 1e-8) on the FP32 master weights
-__global__ void __launch_bounds__(256) adam_kernel(float* prm, float* m, float* v, const float* g, float lr, float c1,
-                                                   float c2, Packed k)
+struct AdamArgs {
+    float *prm, *m, *v;
+    float lr, c1, c2;
+    Packed k;
+};
+
+// Fixed-order sum of the per-tile gradients (and of the loss partials), and with
+// ADAM the update of the parameter summed.  Bound by the latency of its loads: a
+// thread keeps 64 in flight (16: 7.5 us for 128 tiles, and 5.3 us for the update
+// as a launch of its own).
+template <bool ADAM>
+__global__ void __launch_bounds__(256) grad_reduce_kernel(const float* __restrict__ partial,
+                                                          const float* __restrict__ lossp, long nw,
+                                                          float* __restrict__ grad, double* __restrict__ loss,
+                                                          AdamArgs o)
 {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= NPARAM) return;
-    const float gi = g[p];
-    const float mi = 0.9f * m[p] + 0.1f * gi;
-    const float vi = 0.999f * v[p] + 0.001f * gi * gi;
-    m[p] = mi;
-    v[p] = vi;
-    const float x = prm[p] - lr * (mi / c1) / (sqrtf(vi / c2) + 1e-8f);
-    prm[p] = x;
-    pack_one(k, p, x);
+    const long p = (long)blockIdx.x * 256 + threadIdx.x;
+    if (p < NPARAM) {
+        double s = 0.0;
+#pragma unroll 64
+        for (long w = 0; w < nw; ++w) s += (double)partial[w * NPARAM + p];
+        const float gi = (float)s;
+        grad[p] = gi;
+        if constexpr (ADAM) {
+            const float mi = 0.9f * o.m[p] + 0.1f * gi;
+            const float vi = 0.999f * o.v[p] + 0.001f * gi * gi;
+            o.m[p] = mi;
+            o.v[p] = vi;
+            const float x = o.prm[p] - o.lr * (mi / o.c1) / (sqrtf(vi / o.c2) + 1e-8f);
+            o.prm[p] = x;
+            pack_one(o.k, (int)p, x);
+        }
+    } else if (p == NPARAM) {
+        double s = 0.0;
+#pragma unroll 64
+        for (long w = 0; w < nw; ++w) s += (double)lossp[w];
+        *loss = s;
+    }
 }
 
 struct TendArgs {
@@ -1071,7 +1052,8 @@ int launch_fwd(const FwdArgs& a0, hipStream_t s)
     return ok(hipGetLastError()) ? 0 : MHD_E_DEVICE;
 }
 
-int run_train(mhd_closure* c, int batch, const long* dcells, long step)
+// one gradient of `batch` samples; with `adam`, the update too
+int run_train(mhd_closure* c, int batch, const long* dcells, long step, const AdamArgs* adam = nullptr)
 {
     const long nw = (batch + CELLS_PER_WAVE - 1) / CELLS_PER_WAVE;
     int e = ensure((void**)&c->partial, &c->pcap, nw, NPARAM * sizeof(float));
@@ -1092,9 +1074,14 @@ int run_train(mhd_closure* c, int batch, const long* dcells, long step)
     a.b1 = c->k.b1; a.b2 = c->k.b2; a.b3 = c->k.b3;
     a.partial = c->partial;
     a.lossp = c->lossp;
-    hipLaunchKernelGGL(mlp_train_kernel, dim3((unsigned)nw), dim3(64), 0, c->s, a);
-    hipLaunchKernelGGL(grad_reduce_kernel, dim3(nblk(NPARAM + 1)), dim3(256), 0, c->s, c->partial, c->lossp, nw,
-                       c->g, c->dloss);
+    hipLaunchKernelGGL(mlp_train_kernel, dim3((unsigned)nw), dim3(TRAIN_NT), 0, c->s, a);
+    const dim3 gr(nblk(NPARAM + 1));
+    if (adam)
+        hipLaunchKernelGGL(grad_reduce_kernel<true>, gr, dim3(256), 0, c->s, c->partial, c->lossp, nw, c->g, c->dloss,
+                           *adam);
+    else
+        hipLaunchKernelGGL(grad_reduce_kernel<false>, gr, dim3(256), 0, c->s, c->partial, c->lossp, nw, c->g,
+                           c->dloss, AdamArgs{});
     return ok(hipGetLastError()) ? 0 : MHD_E_DEVICE;
 }
 
@@ -1475,14 +1462,12 @@ int mhd_closure_train(mhd_closure_t* c, int steps, int batch, double lr, double*
     int e = prepare(c);
     if (e) return e;
     for (int it = 0; it < steps; ++it) {
-        e = run_train(c, batch, nullptr, c->adam_t);
+        const double t = (double)(c->adam_t + 1);
+        const AdamArgs o = {c->prm, c->m, c->v, (float)lr, 1.0f - (float)std::pow(0.9, t),
+                            1.0f - (float)std::pow(0.999, t), c->k};
+        e = run_train(c, batch, nullptr, c->adam_t, &o);
         if (e) return e;
         c->adam_t += 1;
-        const float c1 = 1.0f - (float)std::pow(0.9, (double)c->adam_t);
-        const float c2 = 1.0f - (float)std::pow(0.999, (double)c->adam_t);
-        hipLaunchKernelGGL(adam_kernel, dim3(nblk(NPARAM)), dim3(256), 0, c->s, c->prm, c->m, c->v, c->g, (float)lr,
-                           c1, c2, c->k);
-        if (!ok(hipGetLastError())) return MHD_E_DEVICE;
     }
     if (loss) {
         double L = 0.0;
