@@ -59,7 +59,7 @@ struct ExpandK {
                 dst[r] = {0.0, 0.0};
                 if (ok && j < NB0) {
                     const long n = (long)(j + r * NB0) * st;
-                    if constexpr (DIR == 1) dst[r] = ld_pair(a.in, ia + n);
+                    if constexpr (DIR != 0) dst[r] = ld_pair(a.in, ia + n);
                     else dst[r] = {a.in[ia + n], a.in[ib + n]};
                 }
             }
@@ -140,7 +140,7 @@ static int launch_expand_n(const ExpandArgs& a, hipStream_t s)
     if (a.dir == 0) return launch_expand_one<PL, 0, spec_b<double, PL, 0>()>(a, s);
     constexpr int B = spec_b<double, PL, 1>();
     if (a.g.nx % (2 * B) == 0) return launch_expand_one<PL, 1, B>(a, s);
-    return launch_expand_one<PL, 1, 1>(a, s);
+    return launch_expand_one<PL, 2, B>(a, s);
 }
 
 }  // namespace mhd

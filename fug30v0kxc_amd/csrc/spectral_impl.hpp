@@ -190,6 +190,12 @@ __device__ __forceinline__ cpx<TC> apply_mul(int kind, cpx<TC> z, int k, double 
     }
 }
 
+// DIR: 0 along x, 1 along y, 2 along y where B does not divide the column pairs
+// of a row: the last group of each row is partly filled.  (Those boxes ran groups
+// of one pair, workgroups of 15 threads and 16-byte row segments at 30 x 30: the
+// y passes of a step, second derivatives, EMF and inverse, went from 17.4, 9.3 and
+// 10.4 us to 11.9, 8.1 and 8.2 at 60 planes FP64.  A kernel of its own, so that
+// full groups carry no mask.)
 template <typename PL, int DIR, int B>
 struct Lines {
     static constexpr int N = PL::N;
@@ -204,7 +210,11 @@ struct Lines {
     static __host__ __device__ __forceinline__ long groups(const Geom& g)
     {
         if constexpr (DIR == 0) return ((long)g.nz * g.ny / 2 + B - 1) / B;
-        else return (long)g.nz * (g.nx / (2 * B));
+        else return (long)g.nz * row_groups(g);
+    }
+    static __host__ __device__ __forceinline__ int row_groups(const Geom& g)
+    {
+        return DIR == 2 ? (g.nx / 2 + B - 1) / B : g.nx / (2 * B);
     }
     // global index of element 0 of the transform's lines a and b in group grp
     static __device__ __forceinline__ bool base(const Geom& g, long grp, int t, long& ia, long& ib, long& step,
@@ -219,13 +229,13 @@ struct Lines {
             step = 1;
             return cl < (long)g.nz * g.ny / 2;
         } else {
-            const int tpp = g.nx / (2 * B);
+            const int tpp = row_groups(g);
             k = (int)(grp / tpp);
             const int x0 = (int)(grp - (long)k * tpp) * 2 * B;
             ia = (long)k * g.nxy + x0 + 2 * t;
             ib = ia + 1;
             step = g.nx;
-            return true;
+            return DIR == 1 || x0 + 2 * t < g.nx;
         }
     }
 };
@@ -266,7 +276,7 @@ struct SpecK {
     // so a line is fetched once.  Identity otherwise.
     static __device__ __forceinline__ long paired_group(long item, long G, long ngrp)
     {
-        constexpr bool half_line = DIR == 1 && 2 * B * (int)sizeof(TC) < 128;
+        constexpr bool half_line = DIR != 0 && 2 * B * (int)sizeof(TC) < 128;
         if constexpr (half_line) {
             if (G % 16 == 0 && ngrp % 16 == 0) {
                 const long c = item & 15;
@@ -303,7 +313,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::r2hc_store(cpx
             TC a, b;
             if (n <= N / 2) { a = (TC)0.5 * (zk.x + zn.x); b = (TC)0.5 * (zk.y + zn.y); }
             else { a = (TC)0.5 * (zk.y - zn.y); b = (TC)0.5 * (zn.x - zk.x); }
-            if constexpr (DIR == 1) st_pair(out0, ia + n * st, a, b);
+            if constexpr (DIR != 0) st_pair(out0, ia + n * st, a, b);
             else {
                 out0[ia + n * st] = a;
                 out0[ib + n * st] = b;
@@ -349,7 +359,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_cross3(co
             const int n = j + r * NB0;
             dst[0][r] = dst[1][r] = dst[2][r] = {(TC)0, (TC)0};
             if (ok && j < NB0) {
-                if constexpr (DIR == 1) {
+                if constexpr (DIR != 0) {
                     const long i = ia + n * st;
                     const cpx<TC> x0 = ld_pair(a0, i), x1 = ld_pair(a1, i), x2 = ld_pair(a2, i);
                     const cpx<TC> y0 = ld_pair(b0, i), y1 = ld_pair(b1, i), y2 = ld_pair(b2, i);
@@ -446,7 +456,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_deriv2(co
             const long n = (long)(j + r * NB0) * st;
             dst[r] = {(TC)0, (TC)0};
             if (ok && j < NB0) {
-                if constexpr (DIR == 1) dst[r] = ld_pair(p, ia + n);
+                if constexpr (DIR != 0) dst[r] = ld_pair(p, ia + n);
                 else dst[r] = {p[ia + n], p[ib + n]};
             }
         }
@@ -528,7 +538,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_deriv2(co
 #pragma unroll
                     for (int r = 0; r < R0; ++r) {
                         const int n = j + r * NB0;
-                        if constexpr (DIR == 1) st_pair_nt(out, ia + n * st, v[r].x, v[r].y);
+                        if constexpr (DIR != 0) st_pair_nt(out, ia + n * st, v[r].x, v[r].y);
                         else {
                             st_nt(out, ia + n * st, v[r].x);
                             st_nt(out, ib + n * st, v[r].y);
@@ -570,7 +580,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
     // next group.  Within every 16 items, item c (< 8) takes group 2c and item
     // c + 8 group 2c + 1: workgroups w and w + 8 run on the same XCD (they are
     // dealt round-robin over 8) at the same time, so a line is fetched once.
-    constexpr bool half_line = DIR == 1 && 2 * B * (int)sizeof(TC) < 128;
+    constexpr bool half_line = DIR != 0 && 2 * B * (int)sizeof(TC) < 128;
     const bool pair = half_line && (G % 16 == 0) && (ngrp % 16 == 0);
     // (job, line group) of an item
     auto decode = [&](long item, int& jb, long& grp) {
@@ -598,7 +608,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
                 const int n = j + r * NB0;
                 dst[r] = {(TC)0, (TC)0};
                 if (ok && j < NB0 && !(L.skip && n >= N / 2 - icut && n <= N / 2 + icut)) {
-                    if constexpr (DIR == 1) dst[r] = ld_pair(src, ia + n * st);
+                    if constexpr (DIR != 0) dst[r] = ld_pair(src, ia + n * st);
                     else dst[r] = {src[ia + n * st], src[ib + n * st]};
                 }
             }
@@ -609,7 +619,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
                 const int n = j + r * NB0;
                 dst[r] = {(TC)0, (TC)0};
                 if (ok && j < NB0) {
-                    if constexpr (DIR == 1) dst[r] = ld.pair(ia + n * st);
+                    if constexpr (DIR != 0) dst[r] = ld.pair(ia + n * st);
                     else dst[r] = {ld(ia + n * st), ld(ib + n * st)};
                 }
             }
@@ -669,7 +679,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
                     for (int r = 0; r < R0; ++r) {
                         const int n = j + r * NB0;
                         const TC xa = v[r].x * sc + ad, xb = v[r].y * sc + ad;
-                        if constexpr (DIR == 1) st_pair(out, ia + n * st, xa, xb);
+                        if constexpr (DIR != 0) st_pair(out, ia + n * st, xa, xb);
                         else {
                             out[ia + n * st] = xa;
                             out[ib + n * st] = xb;
@@ -696,7 +706,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
 #pragma unroll
                     for (int r = 0; r < R0; ++r) {
                         const int n = j + r * NB0;
-                        if constexpr (DIR == 1) st_pair_nt(out0, ia + n * st, v[r].x + add, v[r].y + add);
+                        if constexpr (DIR != 0) st_pair_nt(out0, ia + n * st, v[r].x + add, v[r].y + add);
                         else {
                             st_nt(out0, ia + n * st, v[r].x + add);
                             st_nt(out0, ib + n * st, v[r].y + add);
@@ -725,7 +735,7 @@ constexpr int spec_b()
     constexpr int tpt = plan_tpt<PL>();
     constexpr int sp = RegFFT<TC, PL>::SP * (int)sizeof(cpx<TC>);
     constexpr int twb = RegFFT<TC, PL>::TWN * (int)sizeof(cpx<TC>);
-    constexpr int lim = (DIR == 1 && sizeof(TC) == 8) ? SPEC_LDS_Y : SPEC_LDS_X;
+    constexpr int lim = (DIR != 0 && sizeof(TC) == 8) ? SPEC_LDS_Y : SPEC_LDS_X;
     // FP64 y groups of 8 pairs (128-byte rows); 16 (256-byte rows) where a
     // transform takes at most 16 threads, so the group stays at 256 threads
     int b = DIR == 0 ? (128 / tpt > 0 ? 128 / tpt : 1) : (sizeof(TC) == 8 ? (tpt <= 16 ? 16 : 8) : 16);
@@ -788,7 +798,7 @@ static int launch_one(const SpecLaunch& L, hipStream_t s)
 template <typename TC, typename PL, int DIR, int B>
 static int launch_mode(const SpecLaunch& L, hipStream_t s)
 {
-    if constexpr (DIR == 1) {
+    if constexpr (DIR != 0) {
         if (L.cross3) return launch_one<TC, PL, DIR, B, SM_R2HC, LD_CROSS3>(L, s);
     }
     const int lop = L.job[0].load_op;
@@ -821,7 +831,9 @@ static int launch_plan(const SpecLaunch& L, hipStream_t s)
     constexpr int BC = sizeof(TC) == 8 && B0 >= 8 ? B0 / 2 : B0;
     if (L.cross3 && L.g.nx % (2 * BC) == 0) return launch_one<TC, PL, 1, BC, SM_R2HC, LD_CROSS3>(L, s);
     if (L.g.nx % (2 * B0) == 0) return launch_mode<TC, PL, 1, B0>(L, s);
-    return launch_mode<TC, PL, 1, 1>(L, s);
+    if (B2 != B0 && L.mode == SM_DERIV2) return launch_one<TC, PL, 2, B2, SM_DERIV2, LD_PLAIN>(L, s);
+    if (BC != B0 && L.cross3) return launch_one<TC, PL, 2, BC, SM_R2HC, LD_CROSS3>(L, s);
+    return launch_mode<TC, PL, 2, B0>(L, s);
 }
 
 template <typename TC, int N>
