@@ -845,7 +845,7 @@ static int launch_n(const SpecLaunch& L, hipStream_t s)
     if constexpr (!std::is_void<typename AltPlan2<N>::type>::value) {
         if (L.variant == 2) return launch_plan<TC, typename AltPlan2<N>::type>(L, s);
     }
-    if (L.mode == SM_DERIV2) return launch_plan<TC, typename D2Plan<N>::type>(L, s);
+    if (L.mode == SM_DERIV2) return launch_plan<TC, typename D2Plan<N, TC>::type>(L, s);
     return launch_plan<TC, FftPlan<N>>(L, s);
 }
 
