@@ -32,6 +32,10 @@ struct FftPlan;
 // registers, high occupancy) beat radix-16 ones although they add LDS passes
 // (measured at 256x256x160 FP64: x d1+d2 243 us with 4x4x4x4 vs 265 us with
 // 16x16; x d1 143 us vs 162 us).
+// Up to 256 every multiple of 4 with no factors but 2, 3 and 5 has a plan: the
+// transforms of a step at 100 x 144 x 61 FP64 take 215 us so, 467 with the
+// run-time radix kernels and the quad kernels behind them.  Twice an odd number stays there (a radix 2 would set
+// the threads of a transform and leave half of them idle in the other passes).
 MHD_PLAN(8, 8)
 MHD_PLAN(12, 4, 3)
 MHD_PLAN(16, 4, 4)
@@ -39,16 +43,24 @@ MHD_PLAN(20, 4, 5)
 MHD_PLAN(24, 8, 3)
 MHD_PLAN(30, 2, 3, 5)
 MHD_PLAN(32, 4, 8)
+MHD_PLAN(36, 4, 3, 3)
 MHD_PLAN(40, 8, 5)
 MHD_PLAN(48, 4, 4, 3)
 MHD_PLAN(60, 4, 3, 5)
 MHD_PLAN(64, 4, 4, 4)
+MHD_PLAN(72, 8, 3, 3)
 MHD_PLAN(80, 4, 4, 5)
 MHD_PLAN(96, 4, 8, 3)
+MHD_PLAN(100, 4, 5, 5)
+MHD_PLAN(108, 4, 3, 3, 3)
 MHD_PLAN(120, 8, 3, 5)
 MHD_PLAN(128, 4, 4, 8)
+MHD_PLAN(144, 4, 4, 3, 3)
 MHD_PLAN(160, 8, 4, 5)
+MHD_PLAN(180, 4, 3, 3, 5)
 MHD_PLAN(192, 4, 4, 4, 3)
+MHD_PLAN(200, 8, 5, 5)
+MHD_PLAN(216, 8, 3, 3, 3)
 MHD_PLAN(240, 4, 4, 3, 5)
 MHD_PLAN(256, 4, 4, 4, 4)
 MHD_PLAN(320, 4, 4, 4, 5)
@@ -95,9 +107,12 @@ template <int N, typename TC>
 struct D2Plan {
     using type = FftPlan<N>;
 };
+template <typename TC> struct D2Plan<72, TC> { using type = Plan<72, 3, 8, 3>; };
 template <typename TC> struct D2Plan<120, TC> { using type = Plan<120, 3, 8, 5>; };
 template <typename TC> struct D2Plan<128, TC> { using type = Plan<128, 4, 8, 4>; };
 template <typename TC> struct D2Plan<160, TC> { using type = Plan<160, 4, 8, 5>; };
+template <typename TC> struct D2Plan<200, TC> { using type = Plan<200, 5, 8, 5>; };
+template <typename TC> struct D2Plan<216, TC> { using type = Plan<216, 3, 8, 3, 3>; };
 template <typename TC> struct D2Plan<480, TC> { using type = Plan<480, 4, 8, 3, 5>; };
 template <typename TC> struct D2Plan<512, TC> { using type = Plan<512, 4, 4, 8, 4>; };
 // FP32 passes of 512 points have the registers for three radix-8 passes, one LDS

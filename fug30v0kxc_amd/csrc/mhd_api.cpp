@@ -246,6 +246,9 @@ int kerr(int e) { return e ? MHD_E_DEVICE : 0; }
 // workgroups of columns: `most`, or fewer where even 8 planes would leave the
 // device with less than two workgroups per compute unit.  Recorded launches run
 // together with those of other boxes, so there the walk is not cut short.
+// 64^2 x 48 FP64: hydro_col 32 + 15 us (walls) -> 25, mag_rhs 17.5 -> 7.8, jsq 11 -> 5.2;
+// from 256^2 columns on longer walks are the faster ones (mag_rhs and jsq 30 us
+// less at 8 planes than at 24, hydro_col alike within 3 %).
 int walk_planes(const mhd_ctx* c, long groups, int planes, int most)
 {
     const long fit = groups * planes / (2L * c->ncu);

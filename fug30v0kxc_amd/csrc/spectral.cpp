@@ -6,26 +6,21 @@
 
 namespace mhd {
 
-int launch_spectral_g0(int n, const SpecLaunch& L, int f32, hipStream_t s);
-int launch_spectral_g0_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
-int launch_spectral_g0_expand(int n, const ExpandArgs& a, hipStream_t s);
-int launch_spectral_g1(int n, const SpecLaunch& L, int f32, hipStream_t s);
-int launch_spectral_g1_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
-int launch_spectral_g1_expand(int n, const ExpandArgs& a, hipStream_t s);
-int launch_spectral_g2(int n, const SpecLaunch& L, int f32, hipStream_t s);
-int launch_spectral_g2_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
-int launch_spectral_g2_expand(int n, const ExpandArgs& a, hipStream_t s);
-int launch_spectral_g3(int n, const SpecLaunch& L, int f32, hipStream_t s);
-int launch_spectral_g3_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
-int launch_spectral_g3_expand(int n, const ExpandArgs& a, hipStream_t s);
-int launch_spectral_g4(int n, const SpecLaunch& L, int f32, hipStream_t s);
-int launch_spectral_g4_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
-int launch_spectral_g4_expand(int n, const ExpandArgs& a, hipStream_t s);
-int launch_spectral_g5(int n, const SpecLaunch& L, int f32, hipStream_t s);
-int launch_spectral_g5_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);
-int launch_spectral_g5_expand(int n, const ExpandArgs& a, hipStream_t s);
+#define MHD_DECL(f)                                                              \
+    int f(int n, const SpecLaunch& L, int f32, hipStream_t s);                    \
+    int f##_mag(int n, int which, const MagSpecArgs& a, int f32, hipStream_t s);  \
+    int f##_expand(int n, const ExpandArgs& a, hipStream_t s);
+MHD_DECL(launch_spectral_g0)
+MHD_DECL(launch_spectral_g1)
+MHD_DECL(launch_spectral_g2)
+MHD_DECL(launch_spectral_g3)
+MHD_DECL(launch_spectral_g4)
+MHD_DECL(launch_spectral_g5)
+MHD_DECL(launch_spectral_g6)
+MHD_DECL(launch_spectral_g7)
+#undef MHD_DECL
 
-#define MHD_ALL_SIZES(X) X(8) X(12) X(16) X(20) X(24) X(30) X(32) X(40) X(48) X(60) X(64) X(80) X(96) X(120) X(128) X(160) X(192) X(240) X(256) X(320) X(384) X(480) X(512) X(640) X(768) X(1024)
+#define MHD_ALL_SIZES(X) X(8) X(12) X(16) X(20) X(24) X(30) X(32) X(36) X(40) X(48) X(60) X(64) X(72) X(80) X(96) X(100) X(108) X(120) X(128) X(144) X(160) X(180) X(192) X(200) X(216) X(240) X(256) X(320) X(384) X(480) X(512) X(640) X(768) X(1024)
 
 bool spectral_len_fixed(int n)
 {
@@ -56,43 +51,45 @@ int spectral_variants(int n)
     return 1;
 }
 
+// the file that instantiates a length's kernels
+static int size_group(int n)
+{
+    switch (n) {
+    case 36: case 72: case 100: case 108: return 6;
+    case 144: case 180: case 200: case 216: return 7;
+    }
+    return n <= 60 ? 0 : n <= 128 ? 1 : n <= 256 ? 2 : n <= 480 ? 3 : n <= 640 ? 4 : 5;
+}
+#define MHD_GROUP_FNS(k)                                                                                  \
+    launch_spectral_g0##k, launch_spectral_g1##k, launch_spectral_g2##k, launch_spectral_g3##k,           \
+        launch_spectral_g4##k, launch_spectral_g5##k, launch_spectral_g6##k, launch_spectral_g7##k
+
 static int launch_group(const SpecLaunch& L, int compute_f32, hipStream_t s)
 {
+    static constexpr decltype(&launch_spectral_g0) fn[] = {MHD_GROUP_FNS()};
     const int n = (L.dir == 0) ? L.g.nx : L.g.ny;
     if (!spectral_len_fixed(n)) return launch_spectral_generic(L, compute_f32, s);
-    if (n <= 60) return launch_spectral_g0(n, L, compute_f32, s);
-    if (n <= 128) return launch_spectral_g1(n, L, compute_f32, s);
-    if (n <= 256) return launch_spectral_g2(n, L, compute_f32, s);
-    if (n <= 480) return launch_spectral_g3(n, L, compute_f32, s);
-    if (n <= 640) return launch_spectral_g4(n, L, compute_f32, s);
-    return launch_spectral_g5(n, L, compute_f32, s);
+    return fn[size_group(n)](n, L, compute_f32, s);
 }
 
 static int launch_mag_x(int which, const MagSpecArgs& a, int f32, hipStream_t s)
 {
+    static constexpr decltype(&launch_spectral_g0_mag) fn[] = {MHD_GROUP_FNS(_mag)};
     const int n = a.g.nx;
     if (!spectral_len_fixed(n)) return -20;
-    if (n <= 60) return launch_spectral_g0_mag(n, which, a, f32, s);
-    if (n <= 128) return launch_spectral_g1_mag(n, which, a, f32, s);
-    if (n <= 256) return launch_spectral_g2_mag(n, which, a, f32, s);
-    if (n <= 480) return launch_spectral_g3_mag(n, which, a, f32, s);
-    if (n <= 640) return launch_spectral_g4_mag(n, which, a, f32, s);
-    return launch_spectral_g5_mag(n, which, a, f32, s);
+    return fn[size_group(n)](n, which, a, f32, s);
 }
 int launch_emf_x(const MagSpecArgs& a, int f32, hipStream_t s) { return launch_mag_x(0, a, f32, s); }
 int launch_bandj_x(const MagSpecArgs& a, int f32, hipStream_t s) { return launch_mag_x(1, a, f32, s); }
 
 int launch_expand(const ExpandArgs& a, hipStream_t s)
 {
+    static constexpr decltype(&launch_spectral_g0_expand) fn[] = {MHD_GROUP_FNS(_expand)};
     const int n = a.dir == 0 ? a.g.nx : a.g.ny;
     if (!spectral_len_fixed(n)) return -20;
-    if (n <= 60) return launch_spectral_g0_expand(n, a, s);
-    if (n <= 128) return launch_spectral_g1_expand(n, a, s);
-    if (n <= 256) return launch_spectral_g2_expand(n, a, s);
-    if (n <= 480) return launch_spectral_g3_expand(n, a, s);
-    if (n <= 640) return launch_spectral_g4_expand(n, a, s);
-    return launch_spectral_g5_expand(n, a, s);
+    return fn[size_group(n)](n, a, s);
 }
+#undef MHD_GROUP_FNS
 
 // Three LD_CROSS jobs whose factors are the components of two vectors a, b
 // with job q = a_{q+1} b_{q+2} - a_{q+2} b_{q+1}: the EMF u x B.
