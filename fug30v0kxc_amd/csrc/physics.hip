@@ -309,15 +309,19 @@ __device__ __forceinline__ void MeanEmfKernel<TW>::body(const MagArgs& a, uint3 
 // one-sided d2bydz rows (flag 3) with direct loads.  D_z of d (line 419,
 // d1bydz flag 5) comes from a third window, in the working precision (as a
 // separate z pass would compute and store it), instead of a stored array.
-template <typename TW>
+// SKIP (MagArgs::clean, FP64): the columns of the 2/3 band read neither pol, tor
+// nor their histories.  228 -> 197 us at 256^2 x 160 FP64; in FP32 the masked
+// loads cost what they save (153 and 152), and the batched kernel loses (53 ->
+// 71 us over six boxes), so those launch the plain one.
+template <typename TW, bool SKIP>
 struct MagRhsKernel {
     using Args = MagArgs;
     static constexpr int NT = 256;
     static __device__ __forceinline__ void body(const MagArgs& a, uint3 bid, uint3 gdim);
 };
 
-template <typename TW>
-__device__ __forceinline__ void MagRhsKernel<TW>::body(const MagArgs& a, uint3 bid, uint3 gdim)
+template <typename TW, bool SKIP>
+__device__ __forceinline__ void MagRhsKernel<TW, SKIP>::body(const MagArgs& a, uint3 bid, uint3 gdim)
 {
     (void)bid;
     (void)gdim;
@@ -342,7 +346,7 @@ __device__ __forceinline__ void MagRhsKernel<TW>::body(const MagArgs& a, uint3 b
     // magdealias clears pol and tor on the band (56 % of the plane) every step,
     // so there neither they nor their histories, whose sum is cleared again,
     // need be read; the right-hand sides and the zeros are still written
-    const bool zero = a.ab3 && a.clean && band[0] && band[1];
+    const bool zero = SKIP && a.ab3 && band[0] && band[1];
     const double* pol = a.pol;
     const double* tor = a.tor;
     const TW* __restrict__ dd = (const TW*)a.d;
@@ -709,8 +713,10 @@ int launch_mag_rhs(const MagArgs& a, hipStream_t s)
 {
     if (a.zc <= 0) return -10;
     if (a.g.nxy % 2) return -10;   // two columns per thread (nx is even)
-    MHD_LAUNCH_W(MagRhsKernel, dim3(nblk(a.g.nxy / 2), (unsigned)((a.g.nz + a.zc - 1) / a.zc)), dim3(NT), 0, s, a);
-    return 0;
+    const dim3 grid(nblk(a.g.nxy / 2), (unsigned)((a.g.nz + a.zc - 1) / a.zc));
+    if (a.wf32) return mhd_launch<MagRhsKernel<float, false>>(grid, dim3(NT), 0, s, a);
+    if (a.clean) return mhd_launch<MagRhsKernel<double, true>>(grid, dim3(NT), 0, s, a);
+    return mhd_launch<MagRhsKernel<double, false>>(grid, dim3(NT), 0, s, a);
 }
 int launch_bandj_spec(const MagArgs& a, hipStream_t s)
 {
