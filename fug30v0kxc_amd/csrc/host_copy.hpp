@@ -22,6 +22,11 @@ namespace mhd {
 constexpr int XFER_CHUNKS = 16;            // DMA chunks of one field, at most
 constexpr int XFER_THREADS = 16;
 constexpr long XFER_SERIAL = 1L << 17;     // doubles per thread below which threads do not pay
+// Fields from 32 MB on are copied by threads: that is where the C allocator's
+// largest threshold for a mapping of its own lies, so their destinations are
+// fresh pages.  Smaller ones are mostly memory in use before, which one thread
+// copies faster than a team starts: 48 fields of 1.5 to 12 MB took 15 ms longer.
+constexpr long XFER_MIN = 1L << 22;
 
 inline int host_threads(long n, long grain)
 {
@@ -73,7 +78,7 @@ void host_parallel(long n, long grain, Fn&& f)
 // hbuf (n doubles); ev: XFER_CHUNKS events.  Returns with the copy complete.
 inline hipError_t fetch_doubles(double* dst, const double* from, long n, double* hbuf, hipEvent_t* ev, hipStream_t s)
 {
-    const int T = host_threads(n, XFER_SERIAL);
+    const int T = n < XFER_MIN ? 1 : host_threads(n, XFER_SERIAL);
     if (T == 1) {
         // an event to wait for would cost 5 us a call
         hipError_t e = hipMemcpyAsync(hbuf, from, n * sizeof(double), hipMemcpyDeviceToHost, s);
@@ -123,7 +128,7 @@ inline hipError_t fetch_doubles(double* dst, const double* from, long n, double*
 // success and s has been synchronised (hbuf is in use until then)
 inline hipError_t send_doubles(double* to, const double* src, long n, double* hbuf, hipStream_t s)
 {
-    const int T = host_threads(n, XFER_SERIAL);
+    const int T = n < XFER_MIN ? 1 : host_threads(n, XFER_SERIAL);
     const int C = T == 1 ? 1 : XFER_CHUNKS;
     auto lo = [&](int c) { return n * c / C; };
     std::atomic<int> done[XFER_CHUNKS] = {};

@@ -1346,8 +1346,9 @@ int mhd_set_state(mhd_ctx_t* c, const double* r, const double* t, const double* 
         const long m = c->nxy;
         std::vector<double> mxv(nz, 0.0), myv(nz, 0.0), fl(n);
         double mz = 0.0;
+        const long grain = n < XFER_MIN ? nz : std::max(1L, XFER_SERIAL / m);   // planes per thread, at least
         // planes (and elements) are independent, so the threads' results are those of one
-        host_parallel(nz, std::max(1L, XFER_SERIAL / m), [&](long k0, long k1) {
+        host_parallel(nz, grain, [&](long k0, long k1) {
             for (long k = k0; k < k1; ++k) {
                 for (long q = 0; q < m; ++q) {
                     mxv[k] += bx[k * m + q];
@@ -1360,7 +1361,7 @@ int mhd_set_state(mhd_ctx_t* c, const double* r, const double* t, const double* 
         for (long q = 0; q < m; ++q) mz += bz[q];
         mz /= (double)m;
         auto send = [&](void* dst, const double* b, auto mean) -> int {
-            host_parallel(nz, std::max(1L, XFER_SERIAL / m), [&](long k0, long k1) {
+            host_parallel(nz, grain, [&](long k0, long k1) {
                 for (long k = k0; k < k1; ++k)
                     for (long q = k * m; q < (k + 1) * m; ++q) fl[q] = b[q] - mean(k);
             });

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 NAMES = ("r", "t", "u", "v", "w", "bx", "by", "bz")
 
 
-@pytest.mark.parametrize("shape", [(128, 96, 41), (64, 64, 33), (30, 30, 7)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("shape", [(256, 128, 129), (128, 96, 41), (30, 30, 7)], ids=lambda s: "x".join(map(str, s)))
 def test_round_trip(shape):
     from fug30v0kxc_amd import MHD_PREC_MIXED, Solver
     nx, ny, nz = shape
