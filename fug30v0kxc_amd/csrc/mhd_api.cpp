@@ -904,14 +904,20 @@ int run_nusselt(mhd_ctx* c, double* nu)
 
 int run_checkdivb(mhd_ctx* c, double out[2])
 {
-    // src/utils.F90:262-264: d/dx bx + d/dy by + d/dz bz (flag 5)
+    // src/utils.F90:262-264: d/dx bx + d/dy by + d/dz bz (flag 5).  In the mixed
+    // mode the three derivatives are FP32 and nearly cancel: the extremes carry
+    // their rounding (1e-8 to 2e-7 of the largest derivative) into 64-bit
+    // results.  So there the transforms keep one order of operations whatever
+    // plan a length has (direct): a caller sees the same digits.
     const int wf = c->wf32;
     void** W = c->wk;
     SpecLaunch L = spec_base(c, 0, SM_DERIV1);
+    L.direct = wf;
     L.job[0] = sjob(c->bx, wf, W[W_UY], nullptr, MUL_D1, 0, wf);
     L.njobs = 1;
     TRY(spec(c, L));
     SpecLaunch M = spec_base(c, 1, SM_DERIV1);
+    M.direct = wf;
     M.job[0] = sjob(c->by, wf, W[W_UYS], nullptr, MUL_D1, 0, wf);
     M.njobs = 1;
     TRY(spec(c, M));

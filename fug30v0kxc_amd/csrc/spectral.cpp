@@ -60,6 +60,8 @@ static int size_group(int n)
     }
     return n <= 60 ? 0 : n <= 128 ? 1 : n <= 256 ? 2 : n <= 480 ? 3 : n <= 640 ? 4 : 5;
 }
+// lengths with a plan that direct launches do not use (SpecLaunch::direct)
+static bool spectral_len_direct(int n) { return size_group(n) >= 6; }
 #define MHD_GROUP_FNS(k)                                                                                  \
     launch_spectral_g0##k, launch_spectral_g1##k, launch_spectral_g2##k, launch_spectral_g3##k,           \
         launch_spectral_g4##k, launch_spectral_g5##k, launch_spectral_g6##k, launch_spectral_g7##k
@@ -68,7 +70,7 @@ static int launch_group(const SpecLaunch& L, int compute_f32, hipStream_t s)
 {
     static constexpr decltype(&launch_spectral_g0) fn[] = {MHD_GROUP_FNS()};
     const int n = (L.dir == 0) ? L.g.nx : L.g.ny;
-    if (!spectral_len_fixed(n)) return launch_spectral_generic(L, compute_f32, s);
+    if (!spectral_len_fixed(n) || (L.direct && spectral_len_direct(n))) return launch_spectral_generic(L, compute_f32, s);
     return fn[size_group(n)](n, L, compute_f32, s);
 }
 

@@ -85,6 +85,10 @@ struct SpecLaunch {
     int variant;      // radix plan: 0 the default, 1 and 2 the length's alternatives (if any)
     int max_groups;   // optional further cap on the grid; 0 = none
     int group_major;  // set by the launcher: items ordered line group first (see spec_kernel)
+    // SM_DERIV1: lines without a register plan, and those of the eight lengths
+    // from 36 to 216 that gained theirs last (spectral_len_direct), are
+    // transformed output point by output point in the run-time radix kernel
+    int direct;
     int skip;         // SM_HC2R: the rows within icut of N/2 are zero and not read (magdealias's band)
     int cross3;       // set by the launcher: the three jobs form one cross product (LD_CROSS3)
     // set by the launcher for lengths without a register-blocked plan: the
@@ -133,7 +137,7 @@ bool spectral_len_supported(int n);
 // the length has a register-blocked plan
 bool spectral_len_fixed(int n);
 // run-time radix plan of an even length (false: odd or too long)
-bool generic_plan(int n, int radix[SPEC_GEN_MAX_PASSES], int* npass);
+bool generic_plan(int n, int radix[SPEC_GEN_MAX_PASSES], int* npass, bool direct = false);
 int launch_spectral_generic(const SpecLaunch& L, int compute_f32, hipStream_t s);
 // radix plans of the length: SpecLaunch::variant runs from 0 to this - 1
 int spectral_variants(int n);

@@ -159,7 +159,7 @@ __device__ __forceinline__ cpx<TC>* gen_fft(cpx<TC>* a, cpx<TC>* b, const cpx<TC
     int Ns = 1;
     for (int p = 0; p < L.gen_npass; ++p) {
         const int R = L.gen_radix[p];
-        switch (R) {
+        switch (L.direct ? 0 : R) {
         case 2: gen_pass_r<TC, 2, INV>(a, b, tw, N, nlb, Ns); break;
         case 3: gen_pass_r<TC, 3, INV>(a, b, tw, N, nlb, Ns); break;
         case 4: gen_pass_r<TC, 4, INV>(a, b, tw, N, nlb, Ns); break;
@@ -440,14 +440,15 @@ int gen_mode(const SpecLaunch& L, hipStream_t s)
 
 }  // namespace
 
-bool generic_plan(int n, int radix[SPEC_GEN_MAX_PASSES], int* npass)
+bool generic_plan(int n, int radix[SPEC_GEN_MAX_PASSES], int* npass, bool direct)
 {
     if (n < 2 || n % 2 || n > SPEC_GEN_MAX_N) return false;
     int p = 0, m = n;
-    // one 8 where the power of two is odd and at least 8, then 4s
+    // one 8 where the power of two is odd and at least 8 (point by point: only
+    // 4s and a 2), then 4s
     int e2 = 0;
     while (m % (2 << e2) == 0) ++e2;
-    if (e2 >= 3 && e2 % 2) { radix[p++] = 8; m /= 8; }
+    if (!direct && e2 >= 3 && e2 % 2) { radix[p++] = 8; m /= 8; }
     while (m % 4 == 0 && p < SPEC_GEN_MAX_PASSES) { radix[p++] = 4; m /= 4; }
     for (int f = 2; m > 1 && p < SPEC_GEN_MAX_PASSES; ++f)
         while (m % f == 0 && p < SPEC_GEN_MAX_PASSES) { radix[p++] = f; m /= f; }
@@ -459,7 +460,7 @@ int launch_spectral_generic(const SpecLaunch& L0, int f32, hipStream_t s)
 {
     SpecLaunch L = L0;
     const int N = L.dir == 0 ? L.g.nx : L.g.ny;
-    if (!generic_plan(N, L.gen_radix, &L.gen_npass)) return -20;
+    if (!generic_plan(N, L.gen_radix, &L.gen_npass, L.direct != 0)) return -20;
     // lines per workgroup: about 1024 points, at most 64 KB of LDS where one
     // line fits in that
     const size_t csz = f32 ? sizeof(cpx<float>) : sizeof(cpx<double>);
