@@ -17,7 +17,7 @@ energy) are reported under "mixed".
 Prints one JSON line.  The roofline object covers the dominant kernel family,
 hydro_col (the whole hydrodynamic right-hand side after the x/y transform
 passes, with the fused AB3 update of u, v, w, rho, T: 47 arrays per cell in
-FP64, 268 bytes per cell in the mixed mode), timed with HIP events on the
+FP64, 300 bytes per cell in the mixed mode), timed with HIP events on the
 solver's stream over the timed steps; roofline_xderiv2 does the same for the
 x-direction first+second derivative pass of T, u, v, w (with the Maxwell
 stresses and d/dx of rho in the same launch) over a few further steps.  step_roofline puts
@@ -470,15 +470,16 @@ def measured_traffic(precision, kernel):
 # algorithmic bytes per cell of one launch of each timed kernel family
 #  xderiv2: reads T, u, v, w, rho and the three field components, writes both
 #           outputs of T, u, v, w and the first derivative of rho, working
-#           precision: 17 arrays
-#  yderiv2: the same along y, reading d/dx u and d/dx v too: 19 arrays
+#           precision: 17 arrays; mixed also the three stresses' derivatives: 20
+#  yderiv2: the same along y, reading d/dx u and d/dx v too: 19 arrays; mixed also
+#           the three stresses' derivatives and d/dy of d/dx u, d/dx v: 24
 #  hydro:   hydro_col with the fused AB3 update (interior and wall planes, one launch):
-#           reads the state (5), B and J^2 (4), the 18 x/y derivative arrays and
+#           reads the state (5), B and J^2 (4), the 18 (mixed 26) x/y derivative arrays and
 #           history levels 1, 2 of 5 fields; writes 5 RHS and the 5 new state
 #           fields.  FP64: 47 x 8 = 376 B.  Mixed: FP32 state shadows, B, J^2,
 #           derivatives and history, plus the FP64 state read and written and
-#           the new FP32 shadows: 4 (5 + 4 + 18 + 10 + 5 + 5) + 8 (5 + 5) = 268 B.
-KERNEL_BYTES_PER_CELL = {"xderiv2": {8: 136, 4: 68}, "yderiv2": {8: 152, 4: 76}, "hydro": {8: 376, 4: 268}}
+#           the new FP32 shadows: 4 (5 + 4 + 26 + 10 + 5 + 5) + 8 (5 + 5) = 300 B.
+KERNEL_BYTES_PER_CELL = {"xderiv2": {8: 136, 4: 80}, "yderiv2": {8: 152, 4: 96}, "hydro": {8: 376, 4: 300}}
 KERNEL_DESC = {"xderiv2": "SpecK<T, plan, 0, 2, 1, 0> (xderiv2: d/dx and d2/dx2 of T, u, v, w with the x "
                           "derivatives of the Maxwell stresses; d/dx of rho)",
                "yderiv2": "SpecK<T, plan, 1, B, 1, 0> (yderiv2: the same along y, with d/dy of d/dx u, d/dx v)",

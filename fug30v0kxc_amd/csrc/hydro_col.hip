@@ -21,8 +21,9 @@
 // with divu = ux + vy + d1bydz(w, 1).  The d/dx d/dx u and d/dy d/dy v parts
 // ride in the x / y passes' second outputs (MUL_D2C), since they differ from
 // d2bydx / d2bydy at the Nyquist mode, and so do dxm, dym, the other Maxwell
-// stresses and the mixed derivatives (the passes' auxiliary lines): each
-// momentum equation reads one array per horizontal direction (uxs .. wys).
+// stresses and the mixed derivatives (the passes' auxiliary lines): in FP64 each
+// momentum equation reads one array per horizontal direction (uxs .. wys), in the
+// mixed mode their FP32 terms one by one (xbb .. vxy), added here in FP64.
 #include <type_traits>
 
 #include "launch.hpp"
@@ -149,6 +150,10 @@ __device__ __forceinline__ void HydroColKernel<TW, MIX, PART>::body(const HydroC
             tdot = tdot + p.sckg * (w1 + w2) * (w1 + w2);
         }
         // 245-261
+        if constexpr (MIX) {
+            udot = udot + at(a.ybb, q);
+            vdot = vdot + at(a.xbb, q);
+        }
         {
             const double w3 = d.wx, w4 = d.uzu;
             udot = udot - rr * w0 * w4;
@@ -157,6 +162,7 @@ __device__ __forceinline__ void HydroColKernel<TW, MIX, PART>::body(const HydroC
         }
         // 287-309
         udot = udot + d.zzx;
+        if constexpr (MIX) wdot = wdot + at(a.xzx, q);
         wdot = wdot + p.thmplus1 * rr;
         {
             const double w1 = d.wy, w2 = d.vzu;
@@ -169,18 +175,30 @@ __device__ __forceinline__ void HydroColKernel<TW, MIX, PART>::body(const HydroC
         wdot = wdot - rr * p.cor * (-u0 * p.cpsi);
         // 331-338
         vdot = vdot + d.zzy;
+        if constexpr (MIX) wdot = wdot + at(a.yzy, q);
         // 360-432, 181-184, 230-338: the horizontal viscous and Maxwell stresses
         // and the composite fluxes' horizontal parts
         udot = udot + p.sck * d.uzz;
         vdot = vdot + p.sck * d.vzz;
-        udot = udot + at(a.uxs, q);
-        vdot = vdot + at(a.vxs, q);
-        wdot = wdot + at(a.wxs, q);
-        udot = udot + at(a.uys, q);
-        vdot = vdot + at(a.vys, q);
-        wdot = wdot + at(a.wys, q);
-        udot = udot + scko3 * d.dzwx;
-        vdot = vdot + scko3 * d.dzwy;
+        if constexpr (MIX) {
+            udot = udot + at(a.uxs, q);
+            vdot = vdot + p.sck * at(a.vxs, q);
+            wdot = wdot + p.sck * at(a.wxs, q);
+            udot = udot + p.sck * at(a.uys, q);
+            vdot = vdot + at(a.vys, q);
+            wdot = wdot + p.sck * at(a.wys, q);
+            udot = udot + (scko3 * (at(a.vxy, q) + d.dzwx) + at(a.dxm, q));
+            vdot = vdot + (scko3 * (at(a.uxy, q) + d.dzwy) + at(a.dym, q));
+        } else {
+            udot = udot + at(a.uxs, q);
+            vdot = vdot + at(a.vxs, q);
+            wdot = wdot + at(a.wxs, q);
+            udot = udot + at(a.uys, q);
+            vdot = vdot + at(a.vys, q);
+            wdot = wdot + at(a.wys, q);
+            udot = udot + scko3 * d.dzwx;
+            vdot = vdot + scko3 * d.dzwy;
+        }
         wdot = wdot + d.c3 + d.c4;
         // 455-470: d(rho)/dz on the walls from dw/dt = 0
         double rzu = d.rzu, rzc = d.rzc;

@@ -50,7 +50,10 @@ namespace {
 enum Wk {
     W_RX, W_TX, W_TXX, W_UX, W_UXS, W_VX, W_VXS, W_WX, W_WXS,
     W_RY, W_TY, W_TYY, W_UY, W_UYS, W_VY, W_VYS, W_WY, W_WYS,
-    W_COUNT
+    // mixed mode only
+    W_XBB, W_XZX, W_DXM, W_YBB, W_YZY, W_DYM, W_UXY, W_VXY,
+    W_COUNT,
+    W_COUNT_FP64 = W_XBB
 };
 
 constexpr int MAXEV = 8192;
@@ -384,6 +387,9 @@ HydroColArgs colargs(mhd_ctx* c)
     a.vx = W[W_VX]; a.vxs = W[W_VXS]; a.wx = W[W_WX]; a.wxs = W[W_WXS];
     a.ry = W[W_RY]; a.ty = W[W_TY]; a.tyy = W[W_TYY]; a.uy = W[W_UY]; a.uys = W[W_UYS];
     a.vy = W[W_VY]; a.vys = W[W_VYS]; a.wy = W[W_WY]; a.wys = W[W_WYS];
+    a.xbb = W[W_XBB]; a.xzx = W[W_XZX]; a.dxm = W[W_DXM];
+    a.ybb = W[W_YBB]; a.yzy = W[W_YZY]; a.dym = W[W_DYM];
+    a.uxy = W[W_UXY]; a.vxy = W[W_VXY];
     a.rdot = level_ptr(c, 3, 3);
     a.tdot = level_ptr(c, 4, 3);
     a.udot = level_ptr(c, 0, 3);
@@ -487,44 +493,56 @@ int run_hydro_deriv(mhd_ctx* c, const double* cf = nullptr)
         L.bf[0] = c->bx; L.bf[1] = c->by; L.bf[2] = c->bz;
         if (mx) { L.bmean[0] = c->bxbar; L.bmean[1] = c->bybar; L.bmean[2] = c->bzm; }
     };
-    auto stress = [](SpecJob& j, double c2, double c11, int op, int ai, int aj, double scale) {
+    // (own: the mixed mode's array of the stress alone, AuxOp)
+    auto stress = [&](SpecJob& j, double c2, double c11, int op, int ai, int aj, double scale, int own) {
         j.mc[0] = c2; j.mc[1] = c11;
         j.aux = op; j.ai = ai; j.aj = aj; j.ascale = scale;
+        if (mx) {
+            j.out[2] = W[own];
+            if (c11 == 0.0) j.mul[1] = MUL_D2;   // sck is applied in FP64 by the column kernel
+        }
     };
     enum { BX = 0, BY = 1, BZ = 2 };
     // x pass: d/dx of u, v, w, t, r; the second outputs (HydroColArgs) hold
     // sck d2/dx2 with u's scko3 d/dx d/dx u of the composite flux (lines 181,
-    // 258) and d/dx of F/2 (bx^2-by^2-bz^2), F by bx, F bz bx
+    // 258) and, in FP64, d/dx of F/2 (bx^2-by^2-bz^2), F by bx, F bz bx
     {
         SpecLaunch L = spec_base(c, 0, SM_DERIV2);
         with_b(L);
         L.job[0] = sjob(U_, sf, W[W_UX], W[W_UXS], MUL_D1, MUL_D2C, wf);
-        stress(L.job[0], P.sck, P.scko3, AUX_MAXW, BX, 0, P.fo2);
+        stress(L.job[0], P.sck, P.scko3, AUX_MAXW, BX, 0, P.fo2, W_DXM);
         L.job[1] = sjob(V_, sf, W[W_VX], W[W_VXS], MUL_D1, MUL_D2C, wf);
-        stress(L.job[1], P.sck, 0.0, AUX_PROD, BY, BX, f);
+        stress(L.job[1], P.sck, 0.0, AUX_PROD, BY, BX, f, W_XBB);
         L.job[2] = sjob(W_, sf, W[W_WX], W[W_WXS], MUL_D1, MUL_D2C, wf);
-        stress(L.job[2], P.sck, 0.0, AUX_PROD, BZ, BX, f);
+        stress(L.job[2], P.sck, 0.0, AUX_PROD, BZ, BX, f, W_XZX);
         L.job[3] = sjob(T_, sf, W[W_TX], W[W_TXX], MUL_D1, MUL_D2, wf);
         L.job[4] = sjob(R_, sf, W[W_RX], nullptr, MUL_D1, 0, wf);
         L.njobs = 5;
         TRY(spec(c, L, MHD_K_XDERIV2));
     }
     // y pass: the same along y (v's second output carries scko3 d/dy d/dy v),
-    // with d/dy of scko3 vx and scko3 ux of the composite fluxes
+    // with d/dy of scko3 vx and scko3 ux of the composite fluxes, in the mixed
+    // mode d/dy of vx and ux as jobs of their own
     {
         SpecLaunch L = spec_base(c, 1, SM_DERIV2);
         with_b(L);
         L.job[0] = sjob(U_, sf, W[W_UY], W[W_UYS], MUL_D1, MUL_D2C, wf);
-        stress(L.job[0], P.sck, 0.0, AUX_PROD, BY, BX, f);
-        L.job[0].xin = W[W_VX]; L.job[0].xcoef = P.scko3;
+        stress(L.job[0], P.sck, 0.0, AUX_PROD, BY, BX, f, W_YBB);
         L.job[1] = sjob(V_, sf, W[W_VY], W[W_VYS], MUL_D1, MUL_D2C, wf);
-        stress(L.job[1], P.sck, P.scko3, AUX_MAXW, BY, 0, P.fo2);
-        L.job[1].xin = W[W_UX]; L.job[1].xcoef = P.scko3;
+        stress(L.job[1], P.sck, P.scko3, AUX_MAXW, BY, 0, P.fo2, W_DYM);
         L.job[2] = sjob(W_, sf, W[W_WY], W[W_WYS], MUL_D1, MUL_D2C, wf);
-        stress(L.job[2], P.sck, 0.0, AUX_PROD, BZ, BY, f);
+        stress(L.job[2], P.sck, 0.0, AUX_PROD, BZ, BY, f, W_YZY);
         L.job[3] = sjob(T_, sf, W[W_TY], W[W_TYY], MUL_D1, MUL_D2, wf);
         L.job[4] = sjob(R_, sf, W[W_RY], nullptr, MUL_D1, 0, wf);
         L.njobs = 5;
+        if (mx) {
+            L.job[5] = sjob(W[W_UX], wf, W[W_UXY], nullptr, MUL_D1, 0, wf);
+            L.job[6] = sjob(W[W_VX], wf, W[W_VXY], nullptr, MUL_D1, 0, wf);
+            L.njobs = 7;
+        } else {
+            L.job[0].xin = W[W_VX]; L.job[0].xcoef = P.scko3;
+            L.job[1].xin = W[W_UX]; L.job[1].xcoef = P.scko3;
+        }
         TRY(spec(c, L, MHD_K_YDERIV2));
     }
     HydroColArgs a = colargs(c);
@@ -590,6 +608,7 @@ MagSpecArgs mag_spec_args(mhd_ctx* c, const MagArgs& m)
     a.cc = m.cc; a.d = m.d;
     a.pol = c->pol; a.tor = c->tor; a.polz = m.polz;
     a.out[0] = m.bxh; a.out[1] = m.byh; a.out[2] = m.jzh; a.out[3] = m.bzh; a.out[4] = m.dxbzh;
+    a.out[5] = m.dybzh;
     return a;
 }
 
@@ -731,11 +750,11 @@ int run_bandj(mhd_ctx* c, bool clean)
     x.skip = clean;
     TRY(kerr(launch_bandj_x(x, wf, c->s)));
     // 575-593: y transforms and the mean parts of B (the mixed path keeps B
-    // without its means: no additions); dBz/dy rides with Bz
+    // without its means: no additions); dBz/dy rides with Bz in FP64
     const bool mx = c->su != nullptr;
     SpecLaunch M = spec_base(c, 1, SM_HC2R);
     M.skip = clean;
-    M.job[0] = sjob(m.bzh, wf, c->bz, m.dybzh, 0, MUL_D1, wf);
+    M.job[0] = sjob(m.bzh, wf, c->bz, mx ? nullptr : m.dybzh, 0, MUL_D1, wf);
     M.job[0].adds = mx ? 0.0 : c->sc.bzbar;
     M.job[1] = sjob(m.bxh, wf, c->bx, nullptr, 0, 0, wf);
     M.job[1].addk = mx ? nullptr : c->bxbar;
@@ -744,6 +763,7 @@ int run_bandj(mhd_ctx* c, bool clean)
     M.job[3] = sjob(m.dxbzh, wf, m.dxbzh, nullptr, 0, 0, wf);
     M.job[4] = sjob(m.jzh, wf, m.jzh, nullptr, 0, 0, wf);
     M.njobs = 5;
+    if (mx) M.job[M.njobs++] = sjob(m.dybzh, wf, m.dybzh, nullptr, 0, 0, wf);
     TRY(spec(c, M));
     return kerr(launch_jsq(m, c->s));
 }
@@ -1121,7 +1141,8 @@ int mhd_create(const mhd_params_t* p, int nx, int ny, int nz, int precision, mhd
     bytes += 7 * f64 + 5 * fs;                        // state ping-pong (u v w t r pol tor)
     c->eta_on = p->eta_c > 1.0;
     bytes += 2 * vz + (c->eta_on ? 3 * fw : 0);       // eta(z) profile, J
-    bytes += W_COUNT * fw;                            // work
+    const int nwk = c->wf32 ? W_COUNT : W_COUNT_FP64;
+    bytes += nwk * fw;                                // work
     bytes += al256(nz * (RED_CHUNKS + 1) * 8 * sizeof(double)) + 2 * al256(8 * sizeof(double));  // reductions
     if (hipMalloc((void**)&c->pool, bytes) != hipSuccess) {
         (void)hipStreamDestroy(c->s);
@@ -1161,7 +1182,7 @@ int mhd_create(const mhd_params_t* p, int nx, int ny, int nz, int precision, mhd
         for (int l = 0; l < 3; ++l) c->hist[f][l] = take(fh);
     for (int f = 0; f < 2; ++f)
         for (int l = 0; l < 3; ++l) c->mhist[f][l] = (double*)take(vz);
-    for (int i = 0; i < W_COUNT; ++i) c->wk[i] = take(fw);
+    for (int i = 0; i < nwk; ++i) c->wk[i] = take(fw);
     c->red_partial = (double*)take(al256(nz * (RED_CHUNKS + 1) * 8 * sizeof(double)));
     c->red_result = (double*)take(al256(8 * sizeof(double)));
     c->d_bzbar = (double*)take(al256(8 * sizeof(double)));
@@ -1938,10 +1959,20 @@ int mhd_autotune(mhd_ctx_t* c, mhd_tune_t* out)
                 L.job[j].ai = j;
                 L.job[j].aj = 0;
                 L.job[j].ascale = 1.0;
-                if (dir == 1 && j < 2) L.job[j].xin = in[0];
+                if (c->su) {
+                    static const int o3[2][3] = {{W_XBB, W_XZX, W_DXM}, {W_YBB, W_YZY, W_DYM}};
+                    L.job[j].out[2] = W[o3[dir][j]];
+                } else if (dir == 1 && j < 2) {
+                    L.job[j].xin = in[0];
+                }
             }
             L.job[4] = sjob(in[0], sf, W[dir == 0 ? W_RX : W_RY], nullptr, MUL_D1, 0, wf);
             L.njobs = 5;
+            if (c->su && dir == 1) {
+                L.job[5] = sjob(in[1], sf, W[W_UXY], nullptr, MUL_D1, 0, wf);
+                L.job[6] = sjob(in[2], sf, W[W_VXY], nullptr, MUL_D1, 0, wf);
+                L.njobs = 7;
+            }
         }
         return L;
     };

@@ -59,7 +59,7 @@ struct HydroColArgs {
     double bzm;                         // mixed: Bz-bar
     const double *kappa, *dkappa;
     const double* etar;                 // eta(z)/eta_0 for the Ohmic heating, or null (1)
-    // x pass: d/dx of r, t, u, v, w, d2/dx2 of t, and the x parts of the
+    // x pass: d/dx of r, t, u, v, w, d2/dx2 of t, and in FP64 the x parts of the
     // momentum equations' viscous and Maxwell stresses
     //   uxs = sck*uxx + scko3*d/dx(d/dx u) + d/dx(F/2 (bx^2 - by^2 - bz^2))
     //   vxs = sck*vxx + d/dx(F by bx), wxs = sck*wxx + d/dx(F bz bx)
@@ -69,6 +69,12 @@ struct HydroColArgs {
     //   vys = sck*vyy + scko3*d/dy(d/dy v) + d/dy(scko3 ux + F/2 (by^2 - bx^2 - bz^2))
     //   wys = sck*wyy + d/dy(F bz by)
     const void *ry, *ty, *tyy, *uy, *uys, *vy, *vys, *wy, *wys;
+    // FP32 arrays hold the terms one by one, added in FP64 here: uxs = sck*uxx +
+    // scko3*d/dx(d/dx u), vxs = vxx, wxs = wxx, uys = uyy, vys = sck*vyy +
+    // scko3*d/dy(d/dy v), wys = wyy, the Maxwell stresses xbb = d/dx(F by bx),
+    // xzx = d/dx(F bz bx), dxm = d/dx(F/2 (bx^2 - by^2 - bz^2)), the same along y,
+    // and uxy = d/dy(ux), vxy = d/dy(vx)
+    const void *xbb, *xzx, *dxm, *ybb, *yzy, *dym, *uxy, *vxy;
     void *rdot, *tdot, *udot, *vdot, *wdot;   // newest history level (working precision)
     int zc;                             // planes per thread
     // fused AB3 update of u v w r t (src/main.F90:413-443); ab3 = 0: RHS only.

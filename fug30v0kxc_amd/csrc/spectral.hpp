@@ -23,14 +23,17 @@ enum LoadOp { LD_PLAIN = 0, LD_CROSS = 1,
               // {a_{q+1}, b_{q+2}, a_{q+2}, b_{q+1}} (indices mod 3); the six
               // factor lines of a line group are loaded once for all three
               LD_CROSS3 = 2 };
-// A second-derivative job may carry a second, auxiliary line a whose first
-// derivative joins its second output, out[1] = mul[1](in) + d1(a):
+// A second-derivative job may carry a second, auxiliary line a:
 //   AUX_PROD  a = ascale*(b_i+m_i)*(b_j+m_j) + xcoef*xin     (i, j = ai, aj)
 //   AUX_MAXW  a = ascale*((b_i+m_i)^2 - (b_j+m_j)^2 - (b_l+m_l)^2) + xcoef*xin
-// with b the launch's three field components (SpecLaunch::bf, bmean).  The
-// multipliers are linear, so the Maxwell stress and the composite viscous flux
-// of a momentum component need no transform back, store and re-read of their
-// own: one inverse transform returns the sum.
+// with b the launch's three field components (SpecLaunch::bf, bmean).
+// FP64: its first derivative joins the second output, out[1] = mul[1](in) +
+// d1(a).  The multipliers are linear, so the Maxwell stress and the composite
+// viscous flux of a momentum component need no transform back, store and re-read
+// of their own: one inverse transform returns the sum.
+// FP32: it is an output of its own, out[2] = d1(a), and there is no xin.  The
+// column kernel adds the stresses in FP64; summed in FP32 spectra, a small viscous
+// term next to large stresses that cancel in the equation would be rounded away.
 enum AuxOp { AUX_NONE = 0, AUX_PROD = 1, AUX_MAXW = 2 };
 
 constexpr int SPEC_MAX_JOBS = 8;
@@ -54,12 +57,13 @@ struct SpecJob {
     int aux;          // AuxOp (SM_DERIV2 with out[1])
     int ai, aj;       // its field components
     double ascale;
-    const void* xin;  // its further term xcoef * xin, or null
+    const void* xin;  // FP64: its further term xcoef * xin, or null
     double xcoef;
-    // SM_DERIV2: out[1] may be null (the job's first derivative only).
-    // SM_HC2R: out[1], when set, takes mul[1] of the same line (d/dx or d/dy of
-    // the output, from the spectrum in registers)
-    void* out[2];
+    // SM_DERIV2: out[1] may be null (the job's first derivative only); out[2] see
+    // AuxOp.
+    // SM_HC2R in FP64: out[1], when set, takes mul[1] of the same line (d/dx or
+    // d/dy of the output, from the spectrum in registers)
+    void* out[3];
     int out_f32;
     int mul[2];       // MulKind for out[0], out[1] (SM_DERIV*)
     const double* addk; // optional per-plane value added on store (nz entries)
@@ -111,7 +115,9 @@ struct MagSpecArgs {
     void *cc, *d;
     const double *pol, *tor; // bandj_x
     const void* polz;
-    void* out[5];            // Bx, By, Jz, Bz, dBz/dx
+    // Bx, By, Jz, Bz, dBz/dx; FP32 also dBz/dy, so that both derivatives come from
+    // the FP64 spectrum of pol (FP64 takes it from Bz's spectrum in the y pass)
+    void* out[6];
 };
 // register-blocked lengths nx only (spectral_len_fixed), else -20
 int launch_emf_x(const MagSpecArgs& a, int f32, hipStream_t s);

@@ -341,13 +341,16 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
                     out0[ib + n * st] = bb;
                 }
             } else {
-                constexpr int NOUT = (MODE == SM_DERIV2) ? 2 : 1;
+                constexpr bool SUM = sizeof(TC) == 8;   // AuxOp
+                constexpr int NOUT = (MODE == SM_DERIV2) ? (SUM ? 2 : 3) : 1;
                 for (int o = 0; o < NOUT; ++o) {
-                    if (o == 1 && out1 == nullptr) break;   // a first-derivative job (uniform)
+                    // a first-derivative job, a job without an auxiliary line (uniform)
+                    if (o == 1 && out1 == nullptr) break;
+                    if (o == 2 && !J.aux) break;
                     cpx<TC>* aux = nullptr;
                     // a job with one output needs no third buffer
                     cpx<TC>* work = out1 ? buf2 : spec;
-                    if (o == 1 && J.aux) {
+                    if (o == (SUM ? 1 : 2) && J.aux) {
                         // the auxiliary line's spectrum
                         for (int q = threadIdx.x; q < P; q += GNT) {
                             int b, n;
@@ -360,7 +363,7 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
                                 const TC* __restrict__ p0 = (const TC*)L.bf[al.ai];
                                 const TC* __restrict__ p1 = (const TC*)L.bf[al.aj];
                                 const TC* __restrict__ p2 = (const TC*)L.bf[al.al];
-                                const TC* __restrict__ px = (const TC*)J.xin;
+                                const TC* __restrict__ px = SUM ? (const TC*)J.xin : nullptr;
                                 const long i = ia + n * st, e = ib + n * st;
                                 const bool mw = J.aux == AUX_MAXW;
                                 v = {al.one(p0[i], p1[i], mw ? p2[i] : (TC)0, px ? px[i] : (TC)0),
@@ -376,13 +379,17 @@ __device__ __forceinline__ void GenK<TC, DIR, MODE, LOP>::body(const SpecLaunch&
                     cpx<TC>* dst = aux ? aux : other;
                     for (int q = threadIdx.x; q < P; q += GNT) {
                         const int kk = q - fdiv(q, iN) * N;
-                        cpx<TC> m = apply_mul_rt<TC>(J.mul[o], spec[q], kk, N, L.cx, L.icut, J.mc);
-                        if (aux) m = cadd(m, apply_mul_rt<TC>(MUL_D1, aux[q], kk, N, L.cx, L.icut, J.mc));
+                        cpx<TC> m = o == 2 ? cpx<TC>{(TC)0, (TC)0}
+                                           : apply_mul_rt<TC>(J.mul[o == 0 ? 0 : 1], spec[q], kk, N, L.cx, L.icut, J.mc);
+                        if (aux) {
+                            const cpx<TC> d = apply_mul_rt<TC>(MUL_D1, aux[q], kk, N, L.cx, L.icut, J.mc);
+                            m = o == 2 ? d : cadd(m, d);
+                        }
                         dst[q] = m;
                     }
                     __syncthreads();
                     const cpx<TC>* res = gen_fft<TC, true>(dst, work, twl, L, N, nlb);
-                    store(res, o == 0 ? out0 : out1, (TC)1);
+                    store(res, (TC*)J.out[o], (TC)1);
                     __syncthreads();   // the buffers are reused by the next output
                 }
             }

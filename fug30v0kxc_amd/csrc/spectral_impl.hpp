@@ -138,10 +138,10 @@ struct AuxLoad {
     {
         op = J.aux;
         ai = op ? J.ai : 0;
-        aj = op == AUX_PROD ? J.aj : (ai + 1) % 3;
+        aj = op == AUX_PROD ? J.aj : (ai == 0 ? 1 : 0);
         al = 3 - ai - aj;
         s = (TC)J.ascale;
-        xin = op && J.xin;
+        xin = sizeof(TC) == 8 && op && J.xin;
         xc = (TC)J.xcoef;
         mi = ml = mj = (TC)0;
         if (!op) return;
@@ -461,10 +461,12 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_deriv2(co
             }
         }
     };
-    cpx<TC> f[R0], x[R0], b0[R0], b1[R0], b2[R0];
+    constexpr bool SUM = sizeof(TC) == 8;   // AuxOp
+    cpx<TC> f[R0], x[SUM ? R0 : 1], b0[R0], b1[R0], b2[R0];
     auto load_job = [&](int q, long grp) {
         load((const TC*)L.job[q].in[0], grp, f);
-        if (L.job[q].xin) load((const TC*)L.job[q].xin, grp, x);
+        if constexpr (SUM)
+            if (L.job[q].xin) load((const TC*)L.job[q].xin, grp, x);
     };
     auto load_b = [&](long grp) {
         load((const TC*)L.bf[0], grp, b0);
@@ -499,8 +501,9 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_deriv2(co
                 const AuxLoad<TC> al(L, J, ok ? k : 0);
 #pragma unroll
                 for (int r = 0; r < R0; ++r) {
-                    a[r].x = al.pick(b0[r].x, b1[r].x, b2[r].x, x[r].x);
-                    a[r].y = al.pick(b0[r].y, b1[r].y, b2[r].y, x[r].y);
+                    const cpx<TC> q_ = SUM ? x[SUM ? r : 0] : cpx<TC>{(TC)0, (TC)0};
+                    a[r].x = al.pick(b0[r].x, b1[r].x, b2[r].x, q_.x);
+                    a[r].y = al.pick(b0[r].y, b1[r].y, b2[r].y, q_.y);
                 }
             }
             if (q + 1 < q1) load_job(q + 1, grp);
@@ -513,24 +516,29 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_deriv2(co
             cpx<TC> z[RL], w[RL];
 #pragma unroll
             for (int r = 0; r < RL; ++r) z[r] = v[r];
-            if (J.aux) {
+            // the auxiliary line's spectrum
+            auto aux_to = [&](cpx<TC>* d) {
 #pragma unroll
                 for (int r = 0; r < R0; ++r) v[r] = a[r];
                 F::forward(v, j, lds, twl);
 #pragma unroll
-                for (int r = 0; r < RL; ++r) w[r] = v[r];
-            }
-            auto second = [&](int r) {
-                const int kk = j + r * NBL;
-                const cpx<TC> d2 = apply_mul<TC, N>(J.mul[1], z[r], kk, cx, icut, J.mc);
-                return J.aux ? cadd(d2, apply_mul<TC, N>(MUL_D1, w[r], kk, cx, icut, J.mc)) : d2;
+                for (int r = 0; r < RL; ++r) d[r] = v[r];
             };
-            for (int o = 0; o < 2; ++o) {
-                if (o == 1 && !J.out[1]) break;   // a first-derivative job (uniform)
+            if (SUM && J.aux) aux_to(w);
+            for (int o = 0; o < (SUM ? 2 : 3); ++o) {
+                // a first-derivative job, a job without an auxiliary line (uniform)
+                if (o == 1 && !J.out[1]) break;
+                if (o == 2) {
+                    if (!J.aux) break;
+                    aux_to(z);
+                }
+                const int mul = o == 2 ? (int)MUL_D1 : J.mul[o == 0 ? 0 : 1];
 #pragma unroll
                 for (int r = 0; r < RL; ++r) {
-                    if (o == 0) v[r] = apply_mul<TC, N>(J.mul[0], z[r], j + r * NBL, cx, icut, J.mc);
-                    else v[r] = second(r);
+                    const int kk = j + r * NBL;
+                    v[r] = apply_mul<TC, N>(mul, z[r], kk, cx, icut, J.mc);
+                    if (SUM && o == 1 && J.aux)
+                        v[r] = cadd(v[r], apply_mul<TC, N>(MUL_D1, w[r], kk, cx, icut, J.mc));
                 }
                 F::inverse(v, j, lds, twl);
                 if (ok && j < NB0) {
@@ -686,7 +694,7 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_jobs(cons
                         }
                     }
                 }
-                if (o == 1 || !J.out[1]) break;
+                if (sizeof(TC) == 4 || o == 1 || !J.out[1]) break;
 #pragma unroll
                 for (int r = 0; r < RL; ++r)
                     v[r] = apply_mul<TC, N>(J.mul[1], z[r], j + r * NBL, cx, icut, J.mc);
@@ -783,6 +791,7 @@ static int launch_one(const SpecLaunch& L, hipStream_t s)
         for (int q = 0; q < L.njobs; ++q) {
             const SpecJob& J = L.job[q];
             if (!J.aux) continue;
+            if (sizeof(TC) == 4 && (!J.out[2] || J.xin)) return -23;
             if (!L.bf[0] || !L.bf[1] || !L.bf[2] || !J.out[1] || J.ai < 0 || J.ai > 2) return -23;
             if (J.aux == AUX_PROD && (J.aj < 0 || J.aj > 2 || J.aj == J.ai)) return -23;
         }

@@ -10,8 +10,8 @@
 //
 //   emf_x    forward: rows of E (physical x, halfcomplex y) -> the spectra
 //            C = dEx/dy - dEy/dx, D = dEx/dx + dEy/dy and Ez
-//   bandj_x  inverse: pol, tor and d pol/dz -> the rows of Bx, By, Bz, Jz and
-//            dBz/dx in physical x, halfcomplex y.  With `skip` the 2/3 band of
+//   bandj_x  inverse: pol, tor and d pol/dz -> the rows of Bx, By, Bz, Jz,
+//            dBz/dx and, in FP32, dBz/dy in physical x, halfcomplex y.  With `skip` the 2/3 band of
 //            pol and tor is known to be zero: its modes are not read, its rows
 //            neither transformed nor written (the y pass takes them as zero).
 //
@@ -297,13 +297,14 @@ struct BandjXK : MagBase<TC, PL, B> {
                 load((const TC*)a.polz, C, j, wz);
                 load(a.tor, C, j, wt);
             }
-            for (int o = 3; o < 5; ++o) {
+            for (int o = 3; o < (sizeof(TC) == 4 ? 6 : 5); ++o) {
                 cpx<TC> v[F::RMAX];
 #pragma unroll
                 for (int r = 0; r < RL; ++r) {
                     const double kx = M::kx1(j + r * NBL, a.cx);
+                    const double kd = o == 4 ? kx : ky;
                     if (o == 3) v[r] = {(TC)b[r].x, (TC)b[r].y};
-                    else v[r] = {(TC)(-kx * b[r].y), (TC)(kx * b[r].x)};
+                    else v[r] = {(TC)(-kd * b[r].y), (TC)(kd * b[r].x)};
                 }
                 finish(v, a.out[o]);
             }
