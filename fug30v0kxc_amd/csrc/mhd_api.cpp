@@ -109,6 +109,7 @@ struct mhd_ctx {
     int hzc;           // planes per thread of the column-walking hydro kernel
     int mzc;           // ... of the magnetic column kernels (mag_rhs, jsq)
     double* hbuf;      // pinned host staging (one field)
+    double* hred;      // behind it: the reductions' results, written by their kernel
     hipEvent_t xev[XFER_CHUNKS];   // its transfers' chunks
     int xev_created;
 
@@ -894,15 +895,17 @@ RedArgs rargs(mhd_ctx* c, int op)
     if (c->su) { a.bxm = c->bxbar; a.bym = c->bybar; a.bzm = c->sc.bzbar; }
     a.partial = c->red_partial;
     a.result = c->red_result;
-    a.host = c->hbuf;
+    a.host = c->hred;
     return a;
 }
 
 int fetch_result(mhd_ctx* c, double* out, int n)
 {
-    // the finishing kernel wrote them into the pinned buffer
+    // the finishing kernel wrote them behind the transfers' staging: a
+    // reduction nobody waits for (mhd_global_averages without `out`) may still
+    // be running when the host fills that
     MHD_HIP_CHECK(hipStreamSynchronize(c->s));
-    memcpy(out, c->hbuf, n * sizeof(double));
+    memcpy(out, c->hred, n * sizeof(double));
     return 0;
 }
 
@@ -1208,10 +1211,11 @@ int mhd_create(const mhd_params_t* p, int nx, int ny, int nz, int precision, mhd
         mhd_destroy(c);
         return MHD_E_ALLOC;
     }
-    if (hipHostMalloc((void**)&c->hbuf, (size_t)c->n3 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc((void**)&c->hbuf, ((size_t)c->n3 + 8) * sizeof(double), hipHostMallocDefault) != hipSuccess) {
         mhd_destroy(c);
         return MHD_E_ALLOC;
     }
+    c->hred = c->hbuf + c->n3;
 
     // tables
     std::vector<double> a1, a2, b1, b2, ka, dka, tw64;

@@ -144,7 +144,7 @@ int mhd_mag_init(mhd_ctx_t* ctx);      /* src/magnetic.f90:5-279 */
 int mhd_step(mhd_ctx_t* ctx, int nsteps, double dt_fixed, int ndu06, mhd_diag_t* last);
 
 /* diagnostics (src/utils.F90, src/dbydz.F90:4796-4925) */
-int mhd_global_averages(mhd_ctx_t* ctx, double out[4]); /* ubar, vbar, ke, me (unscaled); subtracts ubar/vbar */
+int mhd_global_averages(mhd_ctx_t* ctx, double out[4]); /* ubar, vbar, ke, me (unscaled; out may be NULL); subtracts ubar/vbar */
 int mhd_nusselt(mhd_ctx_t* ctx, double* nu);
 int mhd_checkdivb(mhd_ctx_t* ctx, double out[2]);       /* divbmax, divbmin */
 int mhd_sminmax(mhd_ctx_t* ctx, int field_id, double out[2]); /* min, max */
