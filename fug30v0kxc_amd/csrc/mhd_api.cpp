@@ -1582,7 +1582,7 @@ int mhd_step(mhd_ctx_t* c, int nsteps, double dt_fixed, int ndu06, mhd_diag_t* l
             if (mag) TRY(run_mag_deriv(c, cf)); // reads the old u v w; + AB3 of pol, tor, magdealias
             TRY(run_ab3(c, cf, mag ? 7 : 5));  // swaps
         }
-        c->band_clean = 1;   // magdealias is part of either update
+        if (mag) c->band_clean = 1;   // magdealias is part of either update
         S.dt2 = dt + S.dt1;
         S.dt1 = dt;
         if (S.nit % 10 == 0) TRY(run_dealias5(c));
@@ -1664,12 +1664,14 @@ void ens_free(mhd_ensemble* e)
 // The kernel launches of ENS_BLOCK steps of one box, recorded instead of
 // issued.  The box's stream is put in capture mode meanwhile: any launch that
 // bypassed the recorder would land in that throwaway graph, and is reported
-// as MHD_E_STATE.  The host-side bookkeeping (driver scalars, history ring)
-// is put back afterwards; the state ping-pong swaps an even number of times.
+// as MHD_E_STATE.  The host-side bookkeeping (driver scalars, history ring,
+// and what is known of the 2/3 band) is put back afterwards; the state ping-pong
+// swaps an even number of times.
 int record_block(mhd_ctx* c, double dt, LaunchRecorder& rec)
 {
     const mhd_scalars_t keep = c->sc;
     const int ring[3] = {c->ring[0], c->ring[1], c->ring[2]};
+    const int clean = c->band_clean;
     MHD_HIP_CHECK(hipStreamBeginCapture(c->s, hipStreamCaptureModeRelaxed));
     launch_recorder() = &rec;
     const int rc = mhd_step(c, ENS_BLOCK, dt, 0, nullptr);
@@ -1683,6 +1685,7 @@ int record_block(mhd_ctx* c, double dt, LaunchRecorder& rec)
     }
     c->sc = keep;
     for (int l = 0; l < 3; ++l) c->ring[l] = ring[l];
+    c->band_clean = clean;
     if (rc) return rc;
     if (ce != hipSuccess) return MHD_E_DEVICE;
     return stray ? MHD_E_STATE : 0;
