@@ -118,7 +118,8 @@ static bool is_cross_product(const SpecLaunch& L)
 // which share their six factor loads (LD_CROSS3).
 int launch_spectral(const SpecLaunch& L, int compute_f32, hipStream_t s)
 {
-    if (L.njobs <= 0) return 0;
+    if (L.njobs == 0) return 0;
+    if (!spec_launch_ok(L, compute_f32)) return -23;
     if (L.mode == SM_R2HC && L.dir == 1 && spectral_len_fixed(L.g.ny) && is_cross_product(L)) {
         SpecLaunch G = L;
         G.cross3 = 1;

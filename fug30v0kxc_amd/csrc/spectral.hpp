@@ -134,7 +134,34 @@ struct ExpandArgs {
 };
 int launch_expand(const ExpandArgs& a, hipStream_t s);
 
-// Returns 0 or a negative code (-20: unsupported length).
+// What the kernels take for granted of a launch's jobs: an auxiliary line
+// (AuxOp) belongs to a second-derivative job with both outputs, in FP32 with its
+// own third output and no further term; it takes two different field components
+// out of three that are there (AuxLoad indexes bf and bmean by them); the jobs
+// that have one come first (body_deriv2 reloads the components during the
+// others).  The second output of an inverse transform is FP64 only.
+inline bool spec_launch_ok(const SpecLaunch& L, int f32)
+{
+    if (L.njobs < 0 || L.njobs > SPEC_MAX_JOBS) return false;
+    for (int q = 0; q < L.njobs; ++q) {
+        const SpecJob& J = L.job[q];
+        if (L.mode == SM_HC2R && f32 && J.out[1]) return false;
+        if (J.aux == AUX_NONE) continue;
+        if (L.mode != SM_DERIV2 || !J.out[1]) return false;
+        if (f32 && (!J.out[2] || J.xin)) return false;
+        if (!L.bf[0] || !L.bf[1] || !L.bf[2] || J.ai < 0 || J.ai > 2) return false;
+        if (J.aux == AUX_PROD) {
+            if (J.aj < 0 || J.aj > 2 || J.aj == J.ai) return false;
+        } else if (J.aux != AUX_MAXW) {
+            return false;
+        }
+        if (q > 0 && L.job[q - 1].aux == AUX_NONE) return false;
+    }
+    return true;
+}
+
+// Returns 0 or a negative code (-20: unsupported length, -23: jobs that
+// spec_launch_ok refuses).
 int launch_spectral(const SpecLaunch& L, int compute_f32, hipStream_t s);
 
 // every even length from 2 to SPEC_GEN_MAX_N: register-blocked kernels for

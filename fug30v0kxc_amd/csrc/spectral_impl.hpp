@@ -785,17 +785,7 @@ static int launch_one(const SpecLaunch& L, hipStream_t s)
     SpecLaunch La = L;
     // items: the (job, line group) pairs, or line groups whose jobs share loads;
     // second derivatives share them where the line groups alone fill the device
-    if (MODE == SM_DERIV2) {
-        La.split = L.njobs == 1 || ngrp < resident;
-        // two different field components, all three present
-        for (int q = 0; q < L.njobs; ++q) {
-            const SpecJob& J = L.job[q];
-            if (!J.aux) continue;
-            if (sizeof(TC) == 4 && (!J.out[2] || J.xin)) return -23;
-            if (!L.bf[0] || !L.bf[1] || !L.bf[2] || !J.out[1] || J.ai < 0 || J.ai > 2) return -23;
-            if (J.aux == AUX_PROD && (J.aj < 0 || J.aj > 2 || J.aj == J.ai)) return -23;
-        }
-    }
+    if (MODE == SM_DERIV2) La.split = L.njobs == 1 || ngrp < resident;
     const bool shared = LOP == LD_CROSS3 || (MODE == SM_DERIV2 && !La.split);
     long grid = ngrp * (shared ? 1 : L.njobs);
     if (L.ncu > 0 && grid > resident) grid = resident;
