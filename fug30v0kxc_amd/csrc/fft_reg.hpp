@@ -102,7 +102,8 @@ template <> struct AltPlan2<256> { using type = Plan<256, 16, 16>; };
 
 // Default plan of the second-derivative passes.  They keep six arrays of the
 // first radix's points and three of the last's in registers, so the radix 8 of
-// a length goes in the middle (at 512 points FP32: 187 registers with 4 4 4 8).
+// a length goes in the middle (at 512 points FP32: 187 registers with 4 4 4 8), and
+// at 480 and 640 points the 5 too (20 FP64 registers fewer than with the 5 last).
 template <int N, typename TC>
 struct D2Plan {
     using type = FftPlan<N>;
@@ -113,8 +114,9 @@ template <typename TC> struct D2Plan<128, TC> { using type = Plan<128, 4, 8, 4>;
 template <typename TC> struct D2Plan<160, TC> { using type = Plan<160, 4, 8, 5>; };
 template <typename TC> struct D2Plan<200, TC> { using type = Plan<200, 5, 8, 5>; };
 template <typename TC> struct D2Plan<216, TC> { using type = Plan<216, 3, 8, 3, 3>; };
-template <typename TC> struct D2Plan<480, TC> { using type = Plan<480, 4, 8, 3, 5>; };
+template <typename TC> struct D2Plan<480, TC> { using type = Plan<480, 4, 8, 5, 3>; };
 template <typename TC> struct D2Plan<512, TC> { using type = Plan<512, 4, 4, 8, 4>; };
+template <typename TC> struct D2Plan<640, TC> { using type = Plan<640, 4, 8, 5, 4>; };
 // FP32 passes of 512 points have the registers for three radix-8 passes, one LDS
 // exchange less (a step of 512^2 x 64 mixed, 4 4 8 4 -> 8 8 8: 3232 -> 3003 us
 // along y, -> 3198 along x; FP64 loses along y, 5235 -> 5306)

@@ -793,21 +793,44 @@ static int launch_one(const SpecLaunch& L, hipStream_t s)
     return mhd_launch<K>(dim3((unsigned)grid), dim3(NT), lds, s, La);
 }
 
-// (mode, load op) pairs the solver uses; every job of L has the same load op
+// (mode, load op) pairs the solver uses besides second derivatives and the EMF's
+// cross products; every job of L has the same load op
 template <typename TC, typename PL, int DIR, int B>
 static int launch_mode(const SpecLaunch& L, hipStream_t s)
 {
-    if constexpr (DIR != 0) {
-        if (L.cross3) return launch_one<TC, PL, DIR, B, SM_R2HC, LD_CROSS3>(L, s);
-    }
-    const int lop = L.job[0].load_op;
-    switch (L.mode * 8 + lop) {
+    switch (L.mode * 8 + L.job[0].load_op) {
     case SM_DERIV1 * 8 + LD_PLAIN: return launch_one<TC, PL, DIR, B, SM_DERIV1, LD_PLAIN>(L, s);
-    case SM_DERIV2 * 8 + LD_PLAIN: return launch_one<TC, PL, DIR, B, SM_DERIV2, LD_PLAIN>(L, s);
     case SM_R2HC * 8 + LD_PLAIN: return launch_one<TC, PL, DIR, B, SM_R2HC, LD_PLAIN>(L, s);
     case SM_HC2R * 8 + LD_PLAIN: return launch_one<TC, PL, DIR, B, SM_HC2R, LD_PLAIN>(L, s);
     }
     return -23;
+}
+
+// along y with groups of B column pairs, partly filled ones where B does not
+// divide a row's
+template <typename TC, typename PL, int B, int MODE, int LOP>
+static int launch_y(const SpecLaunch& L, hipStream_t s)
+{
+    return L.g.nx % (2 * B) == 0 ? launch_one<TC, PL, 1, B, MODE, LOP>(L, s) : launch_one<TC, PL, 2, B, MODE, LOP>(L, s);
+}
+
+// Second derivatives.  Half groups along y where a full one has 512 threads
+// (FP64) or 1024 (FP32), so that two or more workgroups share a CU (256 points: y
+// 449 against 458 us FP64, 246 against 241 FP32; 512 points FP32: 8 pairs spill).
+// In FP64 also where the full group is 4 pairs (480, 640, 768 and 1024 points,
+// 640 to 1024 threads): those spill 150 to 210 registers, 2 pairs and their 32-byte
+// row segments do not (y pass 1478 -> 645 us at 256 x 480 x 64, 1712 -> 872 at
+// 256 x 640 x 64, 1412 -> 763 at 256 x 768 x 48).  FP32 groups of 4 pairs stay: their
+// halves read 16 bytes a row (a step of 256 x 1024 x 48: 2.7 -> 4.2 ms).
+template <typename TC, typename PL>
+static int launch_d2(const SpecLaunch& L, hipStream_t s)
+{
+    if (L.job[0].load_op != LD_PLAIN) return -23;
+    if (L.dir == 0) return launch_one<TC, PL, 0, spec_b<TC, PL, 0>(), SM_DERIV2, LD_PLAIN>(L, s);
+    constexpr int B0 = spec_b<TC, PL, 1>();
+    constexpr int B2 = B0 >= (sizeof(TC) == 4 ? 8 : 4) && B0 * plan_tpt<PL>() >= (sizeof(TC) == 4 ? 1024 : 512)
+                           ? B0 / 2 : B0;
+    return launch_y<TC, PL, B2, SM_DERIV2, LD_PLAIN>(L, s);
 }
 
 template <typename TC, typename PL>
@@ -815,37 +838,34 @@ static int launch_plan(const SpecLaunch& L, hipStream_t s)
 {
     if (L.dir == 0) return launch_mode<TC, PL, 0, spec_b<TC, PL, 0>()>(L, s);
     constexpr int B0 = spec_b<TC, PL, 1>();
+    // the EMF's cross products: 3 lines and their 6 factors per thread, so half
+    // groups in FP64, also of 4 pairs above 512 threads (they spill)
+    constexpr int BC = sizeof(TC) == 8 && (B0 >= 8 || (B0 == 4 && B0 * plan_tpt<PL>() > 512)) ? B0 / 2 : B0;
+    if (L.cross3) return launch_y<TC, PL, BC, SM_R2HC, LD_CROSS3>(L, s);
     // FP32 only, where a full group would be a 1024-thread workgroup (one per
     // CU): at 256 points 8 pairs beat 16 for the first derivatives (76, 72, 45 us
     // against 81, 83, 48); in FP64 4 pairs lose to 8.  The other FP32 modes keep
     // 16 pairs (8 pairs: hc2r 125 against 109, r2hc 63 against 58)
     constexpr int BH = (sizeof(TC) == 4 && B0 >= 8 && B0 * plan_tpt<PL>() >= 1024) ? B0 / 2 : B0;
-    if (BH != B0 && L.mode == SM_DERIV1 && L.g.nx % (2 * BH) == 0) return launch_one<TC, PL, 1, BH, SM_DERIV1, LD_PLAIN>(L, s);
-    // second derivatives: half groups where a full one has 512 threads (FP64) or
-    // 1024 (FP32), so that two or more workgroups share a CU (256 points: y 449
-    // against 458 us FP64, 246 against 241 FP32; 512 points FP32: 8 pairs spill)
-    constexpr int B2 = B0 >= 8 && B0 * plan_tpt<PL>() >= (sizeof(TC) == 4 ? 1024 : 512) ? B0 / 2 : B0;
-    if (B2 != B0 && L.mode == SM_DERIV2 && L.g.nx % (2 * B2) == 0) return launch_one<TC, PL, 1, B2, SM_DERIV2, LD_PLAIN>(L, s);
-    // the EMF's cross products: 3 lines and their 6 factors per thread
-    constexpr int BC = sizeof(TC) == 8 && B0 >= 8 ? B0 / 2 : B0;
-    if (L.cross3 && L.g.nx % (2 * BC) == 0) return launch_one<TC, PL, 1, BC, SM_R2HC, LD_CROSS3>(L, s);
+    if (BH != B0 && L.mode == SM_DERIV1 && L.g.nx % (2 * BH) == 0)
+        return launch_one<TC, PL, 1, BH, SM_DERIV1, LD_PLAIN>(L, s);
     if (L.g.nx % (2 * B0) == 0) return launch_mode<TC, PL, 1, B0>(L, s);
-    if (B2 != B0 && L.mode == SM_DERIV2) return launch_one<TC, PL, 2, B2, SM_DERIV2, LD_PLAIN>(L, s);
-    if (BC != B0 && L.cross3) return launch_one<TC, PL, 2, BC, SM_R2HC, LD_CROSS3>(L, s);
     return launch_mode<TC, PL, 2, B0>(L, s);
 }
 
 template <typename TC, int N>
 static int launch_n(const SpecLaunch& L, hipStream_t s)
 {
+    const bool d2 = L.mode == SM_DERIV2;
     if constexpr (!std::is_void<typename AltPlan<N>::type>::value) {
-        if (L.variant == 1) return launch_plan<TC, typename AltPlan<N>::type>(L, s);
+        using PL = typename AltPlan<N>::type;
+        if (L.variant == 1) return d2 ? launch_d2<TC, PL>(L, s) : launch_plan<TC, PL>(L, s);
     }
     if constexpr (!std::is_void<typename AltPlan2<N>::type>::value) {
-        if (L.variant == 2) return launch_plan<TC, typename AltPlan2<N>::type>(L, s);
+        using PL = typename AltPlan2<N>::type;
+        if (L.variant == 2) return d2 ? launch_d2<TC, PL>(L, s) : launch_plan<TC, PL>(L, s);
     }
-    if (L.mode == SM_DERIV2) return launch_plan<TC, typename D2Plan<N, TC>::type>(L, s);
-    return launch_plan<TC, FftPlan<N>>(L, s);
+    return d2 ? launch_d2<TC, typename D2Plan<N, TC>::type>(L, s) : launch_plan<TC, FftPlan<N>>(L, s);
 }
 
 }  // namespace mhd
