@@ -469,12 +469,11 @@ void fuse_ab3(mhd_ctx* c, HydroColArgs& a, const double* cf, void* hz1, void* hz
     if (c->su) { a.t0 = c->t0; a.r0 = c->r0; }
 }
 
-int run_hydro_deriv(mhd_ctx* c, const double* cf = nullptr)
+// The horizontal pass of hydro_deriv along x or y: first and second derivatives of
+// the state with the Maxwell stresses.  (The launches of a step are built by
+// functions of their own: the autotuner times the same ones.)
+SpecLaunch hydro_launch(mhd_ctx* c, int dir)
 {
-    if (c->closure) {
-        if (cf) return MHD_E_STATE;   // the closure's terms need the unfused update
-        TRY(run_closure_flux(c));
-    }
     const int wf = c->wf32;
     void** W = c->wk;
     const Phys& P = c->ph;
@@ -490,10 +489,9 @@ int run_hydro_deriv(mhd_ctx* c, const double* cf = nullptr)
     const int sf = mx ? 1 : 0;
     // second derivatives of u, v, w carry the Maxwell stresses (of the field
     // components and their means) and mixed derivatives as auxiliary lines
-    auto with_b = [&](SpecLaunch& L) {
-        L.bf[0] = c->bx; L.bf[1] = c->by; L.bf[2] = c->bz;
-        if (mx) { L.bmean[0] = c->bxbar; L.bmean[1] = c->bybar; L.bmean[2] = c->bzm; }
-    };
+    SpecLaunch L = spec_base(c, dir, SM_DERIV2);
+    L.bf[0] = c->bx; L.bf[1] = c->by; L.bf[2] = c->bz;
+    if (mx) { L.bmean[0] = c->bxbar; L.bmean[1] = c->bybar; L.bmean[2] = c->bzm; }
     // (own: the mixed mode's array of the stress alone, AuxOp)
     auto stress = [&](SpecJob& j, double c2, double c11, int op, int ai, int aj, double scale, int own) {
         j.mc[0] = c2; j.mc[1] = c11;
@@ -504,12 +502,10 @@ int run_hydro_deriv(mhd_ctx* c, const double* cf = nullptr)
         }
     };
     enum { BX = 0, BY = 1, BZ = 2 };
-    // x pass: d/dx of u, v, w, t, r; the second outputs (HydroColArgs) hold
-    // sck d2/dx2 with u's scko3 d/dx d/dx u of the composite flux (lines 181,
-    // 258) and, in FP64, d/dx of F/2 (bx^2-by^2-bz^2), F by bx, F bz bx
-    {
-        SpecLaunch L = spec_base(c, 0, SM_DERIV2);
-        with_b(L);
+    if (dir == 0) {
+        // d/dx of u, v, w, t, r; the second outputs (HydroColArgs) hold sck d2/dx2
+        // with u's scko3 d/dx d/dx u of the composite flux (lines 181, 258) and, in
+        // FP64, d/dx of F/2 (bx^2-by^2-bz^2), F by bx, F bz bx
         L.job[0] = sjob(U_, sf, W[W_UX], W[W_UXS], MUL_D1, MUL_D2C, wf);
         stress(L.job[0], P.sck, P.scko3, AUX_MAXW, BX, 0, P.fo2, W_DXM);
         L.job[1] = sjob(V_, sf, W[W_VX], W[W_VXS], MUL_D1, MUL_D2C, wf);
@@ -519,33 +515,39 @@ int run_hydro_deriv(mhd_ctx* c, const double* cf = nullptr)
         L.job[3] = sjob(T_, sf, W[W_TX], W[W_TXX], MUL_D1, MUL_D2, wf);
         L.job[4] = sjob(R_, sf, W[W_RX], nullptr, MUL_D1, 0, wf);
         L.njobs = 5;
-        TRY(spec(c, L, MHD_K_XDERIV2));
+        return L;
     }
-    // y pass: the same along y (v's second output carries scko3 d/dy d/dy v),
-    // with d/dy of scko3 vx and scko3 ux of the composite fluxes, in the mixed
-    // mode d/dy of vx and ux as jobs of their own
-    {
-        SpecLaunch L = spec_base(c, 1, SM_DERIV2);
-        with_b(L);
-        L.job[0] = sjob(U_, sf, W[W_UY], W[W_UYS], MUL_D1, MUL_D2C, wf);
-        stress(L.job[0], P.sck, 0.0, AUX_PROD, BY, BX, f, W_YBB);
-        L.job[1] = sjob(V_, sf, W[W_VY], W[W_VYS], MUL_D1, MUL_D2C, wf);
-        stress(L.job[1], P.sck, P.scko3, AUX_MAXW, BY, 0, P.fo2, W_DYM);
-        L.job[2] = sjob(W_, sf, W[W_WY], W[W_WYS], MUL_D1, MUL_D2C, wf);
-        stress(L.job[2], P.sck, 0.0, AUX_PROD, BZ, BY, f, W_YZY);
-        L.job[3] = sjob(T_, sf, W[W_TY], W[W_TYY], MUL_D1, MUL_D2, wf);
-        L.job[4] = sjob(R_, sf, W[W_RY], nullptr, MUL_D1, 0, wf);
-        L.njobs = 5;
-        if (mx) {
-            L.job[5] = sjob(W[W_UX], wf, W[W_UXY], nullptr, MUL_D1, 0, wf);
-            L.job[6] = sjob(W[W_VX], wf, W[W_VXY], nullptr, MUL_D1, 0, wf);
-            L.njobs = 7;
-        } else {
-            L.job[0].xin = W[W_VX]; L.job[0].xcoef = P.scko3;
-            L.job[1].xin = W[W_UX]; L.job[1].xcoef = P.scko3;
-        }
-        TRY(spec(c, L, MHD_K_YDERIV2));
+    // the same along y (v's second output carries scko3 d/dy d/dy v), with d/dy of
+    // scko3 vx and scko3 ux of the composite fluxes, in the mixed mode d/dy of vx and
+    // ux as jobs of their own
+    L.job[0] = sjob(U_, sf, W[W_UY], W[W_UYS], MUL_D1, MUL_D2C, wf);
+    stress(L.job[0], P.sck, 0.0, AUX_PROD, BY, BX, f, W_YBB);
+    L.job[1] = sjob(V_, sf, W[W_VY], W[W_VYS], MUL_D1, MUL_D2C, wf);
+    stress(L.job[1], P.sck, P.scko3, AUX_MAXW, BY, 0, P.fo2, W_DYM);
+    L.job[2] = sjob(W_, sf, W[W_WY], W[W_WYS], MUL_D1, MUL_D2C, wf);
+    stress(L.job[2], P.sck, 0.0, AUX_PROD, BZ, BY, f, W_YZY);
+    L.job[3] = sjob(T_, sf, W[W_TY], W[W_TYY], MUL_D1, MUL_D2, wf);
+    L.job[4] = sjob(R_, sf, W[W_RY], nullptr, MUL_D1, 0, wf);
+    L.njobs = 5;
+    if (mx) {
+        L.job[5] = sjob(W[W_UX], wf, W[W_UXY], nullptr, MUL_D1, 0, wf);
+        L.job[6] = sjob(W[W_VX], wf, W[W_VXY], nullptr, MUL_D1, 0, wf);
+        L.njobs = 7;
+    } else {
+        L.job[0].xin = W[W_VX]; L.job[0].xcoef = P.scko3;
+        L.job[1].xin = W[W_UX]; L.job[1].xcoef = P.scko3;
     }
+    return L;
+}
+
+int run_hydro_deriv(mhd_ctx* c, const double* cf = nullptr)
+{
+    if (c->closure) {
+        if (cf) return MHD_E_STATE;   // the closure's terms need the unfused update
+        TRY(run_closure_flux(c));
+    }
+    TRY(spec(c, hydro_launch(c, 0), MHD_K_XDERIV2));
+    TRY(spec(c, hydro_launch(c, 1), MHD_K_YDERIV2));
     HydroColArgs a = colargs(c);
     if (cf) fuse_ab3(c, a, cf, level_ptr(c, 3, 1), level_ptr(c, 3, 2));
     TRY(timed(c, MHD_K_HYDRO, [&] { return kerr(launch_hydro_col(a, c->wf32, c->s)); }));
@@ -572,20 +574,25 @@ int run_closure_flux(mhd_ctx* c)
     return e ? (e == MHD_E_ALLOC ? e : MHD_E_DEVICE) : 0;
 }
 
+// d/dx of tau_xx, tau_xy, tau_xz, q_x; d/dy of tau_xy, tau_yy, tau_yz, q_y
+SpecLaunch closure_launch(mhd_ctx* c, int dir)
+{
+    static const int ix[4] = {0, 3, 4, 9}, iy[4] = {3, 1, 5, 10};
+    const int wf = c->wf32;
+    SpecLaunch L = spec_base(c, dir, SM_DERIV1);
+    for (int m = 0; m < 4; ++m)
+        L.job[m] = sjob(c->cflux[dir == 0 ? ix[m] : iy[m]], wf, dir == 0 ? c->cdx[m] : c->cdy[m], nullptr, MUL_D1, 0,
+                        wf);
+    L.njobs = 4;
+    return L;
+}
+
 // -div(tau)/r into udot, vdot, wdot and -div(q) into tdot (newest level)
 int run_closure_tend(mhd_ctx* c)
 {
     const int wf = c->wf32;
-    // x: tau_xx, tau_xy, tau_xz, q_x; y: tau_xy, tau_yy, tau_yz, q_y; z: tau_xz, tau_yz, tau_zz, q_z
-    static const int ix[4] = {0, 3, 4, 9}, iy[4] = {3, 1, 5, 10}, iz[4] = {4, 5, 2, 11};
-    for (int dir = 0; dir < 2; ++dir) {
-        SpecLaunch L = spec_base(c, dir, SM_DERIV1);
-        for (int m = 0; m < 4; ++m)
-            L.job[m] = sjob(c->cflux[dir == 0 ? ix[m] : iy[m]], wf, dir == 0 ? c->cdx[m] : c->cdy[m], nullptr,
-                            MUL_D1, 0, wf);
-        L.njobs = 4;
-        TRY(spec(c, L));
-    }
+    static const int iz[4] = {4, 5, 2, 11};   // tau_xz, tau_yz, tau_zz, q_z
+    for (int dir = 0; dir < 2; ++dir) TRY(spec(c, closure_launch(c, dir)));
     ZLaunch Z = zbase(c);
     for (int m = 0; m < 4; ++m) Z.job[m] = zjob(c->cflux[iz[m]], wf, c->cdz[m], wf, ZK_D1, 5);
     Z.njobs = 4;
@@ -613,6 +620,57 @@ MagSpecArgs mag_spec_args(mhd_ctx* c, const MagArgs& m)
     return a;
 }
 
+// E = u x B (308-316), fused into the first pass of forwardfft: y where the x
+// pass can follow with the spectral derivatives (emf_x), else x
+SpecLaunch emf_launch(mhd_ctx* c, const MagArgs& m)
+{
+    const int wf = c->wf32;
+    SpecLaunch L = spec_base(c, spectral_len_fixed(c->nx) ? 1 : 0, SM_R2HC);
+    // mixed precision: FP32 velocity shadows, B without its means (added by the loads)
+    const bool mx = c->su != nullptr;
+    const void* U_ = mx ? (const void*)c->su : c->u;
+    const void* V_ = mx ? (const void*)c->sv : c->v;
+    const void* W_ = mx ? (const void*)c->sw : c->w;
+    const double* mbx = mx ? c->bxbar : nullptr;
+    const double* mby = mx ? c->bybar : nullptr;
+    const double* mbz = mx ? c->bzm : nullptr;
+    L.job[0] = sjob(V_, wf, m.exh, nullptr, 0, 0, wf);
+    L.job[0].load_op = LD_CROSS; L.job[0].in[1] = c->bz; L.job[0].in[2] = W_; L.job[0].in[3] = c->by;
+    L.job[0].mean[1] = mbz; L.job[0].mean[3] = mby;
+    L.job[1] = sjob(W_, wf, m.eyh, nullptr, 0, 0, wf);
+    L.job[1].load_op = LD_CROSS; L.job[1].in[1] = c->bx; L.job[1].in[2] = U_; L.job[1].in[3] = c->bz;
+    L.job[1].mean[1] = mbx; L.job[1].mean[3] = mbz;
+    L.job[2] = sjob(U_, wf, m.ezh, nullptr, 0, 0, wf);
+    L.job[2].load_op = LD_CROSS; L.job[2].in[1] = c->by; L.job[2].in[2] = V_; L.job[2].in[3] = c->bx;
+    L.job[2].mean[1] = mby; L.job[2].mean[3] = mbx;
+    if (c->eta_on) {
+        // eta(z) extension: E = u x B - zeta C_k (eta/eta_0 - 1) J
+        L.job[0].jin = c->jx; L.job[0].jcoef = c->eta1;
+        L.job[1].jin = c->jy; L.job[1].jcoef = c->eta1;
+        L.job[2].jin = c->jz; L.job[2].jcoef = c->eta1;
+    } else if (c->closure) {
+        // closure: E = u x B + eps
+        for (int q = 0; q < 3; ++q) {
+            L.job[q].jin = c->cflux[6 + q];
+            L.job[q].jcoef = c->cneg1;
+        }
+    }
+    L.njobs = 3;
+    return L;
+}
+
+// the forward transform of three lines in place (mag_init; E along y where emf_x cannot run)
+SpecLaunch forward_launch(mhd_ctx* c, int dir, const MagArgs& m)
+{
+    const int wf = c->wf32;
+    SpecLaunch L = spec_base(c, dir, SM_R2HC);
+    L.job[0] = sjob(m.exh, wf, m.exh, nullptr, 0, 0, wf);
+    L.job[1] = sjob(m.eyh, wf, m.eyh, nullptr, 0, 0, wf);
+    L.job[2] = sjob(m.ezh, wf, m.ezh, nullptr, 0, 0, wf);
+    L.njobs = 3;
+    return L;
+}
+
 // ---------------------------------------------------------------------------
 // mag_deriv, src/magnetic.f90:285-487
 // ---------------------------------------------------------------------------
@@ -620,56 +678,13 @@ MagSpecArgs mag_spec_args(mhd_ctx* c, const MagArgs& m)
 // values in the ping-pong buffers), or null for the right-hand sides only
 int run_mag_deriv(mhd_ctx* c, const double* cf = nullptr)
 {
-    const int wf = c->wf32;
     MagArgs m = margs(c);
-    {
-        // E = u x B (308-316), fused into the first pass of forwardfft: y where
-        // the x pass can follow with the spectral derivatives (emf_x), else x
-        const bool fused = spectral_len_fixed(c->nx);
-        SpecLaunch L = spec_base(c, fused ? 1 : 0, SM_R2HC);
-        // mixed precision: FP32 velocity shadows, B without its means (added by the loads)
-        const bool mx = c->su != nullptr;
-        const void* U_ = mx ? (const void*)c->su : c->u;
-        const void* V_ = mx ? (const void*)c->sv : c->v;
-        const void* W_ = mx ? (const void*)c->sw : c->w;
-        const double* mbx = mx ? c->bxbar : nullptr;
-        const double* mby = mx ? c->bybar : nullptr;
-        const double* mbz = mx ? c->bzm : nullptr;
-        L.job[0] = sjob(V_, wf, m.exh, nullptr, 0, 0, wf);
-        L.job[0].load_op = LD_CROSS; L.job[0].in[1] = c->bz; L.job[0].in[2] = W_; L.job[0].in[3] = c->by;
-        L.job[0].mean[1] = mbz; L.job[0].mean[3] = mby;
-        L.job[1] = sjob(W_, wf, m.eyh, nullptr, 0, 0, wf);
-        L.job[1].load_op = LD_CROSS; L.job[1].in[1] = c->bx; L.job[1].in[2] = U_; L.job[1].in[3] = c->bz;
-        L.job[1].mean[1] = mbx; L.job[1].mean[3] = mbz;
-        L.job[2] = sjob(U_, wf, m.ezh, nullptr, 0, 0, wf);
-        L.job[2].load_op = LD_CROSS; L.job[2].in[1] = c->by; L.job[2].in[2] = V_; L.job[2].in[3] = c->bx;
-        L.job[2].mean[1] = mby; L.job[2].mean[3] = mbx;
-        if (c->eta_on) {
-            // eta(z) extension: E = u x B - zeta C_k (eta/eta_0 - 1) J
-            L.job[0].jin = c->jx; L.job[0].jcoef = c->eta1;
-            L.job[1].jin = c->jy; L.job[1].jcoef = c->eta1;
-            L.job[2].jin = c->jz; L.job[2].jcoef = c->eta1;
-        } else if (c->closure) {
-            // closure: E = u x B + eps
-            for (int q = 0; q < 3; ++q) {
-                L.job[q].jin = c->cflux[6 + q];
-                L.job[q].jcoef = c->cneg1;
-            }
-        }
-        L.njobs = 3;
-        TRY(spec(c, L));
-        if (fused) {
-            MagSpecArgs x = mag_spec_args(c, m);
-            TRY(kerr(launch_emf_x(x, wf, c->s)));
-        } else {
-            SpecLaunch M = spec_base(c, 1, SM_R2HC);
-            M.job[0] = sjob(m.exh, wf, m.exh, nullptr, 0, 0, wf);
-            M.job[1] = sjob(m.eyh, wf, m.eyh, nullptr, 0, 0, wf);
-            M.job[2] = sjob(m.ezh, wf, m.ezh, nullptr, 0, 0, wf);
-            M.njobs = 3;
-            TRY(spec(c, M));
-            TRY(kerr(launch_mag_spec1(m, c->s)));
-        }
+    TRY(spec(c, emf_launch(c, m)));
+    if (spectral_len_fixed(c->nx)) {
+        TRY(kerr(launch_emf_x(mag_spec_args(c, m), c->wf32, c->s)));
+    } else {
+        TRY(spec(c, forward_launch(c, 1, m)));
+        TRY(kerr(launch_mag_spec1(m, c->s)));
     }
     if (cf) {
         m.ab3 = 1;
@@ -696,40 +711,49 @@ int run_mag_deriv(mhd_ctx* c, const double* cf = nullptr)
 // ---------------------------------------------------------------------------
 // bandj, src/magnetic.f90:492-664 (jsq tail shared with mag_init)
 // ---------------------------------------------------------------------------
-int inverse_b_and_j(mhd_ctx* c, MagArgs& m, bool with_b)
+// (with_b: B too, 575-593; y: then its mean parts, which the mixed path keeps apart)
+SpecLaunch inverse_launch(mhd_ctx* c, int dir, const MagArgs& m, bool with_b)
 {
     const int wf = c->wf32;
-    SpecLaunch L = spec_base(c, 0, SM_HC2R);
+    const bool mx = c->su != nullptr;
+    SpecLaunch L = spec_base(c, dir, SM_HC2R);
     int n = 0;
     if (with_b) {
-        L.job[n++] = sjob(m.bxh, wf, m.bxh, nullptr, 0, 0, wf);
-        L.job[n++] = sjob(m.byh, wf, m.byh, nullptr, 0, 0, wf);
-        L.job[n++] = sjob(m.bzh, wf, m.bzh, nullptr, 0, 0, wf);
+        L.job[n++] = sjob(m.bxh, wf, dir == 0 ? m.bxh : c->bx, nullptr, 0, 0, wf);
+        L.job[n++] = sjob(m.byh, wf, dir == 0 ? m.byh : c->by, nullptr, 0, 0, wf);
+        L.job[n++] = sjob(m.bzh, wf, dir == 0 ? m.bzh : c->bz, nullptr, 0, 0, wf);
+        if (dir == 1 && !mx) {
+            L.job[0].addk = c->bxbar;
+            L.job[1].addk = c->bybar;
+            L.job[2].adds = c->sc.bzbar;
+        }
     }
     L.job[n++] = sjob(m.dybzh, wf, m.dybzh, nullptr, 0, 0, wf);
     L.job[n++] = sjob(m.dxbzh, wf, m.dxbzh, nullptr, 0, 0, wf);
     L.job[n++] = sjob(m.jzh, wf, m.jzh, nullptr, 0, 0, wf);
     L.njobs = n;
-    TRY(spec(c, L));
-    SpecLaunch M = spec_base(c, 1, SM_HC2R);
-    n = 0;
-    if (with_b) {
-        // 575-593: inverse transforms, then the mean parts of B
-        // (the mixed path keeps B without its means: no additions)
-        const bool mx = c->su != nullptr;
-        M.job[n] = sjob(m.bxh, wf, c->bx, nullptr, 0, 0, wf);
-        M.job[n++].addk = mx ? nullptr : c->bxbar;
-        M.job[n] = sjob(m.byh, wf, c->by, nullptr, 0, 0, wf);
-        M.job[n++].addk = mx ? nullptr : c->bybar;
-        M.job[n] = sjob(m.bzh, wf, c->bz, nullptr, 0, 0, wf);
-        M.job[n++].adds = mx ? 0.0 : c->sc.bzbar;
-    }
-    M.job[n++] = sjob(m.dybzh, wf, m.dybzh, nullptr, 0, 0, wf);
-    M.job[n++] = sjob(m.dxbzh, wf, m.dxbzh, nullptr, 0, 0, wf);
-    M.job[n++] = sjob(m.jzh, wf, m.jzh, nullptr, 0, 0, wf);
-    M.njobs = n;
-    TRY(spec(c, M));
+    return L;
+}
+
+int inverse_b_and_j(mhd_ctx* c, const MagArgs& m, bool with_b)
+{
+    for (int dir = 0; dir < 2; ++dir) TRY(spec(c, inverse_launch(c, dir, m, with_b)));
     return kerr(launch_jsq(m, c->s));
+}
+
+// The y pass after bandj_x.  FP64: dBz/dy rides with Bz, from its spectrum.
+SpecLaunch bandj_y_launch(mhd_ctx* c, const MagArgs& m, bool clean)
+{
+    SpecLaunch L = inverse_launch(c, 1, m, true);
+    L.skip = clean;
+    if (!c->su) {
+        L.job[2].out[1] = m.dybzh;
+        L.job[2].mul[1] = MUL_D1;
+        std::swap(L.job[0], L.job[2]);   // the longest first
+        L.job[3] = L.job[5];
+        L.njobs = 5;
+    }
+    return L;
 }
 
 // clean: pol and tor are zero in the 2/3 band (magdealias has just run)
@@ -750,22 +774,7 @@ int run_bandj(mhd_ctx* c, bool clean)
     MagSpecArgs x = mag_spec_args(c, m);
     x.skip = clean;
     TRY(kerr(launch_bandj_x(x, wf, c->s)));
-    // 575-593: y transforms and the mean parts of B (the mixed path keeps B
-    // without its means: no additions); dBz/dy rides with Bz in FP64
-    const bool mx = c->su != nullptr;
-    SpecLaunch M = spec_base(c, 1, SM_HC2R);
-    M.skip = clean;
-    M.job[0] = sjob(m.bzh, wf, c->bz, mx ? nullptr : m.dybzh, 0, MUL_D1, wf);
-    M.job[0].adds = mx ? 0.0 : c->sc.bzbar;
-    M.job[1] = sjob(m.bxh, wf, c->bx, nullptr, 0, 0, wf);
-    M.job[1].addk = mx ? nullptr : c->bxbar;
-    M.job[2] = sjob(m.byh, wf, c->by, nullptr, 0, 0, wf);
-    M.job[2].addk = mx ? nullptr : c->bybar;
-    M.job[3] = sjob(m.dxbzh, wf, m.dxbzh, nullptr, 0, 0, wf);
-    M.job[4] = sjob(m.jzh, wf, m.jzh, nullptr, 0, 0, wf);
-    M.njobs = 5;
-    if (mx) M.job[M.njobs++] = sjob(m.dybzh, wf, m.dybzh, nullptr, 0, 0, wf);
-    TRY(spec(c, M));
+    TRY(spec(c, bandj_y_launch(c, m, clean)));
     return kerr(launch_jsq(m, c->s));
 }
 
@@ -846,12 +855,7 @@ int run_mag_init(mhd_ctx* c)
     L.job[2] = sjob(c->bz, wf, m.ezh, nullptr, 0, 0, wf);
     L.njobs = 3;
     TRY(spec(c, L));
-    SpecLaunch M = spec_base(c, 1, SM_R2HC);
-    M.job[0] = sjob(m.exh, wf, m.exh, nullptr, 0, 0, wf);
-    M.job[1] = sjob(m.eyh, wf, m.eyh, nullptr, 0, 0, wf);
-    M.job[2] = sjob(m.ezh, wf, m.ezh, nullptr, 0, 0, wf);
-    M.njobs = 3;
-    TRY(spec(c, M));
+    TRY(spec(c, forward_launch(c, 1, m)));
     TRY(kerr(launch_mag_init_spec(m, c->s, c->d_bzbar)));
     MHD_HIP_CHECK(hipMemcpyAsync(&c->sc.bzbar, c->d_bzbar, sizeof(double), hipMemcpyDeviceToHost, c->s));
     MHD_HIP_CHECK(hipStreamSynchronize(c->s));
@@ -868,17 +872,20 @@ int run_mag_init(mhd_ctx* c)
     return run_mag_boundary(c, 0, 1);
 }
 
-// 5-field dealias (src/main.F90:495-502), in place
+// 5-field dealias (src/main.F90:495-502), in place; the FP64 state is filtered in
+// FP64 in both precision modes
+SpecLaunch dealias_launch(mhd_ctx* c, int dir)
+{
+    double* f5[5] = {c->r, c->t, c->u, c->v, c->w};
+    SpecLaunch L = spec_base(c, dir, SM_DERIV1, true);
+    for (int i = 0; i < 5; ++i) L.job[i] = sjob(f5[i], 0, f5[i], nullptr, MUL_MASK, 0, 0);
+    L.njobs = 5;
+    return L;
+}
+
 int run_dealias5(mhd_ctx* c)
 {
-    // the FP64 state is filtered in FP64 in both precision modes
-    double* f5[5] = {c->r, c->t, c->u, c->v, c->w};
-    for (int dir = 0; dir < 2; ++dir) {
-        SpecLaunch L = spec_base(c, dir, SM_DERIV1, true);
-        for (int i = 0; i < 5; ++i) L.job[i] = sjob(f5[i], 0, f5[i], nullptr, MUL_MASK, 0, 0);
-        L.njobs = 5;
-        TRY(spec64(c, L));
-    }
+    for (int dir = 0; dir < 2; ++dir) TRY(spec64(c, dealias_launch(c, dir)));
     return refresh_shadows(c);
 }
 
@@ -1936,57 +1943,49 @@ int mhd_autotune(mhd_ctx_t* c, mhd_tune_t* out)
     if (!c->have_state) return MHD_E_STATE;
     const int saved_timing = c->timed_kernel;
     c->timed_kernel = MHD_K_NONE;
-    const int wf = c->wf32;
     void** W = c->wk;
-    const void* in[4] = {c->su ? (const void*)c->st : c->t, c->su ? (const void*)c->su : c->u,
-                         c->su ? (const void*)c->sv : c->v, c->su ? (const void*)c->sw : c->w};
-    const int sf = c->su ? 1 : 0;
     double best_ms[2] = {0, 0};
-    // transforms, per direction and kind: the radix plan and the
-    // persistent-grid multiple, on a launch of that kind shaped like the
-    // step's (outputs into work arrays); the current choice (the default at
-    // first) is timed first
-    const int o1[2][4] = {{W_TX, W_UX, W_VX, W_WX}, {W_TY, W_UY, W_VY, W_WY}};
-    const int o2[2][4] = {{W_TXX, W_UXS, W_VXS, W_WXS}, {W_TYY, W_UYS, W_VYS, W_WYS}};
-    auto kind_launch = [&](int dir, int kind) {
-        SpecLaunch L = spec_base(c, dir, kind);
-        for (int j = 0; j < 4; ++j) {
-            void* a = W[o1[dir][j]];
-            if (kind == SM_DERIV2) L.job[j] = sjob(in[j], sf, a, W[o2[dir][j]], MUL_D1, MUL_D2, wf);
-            else if (kind == SM_DERIV1) L.job[j] = sjob(in[j], sf, a, nullptr, MUL_D1, 0, wf);
-            else L.job[j] = sjob(in[j], sf, a, nullptr, 0, 0, wf);
-        }
-        L.njobs = 4;
+    // transforms, per direction and kind: the radix plan and the persistent-grid
+    // multiple, on the launch of that kind that the step makes, into work arrays;
+    // the default is timed first.  A kind that the
+    // box's step does not run (along x the half transforms, where emf_x and bandj_x
+    // take their place) keeps its choice.
+    const bool fused = spectral_len_fixed(c->nx), mag = c->ph.mag;
+    const MagArgs m = margs(c);
+    auto step_launch = [&](int dir, int kind, SpecLaunch& L, bool& f64) -> bool {
+        f64 = false;
         if (kind == SM_DERIV2) {
-            // as in the step: three jobs with auxiliary lines, one without, and a
-            // single-output (first-derivative) job
-            L.bf[0] = in[1]; L.bf[1] = in[2]; L.bf[2] = in[3];
-            for (int j = 0; j < 3; ++j) {
-                L.job[j].aux = j == 0 ? AUX_MAXW : AUX_PROD;
-                L.job[j].ai = j;
-                L.job[j].aj = 0;
-                L.job[j].ascale = 1.0;
-                if (c->su) {
-                    static const int o3[2][3] = {{W_XBB, W_XZX, W_DXM}, {W_YBB, W_YZY, W_DYM}};
-                    L.job[j].out[2] = W[o3[dir][j]];
-                } else if (dir == 1 && j < 2) {
-                    L.job[j].xin = in[0];
-                }
-            }
-            L.job[4] = sjob(in[0], sf, W[dir == 0 ? W_RX : W_RY], nullptr, MUL_D1, 0, wf);
-            L.njobs = 5;
-            if (c->su && dir == 1) {
-                L.job[5] = sjob(in[1], sf, W[W_UXY], nullptr, MUL_D1, 0, wf);
-                L.job[6] = sjob(in[2], sf, W[W_VXY], nullptr, MUL_D1, 0, wf);
-                L.njobs = 7;
-            }
+            L = hydro_launch(c, dir);
+            return true;
         }
-        return L;
+        if (kind == SM_DERIV1) {
+            // the closure's divergences of every step, else the dealias of every tenth
+            if (c->closure) {
+                L = closure_launch(c, dir);
+            } else {
+                L = dealias_launch(c, dir);
+                f64 = true;
+                double* to[5] = {c->r2, c->t2, c->u2, c->v2, c->w2};
+                for (int q = 0; q < 5; ++q) L.job[q].out[0] = to[q];
+            }
+            return true;
+        }
+        if (!mag || (fused && dir == 0)) return false;
+        if (kind == SM_R2HC) {
+            L = fused || dir == 0 ? emf_launch(c, m) : forward_launch(c, dir, m);
+        } else {
+            L = fused ? bandj_y_launch(c, m, true) : inverse_launch(c, dir, m, true);
+            for (int q = 0; q < L.njobs; ++q) L.job[q].out[0] = (void*)L.job[q].in[0];   // not into B
+        }
+        return true;
     };
     for (int dir = 0; dir < 2; ++dir) {
         const int n = dir == 0 ? c->nx : c->ny;
         const int mdef = (dir == 1 && !c->wf32) ? 2 : 1;
         for (int kind = 0; kind < MHD_TK_N; ++kind) {
+            SpecLaunch L;
+            bool f64;
+            if (!step_launch(dir, kind, L, f64)) continue;
             double bk = 1e30;
             int bv = 0, bm = mdef;
             for (int var = 0; var < spectral_variants(n); ++var) {
@@ -1994,9 +1993,9 @@ int mhd_autotune(mhd_ctx_t* c, mhd_tune_t* out)
                     const int mult = mi == 0 ? mdef : 3 - mdef;
                     c->spec_var[dir][kind] = var;
                     c->spec_mult[dir][kind] = mult;
-                    const SpecLaunch L = kind_launch(dir, kind);
+                    step_launch(dir, kind, L, f64);
                     double ms = 0.0;
-                    TRY(time_ms(c, TUNE_REPS, [&] { return spec(c, L); }, &ms));
+                    TRY(time_ms(c, TUNE_REPS, [&] { return f64 ? spec64(c, L) : spec(c, L); }, &ms));
                     if (ms < TUNE_GAIN * bk) { bk = ms; bv = var; bm = mult; }
                 }
             }

@@ -202,8 +202,11 @@ long mhd_dump_header(const mhd_dump_t* meta, int iprec, unsigned char* buf, long
  * context: per transform direction and kind (first derivatives, first and
  * second derivatives, real to halfcomplex and back) the radix plan (the
  * default or one of the length's alternatives) together with the
- * persistent-grid multiple (1 or 2 x resident), on a launch of that kind
- * shaped like the step's; the planes per thread, at most, of the
+ * persistent-grid multiple (1 or 2 x resident), on the launch of that kind
+ * that the step makes (first derivatives: the dealias, with a closure its
+ * divergences).  A kind that the box's step does not run, such as the half
+ * transforms along an x length with a register plan, keeps the choice it had
+ * and serves the operators and mag_init only.  Then the planes per thread, at most, of the
  * column-walking hydro kernel, in the variant the step runs (with the fused
  * AB3 update unless a closure is attached; the magnetic column kernels keep
  * 8 planes).  Boxes too small to fill the GPU with walks of 8 planes take
