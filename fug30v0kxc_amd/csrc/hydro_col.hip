@@ -404,7 +404,7 @@ int launch_hydro_col(const HydroColArgs& a, int mixed, hipStream_t s)
     const int nin = a.g.nz > 8 ? a.g.nz - 8 : 0;   // interior planes
     const unsigned chunks = (unsigned)((nin + a.zc - 1) / a.zc), walls = (unsigned)(a.g.nz < 8 ? a.g.nz : 8);
     auto go = [&](auto all, auto interior, auto wall) -> int {
-        if (!launch_recorder()) return mhd_launch<decltype(all)>(dim3(bx, chunks + walls), dim3(HNT), 0, s, a);
+        if (!launch_recorder()) return mhd_issue<decltype(all)>(dim3(bx, chunks + walls), dim3(HNT), 0, s, a);
         if (chunks) {
             const int e = mhd_launch<decltype(interior)>(dim3(bx, chunks), dim3(HNT), 0, s, a);
             if (e) return e;

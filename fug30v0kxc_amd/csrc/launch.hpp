@@ -98,6 +98,15 @@ int batch_launch(const BatchTable& t, unsigned total, unsigned nt, size_t lds, h
     return hipGetLastError() == hipSuccess ? 0 : -22;
 }
 
+// a launch that is never recorded: no batched kernel is built for it
+template <typename K>
+int mhd_issue(dim3 grid, dim3 block, size_t lds, hipStream_t s, const typename K::Args& a)
+{
+    if (grid.x == 0 || grid.y == 0 || grid.z == 0) return 0;
+    hipLaunchKernelGGL(single_kernel<K>, grid, block, lds, s, a);
+    return hipGetLastError() == hipSuccess ? 0 : -22;
+}
+
 template <typename K>
 int mhd_launch(dim3 grid, dim3 block, size_t lds, hipStream_t s, const typename K::Args& a)
 {
@@ -114,8 +123,7 @@ int mhd_launch(dim3 grid, dim3 block, size_t lds, hipStream_t s, const typename 
         r->recs.push_back(std::move(rec));
         return 0;
     }
-    hipLaunchKernelGGL(single_kernel<K>, grid, block, lds, s, a);
-    return hipGetLastError() == hipSuccess ? 0 : -22;
+    return mhd_issue<K>(grid, block, lds, s, a);
 }
 
 }  // namespace mhd

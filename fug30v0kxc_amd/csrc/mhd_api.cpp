@@ -289,7 +289,6 @@ SpecJob sjob(const void* in, int in_f32, void* o0, void* o1, int m0, int m1, int
     j.in[0] = in;
     j.in_f32 = in_f32;
     j.load_op = LD_PLAIN;
-    j.scale = 1.0;
     j.out[0] = o0;
     j.out[1] = o1;
     j.mul[0] = m0;
@@ -304,8 +303,6 @@ ZJob zjob(const void* in, int in_f32, void* out, int out_f32, int kind, int flag
     memset(&j, 0, sizeof(j));
     j.in = in;
     j.in_f32 = in_f32;
-    j.load_op = 0;
-    j.scale = 1.0;
     j.out = out;
     j.out_f32 = out_f32;
     j.kind = kind;
@@ -321,7 +318,7 @@ ZLaunch zbase(mhd_ctx* c)
     L.ho12 = c->ph.ho12;
     L.sc1 = c->ph.sc1;
     L.w = c->w;
-    L.w_f32 = 0;
+    L.ncu = c->ncu;
     return L;
 }
 
@@ -995,17 +992,23 @@ void ab3_coeffs(mhd_scalars_t& s, double dt, double cf[3])
     }
 }
 
-// f0 = 0: all fields and the means.  f0 = 5: the hydro fields were updated by
-// the fused hydro kernel.  f0 = 7: pol, tor and the means too (fused into
-// mag_rhs and mean_emf).  Then the history ring turns and the state ping-pong
-// swaps.
-int run_ab3(mhd_ctx* c, const double cf[3], int f0 = 0)
+void turn_ring(mhd_ctx* c)
+{
+    // shift 2->1, 3->2 (src/main.F90:448-476): relabel the ring
+    const int r0 = c->ring[0];
+    c->ring[0] = c->ring[1];
+    c->ring[1] = c->ring[2];
+    c->ring[2] = r0;
+}
+
+// The update of all fields and the means (a closure's step), then the history ring
+// turns.
+int run_ab3(mhd_ctx* c, const double cf[3])
 {
     AB3Args a;
     memset(&a, 0, sizeof(a));
     a.g = c->g;
     a.c0 = cf[0]; a.c1 = cf[1]; a.c2 = cf[2];
-    a.f0 = f0;
     double* vars[7] = {c->u, c->v, c->w, c->r, c->t, c->pol, c->tor};
     for (int f = 0; f < 7; ++f) {
         a.var[f] = vars[f];
@@ -1025,24 +1028,24 @@ int run_ab3(mhd_ctx* c, const double cf[3], int f0 = 0)
     a.nfields = a.mag ? 7 : 5;
     a.icutx = c->icutx;
     a.icuty = c->icuty;
-    // f0 = 7: the means were updated by mean_emf
-    if (a.f0 < a.nfields) TRY(timed(c, MHD_K_AB3, [&] { return kerr(launch_ab3(a, c->s)); }));
-    if (f0 >= 5) {
-        std::swap(c->u, c->u2); std::swap(c->v, c->v2); std::swap(c->w, c->w2);
-        std::swap(c->t, c->t2); std::swap(c->r, c->r2);
-        std::swap(c->su, c->su2); std::swap(c->sv, c->sv2); std::swap(c->sw, c->sw2);
-        std::swap(c->st, c->st2); std::swap(c->sr, c->sr2);
-    }
-    if (f0 >= 7) {
+    TRY(timed(c, MHD_K_AB3, [&] { return kerr(launch_ab3(a, c->s)); }));
+    turn_ring(c);
+    return 0;
+}
+
+// The column kernels have updated the hydro fields into the ping-pong buffers and,
+// with mag, pol, tor and (mean_emf) the means.
+void swap_state(mhd_ctx* c, bool mag)
+{
+    std::swap(c->u, c->u2); std::swap(c->v, c->v2); std::swap(c->w, c->w2);
+    std::swap(c->t, c->t2); std::swap(c->r, c->r2);
+    std::swap(c->su, c->su2); std::swap(c->sv, c->sv2); std::swap(c->sw, c->sw2);
+    std::swap(c->st, c->st2); std::swap(c->sr, c->sr2);
+    if (mag) {
         std::swap(c->pol, c->pol2);
         std::swap(c->tor, c->tor2);
     }
-    // shift 2->1, 3->2 (src/main.F90:448-476): relabel the ring
-    const int r0 = c->ring[0];
-    c->ring[0] = c->ring[1];
-    c->ring[1] = c->ring[2];
-    c->ring[2] = r0;
-    return 0;
+    turn_ring(c);
 }
 
 }  // namespace
@@ -1587,7 +1590,7 @@ int mhd_step(mhd_ctx_t* c, int nsteps, double dt_fixed, int ndu06, mhd_diag_t* l
         } else {
             TRY(run_hydro_deriv(c, cf));       // hydro RHS + AB3 of u v w r t into the ping-pong
             if (mag) TRY(run_mag_deriv(c, cf)); // reads the old u v w; + AB3 of pol, tor, magdealias
-            TRY(run_ab3(c, cf, mag ? 7 : 5));  // swaps
+            swap_state(c, mag);
         }
         if (mag) c->band_clean = 1;   // magdealias is part of either update
         S.dt2 = dt + S.dt1;

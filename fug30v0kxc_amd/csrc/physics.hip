@@ -30,17 +30,16 @@ __device__ __forceinline__ bool in_band(int p, int q, int nx, int ny, int icx, i
     return (p >= nx / 2 - icx && p <= nx / 2 + icx) || (q >= ny / 2 - icy && q <= ny / 2 + icy);
 }
 
-// TC: compute/output type; TIN: input element type; KIND: ZKind; PROD: the
-// input is scale*in*in1.  w (upwind selector) has the element type TW.
-template <typename TC, typename TIN, typename TW, int KIND, bool PROD, int ZKC>
+// TC: compute/output type; TIN: input element type; KIND: ZKind
+template <typename TC, typename TIN, int KIND, int ZKC>
 struct ZKernel {
     using Args = ZLaunch;
     static constexpr int NT = 256;
     static __device__ __forceinline__ void body(const ZLaunch& L, uint3 bid, uint3 gdim);
 };
 
-template <typename TC, typename TIN, typename TW, int KIND, bool PROD, int ZKC>
-__device__ __forceinline__ void ZKernel<TC, TIN, TW, KIND, PROD, ZKC>::body(const ZLaunch& L, uint3 bid, uint3 gdim)
+template <typename TC, typename TIN, int KIND, int ZKC>
+__device__ __forceinline__ void ZKernel<TC, TIN, KIND, ZKC>::body(const ZLaunch& L, uint3 bid, uint3 gdim)
 {
     (void)bid;
     (void)gdim;
@@ -53,18 +52,11 @@ __device__ __forceinline__ void ZKernel<TC, TIN, TW, KIND, PROD, ZKC>::body(cons
         if (in_band(ip, jq, L.g.nx, L.g.ny, L.icutx, L.icuty)) return;
     }
     const TIN* __restrict__ in = (const TIN*)J.in;
-    const TIN* __restrict__ in1 = (const TIN*)J.in1;
-    const TC scale = (TC)J.scale;
     TC* __restrict__ out = (TC*)J.out;
     const int flag = J.flag;
-    const TW* __restrict__ wp = (const TW*)L.w;
+    const double* __restrict__ wp = L.w;
     const TC h = (TC)L.ho12, s = (TC)L.sc1;
-    auto ld = [=](int kk) -> TC {
-        const long i = col + (long)kk * nxy;
-        TC v = (TC)in[i];
-        if constexpr (PROD) v = (scale * v) * (TC)in1[i];
-        return v;
-    };
+    auto ld = [=](int kk) -> TC { return (TC)in[col + (long)kk * nxy]; };
     const int k0 = bid.y * ZKC;
     if (k0 >= 3 && k0 + ZKC <= nz - 3) {
         constexpr int LO = (KIND == ZK_D1UP) ? 0 : 1;          // first window slot used
@@ -104,33 +96,27 @@ __device__ __forceinline__ void ZKernel<TC, TIN, TW, KIND, PROD, ZKC>::body(cons
     }
 }
 
-template <typename TC, typename TIN, typename TW, int KIND, bool PROD>
+template <typename TC, typename TIN, int KIND>
 static int launch_z_group(ZLaunch& G, hipStream_t s)
 {
-    const unsigned bx = nblk(G.g.nxy);
-    const long wide = (long)bx * ((G.g.nz + 15) / 16) * G.njobs;
-    if (wide >= 256 || launch_recorder())
-        return mhd_launch<ZKernel<TC, TIN, TW, KIND, PROD, 16>>(dim3(bx, (unsigned)((G.g.nz + 15) / 16), G.njobs),
-                                                                dim3(NT), 0, s, G);
-    return mhd_launch<ZKernel<TC, TIN, TW, KIND, PROD, 4>>(dim3(bx, (unsigned)((G.g.nz + 3) / 4), G.njobs), dim3(NT),
-                                                           0, s, G);
+    const unsigned bx = nblk(G.g.nxy), n16 = (unsigned)((G.g.nz + 15) / 16), n4 = (unsigned)((G.g.nz + 3) / 4);
+    if ((long)bx * n16 * G.njobs >= G.ncu || launch_recorder())
+        return mhd_launch<ZKernel<TC, TIN, KIND, 16>>(dim3(bx, n16, G.njobs), dim3(NT), 0, s, G);
+    return mhd_issue<ZKernel<TC, TIN, KIND, 4>>(dim3(bx, n4, G.njobs), dim3(NT), 0, s, G);
 }
 
-template <typename TC, typename TIN, typename TW>
-static int launch_z_kind(ZLaunch& G, int kind, bool prod, hipStream_t s)
+template <typename TC, typename TIN>
+static int launch_z_kind(ZLaunch& G, int kind, hipStream_t s)
 {
-    switch (kind * 2 + (prod ? 1 : 0)) {
-    case 0: return launch_z_group<TC, TIN, TW, ZK_D1, false>(G, s);
-    case 1: return launch_z_group<TC, TIN, TW, ZK_D1, true>(G, s);
-    case 2: return launch_z_group<TC, TIN, TW, ZK_D1UP, false>(G, s);
-    case 3: return launch_z_group<TC, TIN, TW, ZK_D1UP, true>(G, s);
-    case 4: return launch_z_group<TC, TIN, TW, ZK_D2, false>(G, s);
-    case 5: return launch_z_group<TC, TIN, TW, ZK_D2, true>(G, s);
+    switch (kind) {
+    case ZK_D1: return launch_z_group<TC, TIN, ZK_D1>(G, s);
+    case ZK_D1UP: return launch_z_group<TC, TIN, ZK_D1UP>(G, s);
+    case ZK_D2: return launch_z_group<TC, TIN, ZK_D2>(G, s);
     }
     return -23;
 }
 
-// Jobs are grouped by (input type, kind, product load); one launch per group.
+// Jobs are grouped by (types, kind); one launch per group.
 int launch_z(const ZLaunch& L, hipStream_t s)
 {
     if (L.njobs <= 0) return 0;
@@ -144,23 +130,17 @@ int launch_z(const ZLaunch& L, hipStream_t s)
         G.njobs = 0;
         for (int j = i; j < L.njobs; ++j) {
             const ZJob& b = L.job[j];
-            if (!done[j] && b.in_f32 == a.in_f32 && b.kind == a.kind && b.load_op == a.load_op &&
-                b.out_f32 == a.out_f32) {
+            if (!done[j] && b.in_f32 == a.in_f32 && b.kind == a.kind && b.out_f32 == a.out_f32) {
                 G.job[G.njobs++] = b;
                 done[j] = true;
             }
         }
-        const bool prod = a.load_op != 0;
         int e;
         if (a.out_f32) {
-            if (L.w_f32) e = a.in_f32 ? launch_z_kind<float, float, float>(G, a.kind, prod, s)
-                                      : launch_z_kind<float, double, float>(G, a.kind, prod, s);
-            else e = a.in_f32 ? launch_z_kind<float, float, double>(G, a.kind, prod, s)
-                              : launch_z_kind<float, double, double>(G, a.kind, prod, s);
+            e = a.in_f32 ? launch_z_kind<float, float>(G, a.kind, s) : launch_z_kind<float, double>(G, a.kind, s);
         } else {
             if (a.in_f32) return -24;   // FP32 input with FP64 output is not used
-            e = L.w_f32 ? launch_z_kind<double, double, float>(G, a.kind, prod, s)
-                        : launch_z_kind<double, double, double>(G, a.kind, prod, s);
+            e = launch_z_kind<double, double>(G, a.kind, s);
         }
         if (e) return e;
     }
@@ -353,12 +333,12 @@ __device__ __forceinline__ void MagRhsKernel<TW, SKIP>::body(const MagArgs& a, u
     const double zck = a.p.zck, s = a.p.sc1;
     const TW hz = (TW)a.p.ho12;
     auto ld2 = [](const void* p, long q) { return *(const TW2*)((const TW*)p + q); };
-    auto ldd = [zero](const double* p, long q) {
+    auto ldd = [&](const double* p, long q) {
         D2 v = {0.0, 0.0};
         if (!zero) v = *(const D2*)(p + q);
         return v;
     };
-    auto ldh = [zero](const void* p, long q) {
+    auto ldh = [&](const void* p, long q) {
         TW2 v = {(TW)0, (TW)0};
         if (!zero) v = *(const TW2*)((const TW*)p + q);
         return v;
@@ -715,7 +695,7 @@ int launch_mag_rhs(const MagArgs& a, hipStream_t s)
     if (a.g.nxy % 2) return -10;   // two columns per thread (nx is even)
     const dim3 grid(nblk(a.g.nxy / 2), (unsigned)((a.g.nz + a.zc - 1) / a.zc));
     if (a.wf32) return mhd_launch<MagRhsKernel<float, false>>(grid, dim3(NT), 0, s, a);
-    if (a.clean) return mhd_launch<MagRhsKernel<double, true>>(grid, dim3(NT), 0, s, a);
+    if (a.clean) return mhd_issue<MagRhsKernel<double, true>>(grid, dim3(NT), 0, s, a);
     return mhd_launch<MagRhsKernel<double, false>>(grid, dim3(NT), 0, s, a);
 }
 int launch_bandj_spec(const MagArgs& a, hipStream_t s)
@@ -756,19 +736,18 @@ __device__ __forceinline__ void AB3Kernel<TH>::body(const AB3Args& a, uint3 bid,
     const long q = (long)bid.x * NT + threadIdx.x;
     if (q < a.g.n3) {
         const double c0 = a.c0, c1 = a.c1, c2 = a.c2;
-        // every entry defined; field f is updated when f0 <= f < nfields
+        // every entry defined; field f is updated when f < nfields
         double xn[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int f = 0; f < 7; ++f) {
-            if (f >= a.f0 && f < a.nfields) {
+            if (f < a.nfields) {
                 const double* x = a.var[f];
                 xn[f] = x[q] + c0 * (double)((const TH*)a.hist[f][2])[q] +
                         c1 * (double)((const TH*)a.hist[f][1])[q] + c2 * (double)((const TH*)a.hist[f][0])[q];
             }
         }
         // src/main.F90:417-425: density floor, its history zeroed
-        const bool hydro = a.f0 == 0;
-        if (hydro && xn[3] < 0.05) {
+        if (xn[3] < 0.05) {
             xn[3] = 0.05;
             ((TH*)a.hist[3][0])[q] = (TH)0;
             ((TH*)a.hist[3][1])[q] = (TH)0;
@@ -784,9 +763,9 @@ __device__ __forceinline__ void AB3Kernel<TH>::body(const AB3Args& a, uint3 bid,
         }
 #pragma unroll
         for (int f = 0; f < 7; ++f) {
-            if (f >= a.f0 && f < a.nfields) a.var[f][q] = (f >= 5 && band) ? 0.0 : xn[f];
+            if (f < a.nfields) a.var[f][q] = (f >= 5 && band) ? 0.0 : xn[f];
         }
-        if (a.shadow[0] && hydro) {
+        if (a.shadow[0]) {
             const int k = (int)(q / a.g.nxy);
             ((float*)a.shadow[0])[q] = (float)xn[0];
             ((float*)a.shadow[1])[q] = (float)xn[1];
@@ -805,10 +784,9 @@ __device__ __forceinline__ void AB3Kernel<TH>::body(const AB3Args& a, uint3 bid,
 
 int launch_ab3(const AB3Args& a, hipStream_t s)
 {
-    // with no field to update (f0 = 7) only the nz means are left
-    long n = a.f0 < a.nfields ? (a.g.n3 > a.g.nz ? a.g.n3 : a.g.nz) : a.g.nz;
-    return a.h32 ? mhd_launch<AB3Kernel<float>>(dim3(nblk(n)), dim3(NT), 0, s, a)
-                 : mhd_launch<AB3Kernel<double>>(dim3(nblk(n)), dim3(NT), 0, s, a);
+    const dim3 grid(nblk(a.g.n3));
+    return a.h32 ? mhd_launch<AB3Kernel<float>>(grid, dim3(NT), 0, s, a)
+                 : mhd_launch<AB3Kernel<double>>(grid, dim3(NT), 0, s, a);
 }
 
 // ---------------------------------------------------------------------------

@@ -18,10 +18,7 @@ struct Phys {
 constexpr int Z_MAX_JOBS = 16;
 struct ZJob {
     const void* in;
-    const void* in1;   // LD_PROD second factor
     int in_f32;
-    int load_op;       // 0 plain, 1 scale*in*in1
-    double scale;
     void* out;
     int out_f32;
     int kind;          // ZKind
@@ -30,8 +27,8 @@ struct ZJob {
 struct ZLaunch {
     Geom g;
     double ho12, sc1;
-    const void* w;     // upwind selector (the solver's w)
-    int w_f32;
+    const double* w;   // upwind selector (the solver's w)
+    int ncu;           // compute units of the device
     int band, icutx, icuty;   // band: the columns of the 2/3 band are neither read nor written
     int njobs;
     ZJob job[Z_MAX_JOBS];
@@ -131,7 +128,6 @@ int launch_mag_init_spec(const MagArgs& a, hipStream_t s, double* means_out /*de
 struct AB3Args {
     Geom g;
     double c0, c1, c2;
-    int f0;                   // first field updated (5: pol, tor; 7: the means only)
     double* var[7];           // u v w r t pol tor
     void* hist[7][3];         // [field][level 1..3] physical slots
     int h32;                  // history arrays are float

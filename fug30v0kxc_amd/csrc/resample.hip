@@ -120,7 +120,6 @@ int hc_pass(const double* in, double* out, int nx, int ny, int nz, int dir, int 
     J.in[0] = in;
     J.out[0] = out;
     J.load_op = LD_PLAIN;
-    J.scale = 1.0;
     const int e = launch_spectral(L, 0, s);
     return e == -20 ? MHD_E_SIZE : (e ? MHD_E_DEVICE : 0);
 }

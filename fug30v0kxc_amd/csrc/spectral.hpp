@@ -47,7 +47,6 @@ struct SpecJob {
     const void* in[4];
     int in_f32;
     int load_op;      // LoadOp
-    double scale;
     const double* mean[4]; // optional per-plane means of in[0..3] (nz entries)
     // LD_CROSS only: the load also subtracts jcoef[k] * jin (the eta(z) term
     // -(eta - eta_0) J of the EMF), when jin is set
@@ -87,8 +86,6 @@ struct SpecLaunch {
     int ncu;          // compute units: the persistent grid is occupancy x ncu workgroups
     int grid_mult;    // ... times this (>= 1; 0 = 1), a tunable launch shape
     int variant;      // radix plan: 0 the default, 1 and 2 the length's alternatives (if any)
-    int max_groups;   // optional further cap on the grid; 0 = none
-    int group_major;  // set by the launcher: items ordered line group first (see spec_kernel)
     // SM_DERIV1: lines without a register plan, and those of the eight lengths
     // from 36 to 216 that gained theirs last (spectral_len_direct), are
     // transformed output point by output point in the run-time radix kernel

@@ -359,21 +359,12 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_cross3(co
             const int n = j + r * NB0;
             dst[0][r] = dst[1][r] = dst[2][r] = {(TC)0, (TC)0};
             if (ok && j < NB0) {
-                if constexpr (DIR != 0) {
-                    const long i = ia + n * st;
-                    const cpx<TC> x0 = ld_pair(a0, i), x1 = ld_pair(a1, i), x2 = ld_pair(a2, i);
-                    const cpx<TC> y0 = ld_pair(b0, i), y1 = ld_pair(b1, i), y2 = ld_pair(b2, i);
-                    dst[0][r] = l0.cross_pair(x1, y2, x2, y1, i);
-                    dst[1][r] = l1.cross_pair(x2, y0, x0, y2, i);
-                    dst[2][r] = l2.cross_pair(x0, y1, x1, y0, i);
-                } else {
-                    const long i = ia + n * st, e = ib + n * st;
-                    const TC x0 = a0[i], x1 = a1[i], x2 = a2[i], y0 = b0[i], y1 = b1[i], y2 = b2[i];
-                    const TC u0 = a0[e], u1 = a1[e], u2 = a2[e], w0 = b0[e], w1 = b1[e], w2 = b2[e];
-                    dst[0][r] = {l0.cross(x1, y2, x2, y1, i), l0.cross(u1, w2, u2, w1, e)};
-                    dst[1][r] = {l1.cross(x2, y0, x0, y2, i), l1.cross(u2, w0, u0, w2, e)};
-                    dst[2][r] = {l2.cross(x0, y1, x1, y0, i), l2.cross(u0, w1, u1, w0, e)};
-                }
+                const long i = ia + n * st;
+                const cpx<TC> x0 = ld_pair(a0, i), x1 = ld_pair(a1, i), x2 = ld_pair(a2, i);
+                const cpx<TC> y0 = ld_pair(b0, i), y1 = ld_pair(b1, i), y2 = ld_pair(b2, i);
+                dst[0][r] = l0.cross_pair(x1, y2, x2, y1, i);
+                dst[1][r] = l1.cross_pair(x2, y0, x0, y2, i);
+                dst[2][r] = l2.cross_pair(x0, y1, x1, y0, i);
             }
         }
     };
@@ -789,7 +780,6 @@ static int launch_one(const SpecLaunch& L, hipStream_t s)
     const bool shared = LOP == LD_CROSS3 || (MODE == SM_DERIV2 && !La.split);
     long grid = ngrp * (shared ? 1 : L.njobs);
     if (L.ncu > 0 && grid > resident) grid = resident;
-    if (L.max_groups > 0 && grid > L.max_groups) grid = L.max_groups;
     return mhd_launch<K>(dim3((unsigned)grid), dim3(NT), lds, s, La);
 }
 
