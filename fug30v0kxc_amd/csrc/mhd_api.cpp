@@ -260,6 +260,19 @@ int walk_planes(const mhd_ctx* c, long groups, int planes, int most)
     return fit < 1 ? 1 : fit < most ? (int)fit : most;
 }
 
+// Persistent-grid multiple of a transform kind until mhd_autotune / mhd_set_tune: the
+// autotuner's choices at 256x256x160 (y in FP64 two resident grids, else one), and
+// two for the FP32 second derivatives along x of lengths whose transform leaves half
+// a wave idle (160 threads: 480 and 640 points; a step of 480 x 64 x 96 mixed 737 ->
+// 696 us, 640 x 64 x 96 853 -> 811, 480 x 128 x 40 656 -> 636; the other lengths from
+// 96 to 1024 lose up to 4 % or change nothing).
+int default_mult(const mhd_ctx* c, int dir, int kind)
+{
+    if (dir == 1) return c->wf32 ? 1 : 2;
+    const int t = kind == SM_DERIV2 && c->wf32 ? spectral_d2_threads(c->nx) : 0;
+    return t > 128 && t % 64 ? 2 : 1;
+}
+
 // f64: FP64 transform in the mixed path (launched with spec64)
 SpecLaunch spec_base(mhd_ctx* c, int dir, int mode, bool f64 = false)
 {
@@ -1119,14 +1132,13 @@ int mhd_create(const mhd_params_t* p, int nx, int ny, int nz, int precision, mhd
     c->ring[0] = 0; c->ring[1] = 1; c->ring[2] = 2;
     c->sc.first = 1;
     c->ncu = ncu;
-    // launch shapes until mhd_autotune / mhd_set_tune: the autotuner's choices at
-    // 256x256x160 on MI355X (y transforms with two resident grids in FP64; 8
-    // planes per column-walk thread)
-    for (int k = 0; k < 4; ++k) c->spec_var[0][k] = c->spec_var[1][k] = 0;
-    for (int k = 0; k < 4; ++k) {
-        c->spec_mult[0][k] = 1;
-        c->spec_mult[1][k] = c->wf32 ? 1 : 2;
-    }
+    // launch shapes until mhd_autotune / mhd_set_tune: the default plans and
+    // multiples, 8 planes per column-walk thread
+    for (int d = 0; d < 2; ++d)
+        for (int k = 0; k < 4; ++k) {
+            c->spec_var[d][k] = 0;
+            c->spec_mult[d][k] = default_mult(c, d, k);
+        }
     {
         const int nin = c->nz > 8 ? c->nz - 8 : 1;   // interior planes
         c->hzc = 8 < nin ? 8 : nin;
@@ -1984,11 +1996,11 @@ int mhd_autotune(mhd_ctx_t* c, mhd_tune_t* out)
     };
     for (int dir = 0; dir < 2; ++dir) {
         const int n = dir == 0 ? c->nx : c->ny;
-        const int mdef = (dir == 1 && !c->wf32) ? 2 : 1;
         for (int kind = 0; kind < MHD_TK_N; ++kind) {
             SpecLaunch L;
             bool f64;
             if (!step_launch(dir, kind, L, f64)) continue;
+            const int mdef = default_mult(c, dir, kind);
             double bk = 1e30;
             int bv = 0, bm = mdef;
             for (int var = 0; var < spectral_variants(n); ++var) {

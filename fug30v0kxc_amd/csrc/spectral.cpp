@@ -51,6 +51,16 @@ int spectral_variants(int n)
     return 1;
 }
 
+int spectral_d2_threads(int n)
+{
+    switch (n) {
+#define X(n_) case n_: return plan_tpt<typename D2Plan<n_, float>::type>();
+        MHD_ALL_SIZES(X)
+#undef X
+    }
+    return 0;
+}
+
 // the file that instantiates a length's kernels
 static int size_group(int n)
 {

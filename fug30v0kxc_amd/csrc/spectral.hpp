@@ -171,5 +171,7 @@ bool generic_plan(int n, int radix[SPEC_GEN_MAX_PASSES], int* npass, bool direct
 int launch_spectral_generic(const SpecLaunch& L, int compute_f32, hipStream_t s);
 // radix plans of the length: SpecLaunch::variant runs from 0 to this - 1
 int spectral_variants(int n);
+// threads of a transform in the FP32 second-derivative passes (0: no plan)
+int spectral_d2_threads(int n);
 
 }  // namespace mhd
