@@ -21,9 +21,8 @@ FP64, 300 bytes per cell in the mixed mode), timed with HIP events on the
 solver's stream over the timed steps; roofline_xderiv2 does the same for the
 x-direction first+second derivative pass of T, u, v, w (with the Maxwell
 stresses and d/dx of rho in the same launch) over a few further steps.  step_roofline puts
-the whole step against the same peak at its algorithmic bytes per cell-step
-(139 working-precision array passes, the FP64 state read and written, the RHS
-history: 1448 B in FP64, 780 B mixed).  cpu_baseline times
+the whole step against the same peak at the bytes per cell-step of the passes it
+runs (step_passes: 1044 B in FP64, 720 B mixed).  cpu_baseline times
 the CPU oracle (a C restatement of the reference) on a bounded sample of the
 same workload: a few steps of the full box on all host threads, and one
 step on one thread.
@@ -488,15 +487,44 @@ KERNEL_DESC = {"xderiv2": "SpecK<T, plan, 0, 2, 1, 0> (xderiv2: d/dx and d2/dx2 
                         "u, v, w, rho, T"}
 
 
-# algorithmic bytes per cell-step of the whole step: 139 working-precision array
-# passes, the FP64 state (7 in, 7 out) and the RHS history (21 in, 7 out)
-def step_bytes_per_cell(elem):
-    return 139 * elem + 14 * 8 + 28 * elem
+# bytes per cell of the passes that a step runs, each array read or written once a
+# pass (halo planes and the walls' passes are not counted).  MODES: the part of a
+# plane's modes, ROWS of its rows that the 2/3 truncation leaves; e: working precision
+MODES, ROWS = 4.0 / 9.0, 2.0 / 3.0
 
 
-def step_roofline(cells, ms_per_step, elem):
-    """The whole step against the HBM peak, at the algorithmic bytes per cell-step."""
-    b = step_bytes_per_cell(elem)
+def step_passes(elem, eta=False):
+    e, mixed, j = elem, elem == 4, 3 if eta else 0
+    return {
+        "xderiv2": KERNEL_BYTES_PER_CELL["xderiv2"][e],
+        "yderiv2": KERNEL_BYTES_PER_CELL["yderiv2"][e],
+        "hydro_col": KERNEL_BYTES_PER_CELL["hydro"][e],
+        # u x B from six fields (eta(z): and the current density) along y; then along
+        # x with the curl, three in and three out
+        "emf_y": (9 + j) * e,
+        "emf_x": 6 * e,
+        # pol, tor (FP64) and two levels of their right-hand sides, C, D, E_z; the new
+        # right-hand sides, pol, tor.  FP64 steps read pol, tor and the levels on the
+        # modes that are not zero
+        "mag_rhs": 2 * 8 * (1.0 if mixed else MODES) + 4 * e * (1.0 if mixed else MODES) + 5 * e + 2 * 8,
+        "pol_z": (8 + e) * MODES,
+        # pol, tor, d pol/dz -> Bx, By, Bz, Jz, dBz/dx (mixed: dBz/dy); then along y
+        "bandj_x": (2 * 8 + e) * MODES + (6 if mixed else 5) * e * ROWS,
+        "bandj_y": (6 if mixed else 5) * e * ROWS + 6 * e,
+        # dBz/dx, dBz/dy, Jz, Bx, By -> J^2 (eta(z): and J)
+        "jsq": (6 + j) * e,
+        # every tenth step, r t u v w along x and y (mixed: and their FP32 shadows)
+        "dealias": (20 * 8 + (5 * 8 + 5 * 4 if mixed else 0)) / 10.0,
+    }
+
+
+def step_bytes_per_cell(elem, eta=False):
+    return sum(step_passes(elem, eta).values())
+
+
+def step_roofline(cells, ms_per_step, elem, eta=False):
+    """The whole step against the HBM peak, at the bytes per cell-step of its passes."""
+    b = round(step_bytes_per_cell(elem, eta), 1)
     achieved = b * cells / (ms_per_step * 1e-3) / 1e9
     return {"bound": "hbm", "bytes_per_cell_step": b, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
@@ -615,7 +643,7 @@ def main():
                "config": {"workload": desc + ", mixed precision, diagnostics every 100 steps",
                           "nx": nx, "ny": ny, "nz": nz, "dt": dt, "ndu06": NDU06, "precision": "mixed"},
                "roofline": roofline_of(rm, args.kernel, 4, args.workload), "cpu_baseline": None,
-               "step_roofline": step_roofline(cells, rm["elapsed"] / args.steps * 1e3, 4),
+               "step_roofline": step_roofline(cells, rm["elapsed"] / args.steps * 1e3, 4, "eta_c" in extra),
                "device_bytes": rm["device_bytes"]}
         if "kms2" in rm:
             out["roofline_xderiv2"] = roofline_of(rm, "xderiv2", 4, args.workload, second=True)
@@ -651,7 +679,7 @@ def main():
                  "roofline": roofline_of(rm, args.kernel, 4, args.workload),
                  "roofline_xderiv2": (roofline_of(rm, "xderiv2", 4, args.workload, second=True)
                                       if "kms2" in rm else None),
-                 "step_roofline": step_roofline(cells, rm["elapsed"] / args.steps * 1e3, 4),
+                 "step_roofline": step_roofline(cells, rm["elapsed"] / args.steps * 1e3, 4, "eta_c" in extra),
                  "tune": rm.get("tune"),
                  "device_bytes": rm["device_bytes"]}
         rm["solver"].close()
@@ -673,7 +701,7 @@ def main():
            "roofline": roofline_of(r64, args.kernel, 8, args.workload), "cpu_baseline": cpu,
            "roofline_xderiv2": (roofline_of(r64, "xderiv2", 8, args.workload, second=True)
                                 if "kms2" in r64 else None),
-           "step_roofline": step_roofline(cells, r64["elapsed"] / args.steps * 1e3, 8),
+           "step_roofline": step_roofline(cells, r64["elapsed"] / args.steps * 1e3, 8, "eta_c" in extra),
            "mixed": mixed,
            "tune": r64.get("tune"),
            "device_bytes": r64["device_bytes"],
