@@ -118,8 +118,8 @@ template <typename TC> struct D2Plan<480, TC> { using type = Plan<480, 4, 8, 5, 
 template <typename TC> struct D2Plan<512, TC> { using type = Plan<512, 4, 4, 8, 4>; };
 template <typename TC> struct D2Plan<640, TC> { using type = Plan<640, 4, 8, 5, 4>; };
 // FP32 passes of 512 points have the registers for three radix-8 passes, one LDS
-// exchange less (a step of 512^2 x 64 mixed, 4 4 8 4 -> 8 8 8: 3232 -> 3003 us
-// along y, -> 3198 along x; FP64 loses along y, 5235 -> 5306)
+// exchange less (512^2 x 64 mixed, 4 4 8 4 -> 8 8 8: y 804 -> 588 us, x 343 -> 295;
+// FP64 loses along y, a step 5235 -> 5306)
 template <> struct D2Plan<512, float> { using type = Plan<512, 8, 8, 8>; };
 
 template <typename PL>

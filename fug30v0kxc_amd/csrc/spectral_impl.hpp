@@ -405,10 +405,11 @@ __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_cross3(co
 // What bounds it: HBM through the few waves its registers allow (FP64 210: two
 // per SIMD), LDS busy 35-46 % and the VALU 23-31 % of the time.  The auxiliary
 // lines replace a launch of their own per direction (three first derivatives
-// from one load of b) and, in y, two single-output jobs: at 256^2 x 160 FP64 x
-// 241 + 104 -> 318 us, y 324 + 151 -> 449, FP32 132 + 72 -> 165 and 209 + 91 ->
-// 246; hydro_col reads 18 arrays for 26 (855 -> 723 us).  Reloading b per job
-// (three waves per SIMD) measured slower: x 336, y 460, FP32 213 and 292.
+// from one load of b) and, in y FP64, two single-output jobs: at 256^2 x 160 FP64 x
+// 241 + 104 -> 318 us, y 324 + 151 -> 449, and hydro_col reads 18 arrays for 26 (855
+// -> 723 us).  FP32, whose stresses stay outputs of their own (AuxOp): 132 + 72 ->
+// 179 and 209 + 91 -> 296.  Reloading b per job (three waves per SIMD) measured
+// slower: x 336, y 460 us FP64.
 template <typename TC, typename PL, int DIR, int B, int MODE, int LOP>
 __device__ __forceinline__ void SpecK<TC, PL, DIR, B, MODE, LOP>::body_deriv2(const SpecLaunch& L, uint3 bid,
                                                                               uint3 gdim)
@@ -805,8 +806,9 @@ static int launch_y(const SpecLaunch& L, hipStream_t s)
 }
 
 // Second derivatives.  Half groups along y where a full one has 512 threads
-// (FP64) or 1024 (FP32), so that two or more workgroups share a CU (256 points: y
-// 449 against 458 us FP64, 246 against 241 FP32; 512 points FP32: 8 pairs spill).
+// (FP64) or 1024 (FP32), so that two or more workgroups share a CU (256 points FP64:
+// y 449 against 458 us; FP32: 293 against 276 at 256^2 x 160 and 317 against 284 at 256
+// x 384 x 64, but 50 against 58 at 256^2 x 24 and 118 against 138 at 192^2 x 96).
 // In FP64 also where the full group is 4 pairs (480, 640, 768 and 1024 points,
 // 640 to 1024 threads): those spill 150 to 210 registers, 2 pairs and their 32-byte
 // row segments do not (y pass 1478 -> 645 us at 256 x 480 x 64, 1712 -> 872 at

@@ -21,8 +21,8 @@
 // + 36 -> 97 + 49 FP32 (x, y, C and D).  bandj_x reads 3 fields on the modes that
 // are not zero (44 % of a plane) and writes 5 on the rows that are not (67 %),
 // where a spectral kernel wrote 6 fields and the x pass read and wrote 6; dBz/dy
-// comes from the y pass's spectrum: 163 + 184 + 226 -> 96 + 175 us FP64, 105 + 79
-// + 98 -> 65 + 103 FP32 (spectral, x, y).
+// comes from the y pass's spectrum (FP32: it is a sixth field): 163 + 184 + 226 -> 96
+// + 175 us FP64, 105 + 79 + 98 -> 72 + 86 FP32 (spectral, x, y).
 #include "spectral_impl.hpp"
 
 namespace mhd {
